@@ -15,7 +15,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libepic_gpu.so")
 BUILD = os.path.join(HERE, "_build")
 
-SOURCES = ["abi.hip", "plan.hip", "p2g.hip", "g2p.hip", "fft.hip", "inversion.hip", "split.hip", "merge.hip",
+SOURCES = ["abi.hip", "plan.hip", "p2g.hip", "g2p.hip", "fft.hip", "vtend.hip", "inversion.hip", "split.hip", "merge.hip",
            "correction.hip", "timestep.hip", "diagnostics.hip",
            "resort.hip", "eigen.hip", "ncio.cpp"]
 

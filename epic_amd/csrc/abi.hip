@@ -68,7 +68,7 @@ struct epic_member {
     float2 *twx = nullptr, *twy = nullptr;
     double2 *twx64 = nullptr, *twy64 = nullptr;
     double2 *twz = nullptr;
-    FftPlan px{}, py{}, pz{};
+    FftPlan px{}, pnx{}, py{}, pz{};   // complex lengths nx/2, nx, ny, 2 nz
     // per-phase GPU timers (events on the member stream)
     int profiling = 0;   // 1: eager launches between event pairs; 2: graph replays with wall-clock stamps per phase
     std::vector<hipEvent_t> ev;        // pairs (start, stop) recorded in order
@@ -519,7 +519,6 @@ FftXArgs xargs(epic_member *m)
     a.g = m->g;
     a.plan = m->px;
     a.tw = m->twx;
-    a.tw64 = m->twx64;
     a.fld = m->fld;
     a.fld_out = m->fld;
     return a;
@@ -531,7 +530,6 @@ FftYArgs yargs(epic_member *m)
     a.g = m->g;
     a.plan = m->py;
     a.tw = m->twy;
-    a.tw64 = m->twy64;
     return a;
 }
 
@@ -588,60 +586,23 @@ void build_vor2vel(Plan &P, const Members &ms)
     add_vor2vel_fixup(P, PH_VOR2VEL, fx);
 }
 
-// vorticity_tendency: six flux transforms, two combined inverse transforms
-// per component (the z derivative is added in the last pass), all in FP64
-// from the FP32 node fields: the spectral derivative amplifies white
-// rounding noise at the highest wavenumbers, which FP32 products and
-// transforms would add.  The FP64 spectrum q takes the float2 spectra 2q and
-// 2q + 1 (one allocation).
+// vorticity_tendency; the FP64 x parts take the spectra, which are free
+// between two transforms
 void build_vtend(Plan &P, const Members &ms)
 {
-    std::vector<FftXArgs> xf, xi;
-    std::vector<FftYArgs> yf, yi;
-    std::vector<FixArgs> fx;
+    std::vector<VtendArgs> items;
     for (epic_member *m : ms) {
-        auto sp64 = [&](int q) { return (void *)m->spec[2 * q]; };
-        for (int c = 0; c < 3; ++c)
-            for (int a = 0; a < 2; ++a) {
-                FftXArgs x = xargs(m);
-                x.fp64 = 1;
-                x.mode = 1;
-                x.comp_a = a;
-                x.comp_b = c;
-                // f_x of the y tendency carries -b, f_y of the x tendency +b (inversion.f90:327-335)
-                x.sgn = (a == 0 && c == 1) ? -1 : ((a == 1 && c == 0) ? 1 : 0);
-                x.out = sp64(2 * c + a);
-                xf.push_back(x);
-                FftYArgs y = yargs(m);
-                y.fp64 = 1;
-                y.mode = 0;
-                y.in = sp64(2 * c + a);
-                y.out = sp64(2 * c + a);
-                yf.push_back(y);
-            }
-        for (int c = 0; c < 3; ++c) {
-            FftYArgs y = yargs(m);
-            y.fp64 = 1;
-            y.mode = 2;
-            y.in = sp64(2 * c);
-            y.in2 = sp64(2 * c + 1);
-            y.out = sp64(2 * c);
-            yi.push_back(y);
-            FftXArgs x = xargs(m);
-            x.fp64 = 1;
-            x.mode = 2;
-            x.comp_b = c;
-            x.slot = F_VTEND + c;
-            x.in = sp64(2 * c);
-            xi.push_back(x);
-        }
-        fx.push_back(FixArgs{m->g, m->fld});
+        VtendArgs a{};
+        a.g = m->g;
+        a.px = m->pnx;
+        a.py = m->py;
+        a.twx = m->twx64;
+        a.twy = m->twy64;
+        a.fld = m->fld;
+        a.dx = (double *)m->spec[0];
+        items.push_back(a);
     }
-    add_fft_xf(P, PH_VTEND, xf);
-    add_fft_y(P, PH_VTEND, yf);
-    add_fft_y(P, PH_VTEND, yi);
-    add_fft_xi(P, PH_VTEND, xi);
-    add_vtend_fixup(P, PH_VTEND, fx);
+    add_vtend(P, PH_VTEND, items);
 }
 
 // one LS-RK step (ls_rk.f90:88-136) of every member.  Histograms: stage s
@@ -942,7 +903,8 @@ int epic_create(const epic_grid_t *grid, const epic_phys_t *phys, const epic_fla
         bad(dalloc(&m->far_acc, (int64_t)P2G_NF * FS, m->s)) || bad(dalloc(&m->far_flag, 1, m->s)) ||
         bad(dalloc(&m->far_scale, P2G_NF, m->s)))
         return EPIC_E_NOMEM;
-    static_assert(NSPEC >= 12, "the six FP64 spectra of vorticity_tendency take twelve float2 spectra");
+    // vorticity_tendency's 3 (nz + 1) ny nx doubles: a spectrum holds more than nx/2 (nz + 1) ny of them
+    static_assert(NSPEC >= 6, "the FP64 x parts of vorticity_tendency take six spectra");
     if (bad(dalloc(&m->spec[0], NSPEC * spec_size(g), m->s))) return EPIC_E_NOMEM;
     for (int i = 1; i < NSPEC; ++i) m->spec[i] = m->spec[0] + i * spec_size(g);
     if (bad(dalloc(&m->err_d, 4, m->s)) || bad(dalloc(&m->flags_d, 4, m->s)) || bad(dalloc(&m->tm_d, 1, m->s))) return EPIC_E_NOMEM;
@@ -953,6 +915,7 @@ int epic_create(const epic_grid_t *grid, const epic_phys_t *phys, const epic_fla
     *m->tm_h = StepTime{};
     // twiddles (FP64-accurate roots of unity)
     m->px = make_plan(g.nx / 2);
+    m->pnx = make_plan(g.nx);
     m->py = make_plan(g.ny);
     m->pz = make_plan(2 * g.nz);
     std::vector<float2> tx(g.nx), ty(g.ny);

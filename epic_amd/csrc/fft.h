@@ -77,17 +77,17 @@ template <typename T2> struct TwHalf {   // first half of the table only (n even
     }
 };
 
-// one Stockham stage of radix R over L lines of n points (registers only:
-// the radix is a compile-time constant)
+// one Stockham stage of radix R over L lines of n points, ls apart
+// (registers only: the radix is a compile-time constant)
 // (nb and ns: the plan's quotients by n / R and by Ns)
 template <int R, typename T2, typename TW>
-__device__ inline void fft_stage(const T2 *in, T2 *out, int L, int n, const FastDiv &nbd, const FastDiv &nsd,
+__device__ inline void fft_stage(const T2 *in, T2 *out, int L, int ls, const FastDiv &nbd, const FastDiv &nsd,
                                  int tstep, const TW &tw, bool inv)
 {
     const int nb = nbd.d, Ns = nsd.d;
     for (int t = threadIdx.x; t < L * nb; t += blockDim.x) {
         const int l = fdiv(t, nbd), jj = t - l * nb;
-        const T2 *src = in + l * n;
+        const T2 *src = in + l * ls;
         T2 v[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) v[r] = src[jj + r * nb];
@@ -99,26 +99,25 @@ __device__ inline void fft_stage(const T2 *in, T2 *out, int L, int n, const Fast
             v[r] = cmul(v[r], w);
         }
         butterfly<R>(v, inv);
-        T2 *dst = out + l * n + q * Ns * R + kk;
+        T2 *dst = out + l * ls + q * Ns * R + kk;
 #pragma unroll
         for (int r = 0; r < R; ++r) dst[r * Ns] = v[r];
     }
 }
 
-// L lines of n points each, line l at a[l*n]; every thread of the block
-// calls this.  Returns the buffer holding the result (a or b).  Ends with a
-// barrier.
+// L lines of n points each, line l at a[l*ls] (ls >= n); every thread of the
+// block calls this.  Returns the buffer holding the result (a or b).  Ends
+// with a barrier.
 template <typename T2, typename TW>
-__device__ T2 *lds_fft_tw(T2 *a, T2 *b, int L, const FftPlan &pl, const TW &tw, bool inv)
+__device__ T2 *lds_fft_tw(T2 *a, T2 *b, int L, const FftPlan &pl, const TW &tw, bool inv, int ls)
 {
-    const int n = pl.n;
     T2 *in = a, *out = b;
     for (int st = 0; st < pl.nst; ++st) {
         const int R = pl.radix[st];
-        if (R == 4) fft_stage<4>(in, out, L, n, pl.nb[st], pl.ns[st], pl.tstep[st], tw, inv);
-        else if (R == 2) fft_stage<2>(in, out, L, n, pl.nb[st], pl.ns[st], pl.tstep[st], tw, inv);
-        else if (R == 3) fft_stage<3>(in, out, L, n, pl.nb[st], pl.ns[st], pl.tstep[st], tw, inv);
-        else fft_stage<5>(in, out, L, n, pl.nb[st], pl.ns[st], pl.tstep[st], tw, inv);
+        if (R == 4) fft_stage<4>(in, out, L, ls, pl.nb[st], pl.ns[st], pl.tstep[st], tw, inv);
+        else if (R == 2) fft_stage<2>(in, out, L, ls, pl.nb[st], pl.ns[st], pl.tstep[st], tw, inv);
+        else if (R == 3) fft_stage<3>(in, out, L, ls, pl.nb[st], pl.ns[st], pl.tstep[st], tw, inv);
+        else fft_stage<5>(in, out, L, ls, pl.nb[st], pl.ns[st], pl.tstep[st], tw, inv);
         __syncthreads();
         T2 *tmp = in;
         in = out;
@@ -129,9 +128,9 @@ __device__ T2 *lds_fft_tw(T2 *a, T2 *b, int L, const FftPlan &pl, const TW &tw, 
 
 // tw[t*tws] = e^{-2 pi i t / n}
 template <typename T2>
-__device__ T2 *lds_fft(T2 *a, T2 *b, int L, const FftPlan &pl, const T2 *__restrict__ tw, int tws, bool inv)
+__device__ T2 *lds_fft(T2 *a, T2 *b, int L, const FftPlan &pl, const T2 *__restrict__ tw, int tws, bool inv, int ls)
 {
-    return lds_fft_tw(a, b, L, pl, TwStrided<T2>{tw, tws}, inv);
+    return lds_fft_tw(a, b, L, pl, TwStrided<T2>{tw, tws}, inv, ls);
 }
 
 inline FftPlan make_plan(int n)

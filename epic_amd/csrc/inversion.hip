@@ -95,7 +95,7 @@ template <int NS> __device__ __forceinline__ void zdst(const ColCtx &c, ZCol<NS,
         }
     }
     __syncthreads();
-    double2 *R = lds_fft_tw(c.fa, c.fb, 1, *c.plan, TwHalf<double2>{c.tw, nz}, false);
+    double2 *R = lds_fft_tw(c.fa, c.fb, 1, *c.plan, TwHalf<double2>{c.tw, nz}, false, n2);
     const double s = 0.5 * sqrt(2.0 / (double)nz);
     ZSLOTS(i, z)
     {
@@ -117,7 +117,7 @@ template <int NS> __device__ __forceinline__ void zdct(const ColCtx &c, ZCol<NS,
         }
     }
     __syncthreads();
-    double2 *R = lds_fft_tw(c.fa, c.fb, 1, *c.plan, TwHalf<double2>{c.tw, nz}, false);
+    double2 *R = lds_fft_tw(c.fa, c.fb, 1, *c.plan, TwHalf<double2>{c.tw, nz}, false, n2);
     const double s = 0.5 * sqrt(2.0 / (double)nz);
     ZSLOTS(i, z)
     {
@@ -510,30 +510,6 @@ __global__ __launch_bounds__(256) void k_vor2vel_fixup(const FixArgs *__restrict
     F(F_VELGRADG + DVDZ, k) = dwdy - F(F_VORTG + 0, k);
 }
 
-// vorticity_tendency: zeta walls and z extrapolation (inversion.f90:345-360)
-__global__ __launch_bounds__(256) void k_vtend_fixup(const FixArgs *__restrict__ tab, const int2 *__restrict__ bmap)
-{
-    const ItemBlock ib = item_block(bmap);
-    const Grid &g = tab[ib.item].g;
-    float *const fld = tab[ib.item].fld;
-    const int64_t col = ib.blk * (int64_t)blockDim.x + threadIdx.x;
-    if (col >= (int64_t)g.nx * g.ny) return;
-    const int64_t FS = field_stride(g), PS = plane_stride(g);
-    const int nz = g.nz;
-    auto F = [&](int slot, int k) -> EPIC_GLOBAL float & { return gl(fld)[slot * FS + (int64_t)(k + 1) * PS + col]; };
-    // the transforms wrote the halo planes as the extrapolations 2 v(0) -
-    // v(1) and 2 v(nz) - v(nz-1) of the unmodified tendency; where dzeta/dt
-    // is held at zero on a wall, that extrapolation is -v(1) (-v(nz-1))
-    if (g.zeta_zero[0]) {
-        F(F_VTEND + 2, 0) = 0.0f;
-        F(F_VTEND + 2, -1) = -F(F_VTEND + 2, 1);
-    }
-    if (g.zeta_zero[1]) {
-        F(F_VTEND + 2, nz) = 0.0f;
-        F(F_VTEND + 2, nz + 1) = -F(F_VTEND + 2, nz - 1);
-    }
-}
-
 // register slots per lane for a column of nz + 1 values (0: the LDS form)
 static int col_slots(const Grid &g)
 {
@@ -570,23 +546,11 @@ void add_vor2vel_columns(Plan &P, int phase, const std::vector<ColArgs> &items)
     }
 }
 
-static std::vector<int> column_blocks(const std::vector<FixArgs> &items)
-{
-    std::vector<int> nb;
-    for (const FixArgs &a : items) nb.push_back((int)(((int64_t)a.g.nx * a.g.ny + 255) / 256));
-    return nb;
-}
-
 void add_vor2vel_fixup(Plan &P, int phase, const std::vector<FixArgs> &items)
 {
     std::vector<int> nb;
     for (const FixArgs &a : items) nb.push_back((int)(((int64_t)a.g.nx * a.g.ny * (a.g.nz + 3) + 255) / 256));
     P.add((const void *)k_vor2vel_fixup, 256, 0, phase, items, nb);
-}
-
-void add_vtend_fixup(Plan &P, int phase, const std::vector<FixArgs> &items)
-{
-    P.add((const void *)k_vtend_fixup, 256, 0, phase, items, column_blocks(items));
 }
 
 }  // namespace epic

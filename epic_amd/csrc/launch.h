@@ -133,34 +133,24 @@ void add_grid2par(Plan &P, int phase, const std::vector<G2PArgs> &items);
 void add_rk_stage_tiles(Plan &P, int phase, const std::vector<G2PTileArgs> &items);
 
 // ---- horizontal FFTs (fft.hip) ----
-// fp64: spectra and arithmetic in FP64 (double2 spectra, twiddles tw64);
-// every item of one launch has the same precision.  The FP64 transforms are
-// the vorticity tendency's (modes 1 forward and 2 inverse) and carry the
-// halo planes -1 and nz + 1 at z indices nz + 1 and nz + 2.
 struct FftXArgs {
     Grid g;
     FftPlan plan;          // complex length nx/2
     const float2 *tw;      // e^{-2 pi i t / nx}, t < nx
-    const double2 *tw64;   // the same in FP64
-    int fp64;
-    int mode;              // forward: 0 field, 1 tendency flux, 3 volg / vcell - 1;
-                           // inverse: 0 store, 2 store + d/dz flux
+    int mode;              // forward: 0 field, 3 volg / vcell - 1
     int slot;              // field slot read (forward, mode 0) or written (inverse)
-    int comp_a, comp_b, sgn;
     const float *fld;      // node fields read
     float *fld_out;        // node fields written (inverse)
-    void *out;             // forward: T[j][kx][z] (float2 or double2)
-    const void *in;        // inverse: T[j][kx][z]
+    float2 *out;           // forward: T[j][kx][z]
+    const float2 *in;      // inverse: T[j][kx][z]
 };
 struct FftYArgs {
     Grid g;
     FftPlan plan;          // length ny
     const float2 *tw;      // e^{-2 pi i t / ny}
-    const double2 *tw64;
-    int fp64;
-    int mode;              // 0 forward, 1 inverse, 2 inverse of i kx in + i ky in2
-    const void *in, *in2;
-    void *out;             // may equal in
+    int mode;              // 0 forward, 1 inverse
+    const float2 *in;
+    float2 *out;           // may equal in
 };
 void add_fft_xf(Plan &P, int phase, const std::vector<FftXArgs> &items);
 void add_fft_y(Plan &P, int phase, const std::vector<FftYArgs> &items);
@@ -179,12 +169,22 @@ struct FixArgs {
     float *fld;
 };
 size_t col_lds_bytes(const Grid &g);
-// the largest LDS allocation of the transform work-groups (FP64 x and y
-// passes, vertical columns)
+// the LDS a grid's transforms may take: epic_create refuses grids beyond it
 size_t transform_lds_bytes(const Grid &g);
 void add_vor2vel_columns(Plan &P, int phase, const std::vector<ColArgs> &items);
 void add_vor2vel_fixup(Plan &P, int phase, const std::vector<FixArgs> &items);
-void add_vtend_fixup(Plan &P, int phase, const std::vector<FixArgs> &items);
+
+// ---- vorticity tendency (vtend.hip) ----
+struct VtendArgs {
+    Grid g;
+    FftPlan px, py;            // complex lengths nx and ny
+    const double2 *twx, *twy;  // e^{-2 pi i t / n}, t < n
+    float *fld;                // reads vorticity, velocity and buoyancy, writes F_VTEND
+    double *dx;                // scratch: the x parts, 3 (nz + 1) ny nx
+    int comp;                  // component, set by add_vtend with the two below
+    int lines, planes;         // row pairs per k_flux_dx block, planes per k_flux_dy block
+};
+void add_vtend(Plan &P, int phase, const std::vector<VtendArgs> &members);
 
 // ---- parcel splitting (split.hip) ----
 struct SplitArgs {
