@@ -128,9 +128,9 @@ __global__ __launch_bounds__(256) void k_grid2par(const G2PArgs *__restrict__ ta
 // planes k0-1 .. k0+tz+1, x and y from -1 to 9 around the tile) are staged in
 // LDS once as four planes of field groups (fields 0-3, 4-7, 8-11 as float4,
 // 12-13 as float2), so every corner is three 16-byte and one 8-byte LDS read
-// and neighbouring nodes sit in neighbouring banks; then every thread takes parcels of the
-// chunk through the cell sort (the rows of 8 cells are contiguous slot
-// ranges) with no barrier between parcels.  Support points come from the
+// and neighbouring nodes sit in neighbouring banks; then every thread takes
+// parcels of the chunk's slot range of the cell sort, with no barrier between
+// parcels.  Support points come from the
 // half axes cached for this stage.  The permutation entry of a thread's next
 // parcel is loaded one round ahead, and parcel arrays are addressed as a
 // table pointer plus a 32-bit byte offset.
@@ -158,7 +158,6 @@ __global__ __launch_bounds__(G2P_THREADS, 4) void k_g2p_tiles(const G2PTileArgs 
     extern __shared__ float4 box[];                 // [group][plane][y][x]: 3 float4 groups, then a float2 group
     const int NB = nbox * NN;                       // nodes in the box
     float2 *box2 = (float2 *)(box + 3 * NB);
-    __shared__ int row_slot[64], row_off[65];       // the chunk's rows of 8 cells
     __shared__ unsigned int s_pmax[P2G_NF + 1];     // the next par2grid's maxima (float bits)
     int e = 0;
     if (tid <= P2G_NF) s_pmax[tid] = 0u;   // ordered by the barrier after the box is staged
@@ -193,45 +192,16 @@ __global__ __launch_bounds__(G2P_THREADS, 4) void k_g2p_tiles(const G2PTileArgs 
             }
         }
     }
-    const int nrow = nl * P2G_TY;
-    if (tid < nrow) {   // a partial tile's rows are shorter (wx cells), or beyond the grid (empty)
-        const int k = k0 + tid / P2G_TY, r = tid % P2G_TY;
-        const int wx = min(P2G_TX, g.nx - i0);
-        if (j0 + r < g.ny) {
-            const int c0 = ((k + 1) * g.ny + (j0 + r)) * g.nx + i0;
-            row_slot[tid] = gl(a.cell_start)[c0];
-            row_off[tid + 1] = gl(a.cell_start)[c0 + wx] - gl(a.cell_start)[c0];
-        } else {
-            row_slot[tid] = 0;
-            row_off[tid + 1] = 0;
-        }
-    }
     __syncthreads();
-    if (tid < 64) {   // inclusive scan of the row sizes in one wave
-        int v = (tid < nrow) ? row_off[tid + 1] : 0;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int t = __shfl_up(v, o, 64);
-            if (tid >= o) v += t;
-        }
-        if (tid < nrow) row_off[tid + 1] = v;
-        if (tid == 0) row_off[0] = 0;
-    }
-    __syncthreads();
-    const int total = row_off[nrow];
+    // the chunk's parcels: one contiguous slot range of the sort
+    const int first = gl(a.cell_start)[layer_index(g, tx, ty, k0)];
+    const int total = gl(a.cell_start)[layer_index(g, tx, ty, k0 + nl)] - first;
 
-    // the row holding entry q: largest r with row_off[r] <= q
-    auto row_of = [&](int q) {
-        int r = 0;
-        for (int step = 32; step > 0; step >>= 1)
-            if (r + step < nrow && row_off[r + step] <= q) r += step;
-        return r;
-    };
     // The next round's entry is loaded one round ahead, and the position and
     // half axes of the parcel it names are requested in the middle of the
     // current round (after the gather), so the support points of a round
     // start without waiting for memory.
-    int r_nx = 0, pi_nx = 0;
+    int pi_nx = 0;
     double pn[3] = {0.0, 0.0, 0.0};
     float an[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     auto prefetch = [&](int pj) {
@@ -243,19 +213,15 @@ __global__ __launch_bounds__(G2P_THREADS, 4) void k_g2p_tiles(const G2PTileArgs 
         for (int c = 0; c < 6; ++c) an[c] = at(a.axes[c], oj);
     };
     if (tid < total) {
-        r_nx = row_of(tid);
-        pi_nx = gl(a.perm)[row_slot[r_nx] + (tid - row_off[r_nx])];
+        pi_nx = gl(a.perm)[first + tid];
         prefetch(pi_nx);
     }
     for (int base = 0; base < total; base += G2P_THREADS) {   // uniform rounds: the ballot needs every lane
         const int q = base + tid;
-        const int r = r_nx, pi = pi_nx;
+        const int pi = pi_nx;
         const unsigned o4 = (unsigned)pi * 4u;   // byte offset (pi < 2^30): scalar base + 32-bit offset addressing
         const bool more = q + G2P_THREADS < total;
-        if (more) {
-            r_nx = row_of(q + G2P_THREADS);
-            pi_nx = gl(a.perm)[row_slot[r_nx] + (q + G2P_THREADS - row_off[r_nx])];
-        }
+        if (more) pi_nx = gl(a.perm)[first + q + G2P_THREADS];
         double pos[3] = {pn[0], pn[1], pn[2]};
         const double ve[3] = {an[0], an[1], an[2]};
         const double vt[3] = {an[3], an[4], an[5]};
@@ -263,7 +229,6 @@ __global__ __launch_bounds__(G2P_THREADS, 4) void k_g2p_tiles(const G2PTileArgs 
         bool small = false;
         auto process = [&]() {
             if (q >= total) return;
-            const int k = k0 + r / P2G_TY;
             double B[5];
 #pragma unroll
             for (int c = 0; c < 5; ++c) B[c] = (double)at(a.p.B[c], o4);
@@ -272,7 +237,8 @@ __global__ __launch_bounds__(G2P_THREADS, 4) void k_g2p_tiles(const G2PTileArgs 
 #pragma unroll
             for (int d = 0; d < 3; ++d) cc[d] = (int)floor((pos[d] - g.lower[d]) * g.dxi[d]);
             const int cx = wrap(cc[0], g.nx) - i0, cy = wrap(cc[1], g.ny) - j0;
-            if (cx < 0 || cx >= P2G_TX || cy < 0 || cy >= P2G_TY || cc[2] != k) {
+            const int k = cc[2];
+            if (cx < 0 || cx >= P2G_TX || cy < 0 || cy >= P2G_TY || k < k0 || k >= k0 + nl) {
                 e |= ERR_CELL_MISMATCH;
                 if (more) prefetch(pi_nx);
                 return;
@@ -400,7 +366,7 @@ __global__ __launch_bounds__(G2P_THREADS, 4) void k_g2p_tiles(const G2PTileArgs 
             const int nj = (int)floor((pos[1] - g.lower[1]) * g.dxi[1]);
             const int nk = (int)floor((pos[2] - g.lower[2]) * g.dxi[2]);
             if (nk < -1 || nk > g.nz) e |= ERR_PARCEL_COUNT;
-            else key = ((nk + 1) * g.ny + wrap(nj, g.ny)) * g.nx + wrap(ni, g.nx);
+            else key = cell_index(g, wrap(ni, g.nx), wrap(nj, g.ny), nk);
             at(a.keys, o4) = key;
             small = (vol <= g.vmin);
             if (a.axes_next[0]) {   // the next stage's support axes, from B as stored
@@ -453,7 +419,7 @@ void add_rk_stage_tiles(Plan &P, int phase, const std::vector<G2PTileArgs> &item
     std::vector<int> nb;
     size_t lds = 0;
     for (const G2PTileArgs &a : items) {
-        nb.push_back(a.ntx * a.nty * a.nchz);   // (empty rows: no work)
+        nb.push_back(a.ntx * a.nty * a.nchz);
         lds = std::max(lds, g2p_lds_bytes(a.tz));
     }
     P.add((const void *)k_g2p_tiles, G2P_THREADS, lds, phase, items, nb);

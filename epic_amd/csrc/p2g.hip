@@ -44,7 +44,7 @@ __device__ inline int cell_key(const Grid &g, double x, double y, double z, int 
         err |= ERR_PARCEL_COUNT;
         return -1;
     }
-    return ((k + 1) * g.ny + wrap(j, g.ny)) * g.nx + wrap(i, g.nx);
+    return cell_index(g, wrap(i, g.nx), wrap(j, g.ny), k);
 }
 
 __global__ __launch_bounds__(256) void k_cell_keys(const KeysArgs *__restrict__ tab, const int2 *__restrict__ bmap)
@@ -389,7 +389,6 @@ __global__ __launch_bounds__(64 * TZ * P2G_TPC, 8 / TZ) void k_p2g_tiles(const P
     const int tx = ib.blk % a.ntx;
     const int ty = (ib.blk / a.ntx) % a.nty;
     const int cz = ib.blk / (a.ntx * a.nty);
-    const int i0 = tx * P2G_TX, j0 = ty * P2G_TY;
     const int k0 = -1 + cz * tz;
     const int tid = threadIdx.x;
     constexpr int nbox = box_planes(tz);
@@ -409,8 +408,8 @@ __global__ __launch_bounds__(64 * TZ * P2G_TPC, 8 / TZ) void k_p2g_tiles(const P
     const int cx = ct & 7, cy = (ct >> 3) & 7, lz = ct >> 6;
     const int k = k0 + lz;
     int s0 = 0, s1 = 0;
-    if (k <= g.nz && i0 + cx < g.nx && j0 + cy < g.ny) {   // cells of a partial tile beyond the grid: none
-        const int c = ((k + 1) * g.ny + j0 + cy) * g.nx + i0 + cx;
+    if (k <= g.nz) {   // (cells of a partial tile beyond the grid are empty)
+        const int c = layer_index(g, tx, ty, k) + (ct & (TILE_CELLS - 1));
         s0 = gl(a.cell_start)[c];
         s1 = gl(a.cell_start)[c + 1];
     }
@@ -789,7 +788,7 @@ __global__ __launch_bounds__(256) void k_p2g_finalize(const FinalizeArgs *__rest
     }
     // parcel counts (:201-205, folds :239-243)
     auto cnt = [&](const int *c, int kk) -> int {
-        return (kk >= -1 && kk <= nz) ? gl(c)[((int64_t)(kk + 1) * g.ny + j) * g.nx + i] : 0;
+        return (kk >= -1 && kk <= nz) ? gl(c)[cell_index(g, i, j, kk)] : 0;
     };
     int np = cnt(a.count, k), ns = cnt(a.scount, k);
     if (k == 0) {
@@ -804,7 +803,7 @@ __global__ __launch_bounds__(256) void k_p2g_finalize(const FinalizeArgs *__rest
     gl(a.nsparg)[(int64_t)(k + 1) * PS + base] = ns;
     // clear the histogram the next push fills (never the one read here)
     if (a.clear_count && k <= nz) {
-        const int64_t c = ((int64_t)(k + 1) * g.ny + j) * g.nx + i;
+        const int c = cell_index(g, i, j, k);
         gl(a.clear_count)[c] = 0;
         gl(a.clear_scount)[c] = 0;
     }
