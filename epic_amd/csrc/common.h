@@ -22,7 +22,7 @@ constexpr int P2G_TX = 8;        // p2g tile cells in x
 constexpr int P2G_TY = 8;        // p2g tile cells in y
 constexpr int P2G_BOX = 11;      // node box per tile side: 1 lower + 8 + 2 upper
 constexpr int P2G_NF = 7;        // vol, xi, eta, zeta, tbuoy, dbuoy, hum
-constexpr int P2G_TPC = 2;       // par2grid threads per cell (neighbouring lanes)
+constexpr int P2G_TPC = 2;       // par2grid threads per cell of a chunk (a work-group has 64 tz P2G_TPC)
 
 // error bits reported through the member's device error word
 enum : int {
@@ -197,6 +197,9 @@ __host__ __device__ inline int cell_index(const Grid &g, int i, int j, int k)
 __device__ inline int wrap(int i, int n)
 {
     if ((unsigned)i < (unsigned)n) return i;   // nearly always: skips the integer division
+#ifdef __HIP_DEVICE_COMPILE__
+    asm volatile("" : "+v"(n));   // the division's reciprocal stays here, not in registers of the loop around
+#endif
     int r = i % n;
     return r < 0 ? r + n : r;
 }

@@ -9,7 +9,7 @@
 //   4. k_cell_order    order every cell's slots by caller parcel index
 //                      (epic_cell_sort only: the reference's cell order)
 //   5. k_p2g_tiles     one work-group per (8x8 column tile, z chunk of tz
-//                      layers), one thread per cell: support points in FP64,
+//                      layers), one thread per parcel: support points in FP64,
 //                      each of the 4 x 8 x 7 contributions of a parcel scaled
 //                      by a per-member power of two, rounded and added to a
 //                      64-bit integer LDS accumulator of its node; the box is
@@ -29,6 +29,7 @@
 #include "launch.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace epic {
 
@@ -265,19 +266,20 @@ __global__ void k_cell_order(int64_t nc, const int *__restrict__ cell_start, con
 // ---------------------------------------------------------------------------
 // 5. tile scatter into fixed-point LDS accumulators
 // ---------------------------------------------------------------------------
-// One work-group per (8 x 8 column tile, tz cell layers), P2G_TPC threads per
-// cell taking every P2G_TPC-th parcel of it, in neighbouring lanes: a wave
-// covers 64 / P2G_TPC cells, so its loads share lines, and the points of
-// different cells' parcels rarely add to one node in the same instruction.
+// One work-group per (8 x 8 column tile, tz cell layers); its parcels are one
+// contiguous slot range, and a wave takes 64 consecutive ones at a time, so
+// every lane has a parcel and a round's loads are whole lines.
 // Every contribution w * (vol/4) * value is scaled by a power of two chosen
 // per member and field from k_p2g_max's maxima (so that no single point's
 // contribution exceeds 2^27),
 // rounded to an integer and added to a 64-bit LDS accumulator of its node;
 // the points of one parcel that fall in the same cell are combined first.
-// Most points stay in their parcel's own cell: there the two threads of the
-// cell combine their (rounded) contributions by a lane exchange and each
-// adds the pair's sum to four of the cell's eight corners, so these atomics
-// are half as many and no two lanes of an instruction hit one node.  Integer
+// Most points stay in their parcel's own cell, and neighbouring lanes mostly
+// share a cell: four lanes of one cell exchange their (rounded) own-cell
+// contributions, first the upper and lower planes within a lane pair, then
+// the rows between the pairs, and each adds the four parcels' sums to two of
+// the cell's eight corners, a quarter of the atomics.  Quads across a cell
+// boundary exchange within matching pairs only.  Integer
 // sums do not depend on the order of the additions, so the node sums are
 // bitwise reproducible however the waves are scheduled, with no ordering
 // pass and no barriers between parcels; the only rounding is that of each
@@ -305,15 +307,11 @@ __device__ inline float fixed_scale(float max_abs, int &e)
     return ldexpf(1.0f, 27 - e);
 }
 
-// the value of the other lane of a lane pair (2k, 2k+1): DPP quad
-// permutation [1, 0, 3, 2]; both lanes must be active
-__device__ inline int pair_swap(int v) { return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, false); }
-__device__ inline unsigned long long pair_swap64(unsigned long long v)
-{
-    const unsigned lo = (unsigned)pair_swap((int)(unsigned)v), hi = (unsigned)pair_swap((int)(unsigned)(v >> 32));
-    return ((unsigned long long)hi << 32) | lo;
-}
-
+// values of other lanes of a quad by DPP quad permutations (all four lanes
+// active): the other lane of the pair [1, 0, 3, 2], the same lane of the
+// other pair [2, 3, 0, 1]
+constexpr int QP_PAIR = 0xB1, QP_CROSS = 0x4E, QP_FIRST = 0x00, QP_LAST = 0xFF;
+template <int QP> __device__ inline int quad_perm(int v) { return __builtin_amdgcn_mov_dpp(v, QP, 0xF, 0xF, false); }
 // One fixed-point contribution as a 64-bit accumulator term, in one FP64
 // FMA: w * c is exact in FP64 (two FP32 factors), and adding 1.5 * 2^52
 // rounds it to the nearest integer q (ties to even) with q held in the low
@@ -326,6 +324,11 @@ __device__ inline unsigned long long fixed_term(double w, double c)
 {
     return (unsigned long long)__double_as_longlong(fma(w, c, F_MAGIC_D));
 }
+// The same term as a plain 32-bit integer (|q| < 2^29: the sum of a quad's four
+// fits too), for sums between lanes: half the lane moves, each part of its
+// addition.  fixed_wide makes an accumulator term of such a sum.
+__device__ inline int fixed_term32(double w, double c) { return (int)(unsigned)fixed_term(w, c); }
+__device__ inline unsigned long long fixed_wide(int q) { return (unsigned long long)(long long)q; }
 __device__ inline long long fixed_sum(unsigned long long acc) { return (long long)(acc << 16) >> 16; }
 
 // the gridded quantities of parcel pi, read from its arrays (o4 = 4 pi)
@@ -376,9 +379,16 @@ __global__ __launch_bounds__(256) void k_p2g_max(const P2GMaxArgs *__restrict__ 
 }
 
 // TZ (= a.tz) is a template parameter, so the LDS strides are constants and
-// the 8 x 7 atomics of a cell are its base word plus immediate offsets
+// the 8 x 7 atomics of a cell are its base word plus immediate offsets.
+//
+// What bounds it: VALU issue (the SIMDs about 80 % busy at 128^3), then the LDS
+// atomics; reads are 87 B a parcel.  One lane per consecutive slot, a quad's
+// sums exchanged before its atomics, against two lanes per cell walking the
+// cell's parcels (whose rounds each touched every line of four rows of cells,
+// 455 B read a parcel): 0.91 -> 0.69 ms a launch at 128^3 without humidity,
+// four work-groups per CU (three: 0.79).
 template <int TZ>
-__global__ __launch_bounds__(64 * TZ * P2G_TPC, 8 / TZ) void k_p2g_tiles(const P2GArgs *__restrict__ tab, const int2 *__restrict__ bmap)
+__global__ __launch_bounds__(64 * TZ * P2G_TPC, 4) void k_p2g_tiles(const P2GArgs *__restrict__ tab, const int2 *__restrict__ bmap)
 {
     const ItemBlock ib = item_block(bmap);
     const P2GArgs &a = tab[ib.item];
@@ -401,18 +411,10 @@ __global__ __launch_bounds__(64 * TZ * P2G_TPC, 8 / TZ) void k_p2g_tiles(const P
     for (int u = tid; u < P2G_NF * lfield; u += blockDim.x) acc[u] = 0ull;
     if (tid == 0) s_err = s_far = 0;
 
-    // this thread's cell and its share of the cell's parcels: the P2G_TPC
-    // threads of a cell are neighbouring lanes, so one load instruction
-    // covers 64 / P2G_TPC cells, whose parcels share fewer lines
-    const int ct = tid / P2G_TPC, sub = tid % P2G_TPC;
-    const int cx = ct & 7, cy = (ct >> 3) & 7, lz = ct >> 6;
-    const int k = k0 + lz;
-    int s0 = 0, s1 = 0;
-    if (k <= g.nz) {   // (cells of a partial tile beyond the grid are empty)
-        const int c = layer_index(g, tx, ty, k) + (ct & (TILE_CELLS - 1));
-        s0 = gl(a.cell_start)[c];
-        s1 = gl(a.cell_start)[c + 1];
-    }
+    // the chunk's parcels: one contiguous slot range of the sort
+    const int i0 = tx * P2G_TX, j0 = ty * P2G_TY, nl = min(tz, g.nz + 1 - k0);
+    const int first = gl(a.cell_start)[layer_index(g, tx, ty, k0)];
+    const int nparc = gl(a.cell_start)[layer_index(g, tx, ty, k0 + nl)] - first;
     // fixed-point scales from the member's largest contributions; with no
     // condensation anywhere the total buoyancy equals the buoyancy (field 5
     // is a copy of field 4) and with no humidity field 6 is zero: their
@@ -424,232 +426,272 @@ __global__ __launch_bounds__(64 * TZ * P2G_TPC, 8 / TZ) void k_p2g_tiles(const P
 #pragma unroll
     for (int f = 0; f < P2G_NF; ++f) {
         int e;
-        sc[f] = fixed_scale(mx[f], e);
+        sc[f] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(fixed_scale(mx[f], e))));   // uniform: a scalar register
     }
     const bool own5 = mx[P2G_NF] > 0.0f;   // tbuoy differs from buoy somewhere
     const bool own6 = mx[6] > 0.0f;        // humidity somewhere
     __syncthreads();   // the accumulators are cleared
 
-    // ---- pass 2: support points, trilinear weights, integer accumulation ----
-    // the two threads of a cell take its parcels in turns and run the same
-    // number of rounds (the odd thread idles in the last round of an odd
-    // count), so that they can exchange their own-cell contributions
-    static_assert(P2G_TPC == 2, "lane pairs");
-    const bool odd = sub != 0;
-    const int cown = (lz + 1) * lplane + (cy + 1) * lp + cx + 1;   // own cell's lower corner
-    const int nown = cown + (odd ? lplane : 0);   // this lane's four corners: the lower (even) or upper (odd) plane
-    // every lane of a wave runs the wave's largest number of rounds (the
-    // non-own cells below are shared out over the whole wave), the lanes of
-    // cells with fewer parcels idle
-    int rounds = (s1 - s0 + 1) >> 1;
-    for (int o = 32; o > 0; o >>= 1) rounds = max(rounds, __shfl_xor(rounds, o, 64));
+    // ---- support points, trilinear weights, integer accumulation ----
     const int lane = tid & 63;
+    const bool zup = lane & 1, yup = lane & 2;   // this lane's corners of an own cell: its plane and row
+    const float zsg = zup ? 1.0f : -1.0f, znr = zup ? 0.0f : 1.0f, zfr = 1.0f - znr;
+    const float ysg = yup ? 1.0f : -1.0f, ynr = yup ? 0.0f : 1.0f, yfr = 1.0f - ynr;
     const unsigned long long below = (1ull << lane) - 1ull;
     unsigned short *items = s_items[tid >> 6];
     int err = 0;
-    for (int rd = 0; rd < rounds; ++rd) {
-        const int s = s0 + 2 * rd + sub;
-        const bool have = s < s1;
-        const int pi = have ? gl(a.perm)[s] : 0;   // an idle lane reads parcel 0 and adds nothing
-        const unsigned o4 = (unsigned)pi * 4u;   // byte offset (pi < 2^30): scalar base + 32-bit offset addressing
-        const double pos[3] = {gl(a.p.x)[pi], gl(a.p.y)[pi], gl(a.p.z)[pi]};
-        const double ve[3] = {at(axes[0], o4), at(axes[1], o4), at(axes[2], o4)};
-        const double vt[3] = {at(axes[3], o4), at(axes[4], o4), at(axes[5], o4)};
-        float v[P2G_NF];
-        p2g_values(g, a.p, o4, pos[2], v);
-        double csd[P2G_NF];
+    // two copies of the loop: without humidity anywhere the condensation's
+    // exponential (whose constants would take 20 registers of the loop) and
+    // two of the fields drop out at compile time
+    auto scatter = [&](auto humid) {
+        constexpr bool HUMID = decltype(humid)::value;
+        // the lanes beyond the last parcel take it again, with zero values
+        int pi_nx = (nparc > 0) ? gl(a.perm)[first + min(tid, nparc - 1)] : 0;
+        for (int q0 = tid - lane; q0 < nparc; q0 += blockDim.x) {   // uniform over the wave
+            const int pi = pi_nx;
+            if (q0 + (int)blockDim.x < nparc) pi_nx = gl(a.perm)[first + min(q0 + (int)blockDim.x + lane, nparc - 1)];
+            bool have = q0 + lane < nparc;
+            const unsigned o4 = (unsigned)pi * 4u;   // byte offset (pi < 2^30): scalar base + 32-bit offset addressing
+            const double pos[3] = {gl(a.p.x)[pi], gl(a.p.y)[pi], gl(a.p.z)[pi]};
+            const double ve[3] = {at(axes[0], o4), at(axes[1], o4), at(axes[2], o4)};
+            const double vt[3] = {at(axes[3], o4), at(axes[4], o4), at(axes[5], o4)};
+            float v[P2G_NF];
+            if constexpr (HUMID) {
+                p2g_values(g, a.p, o4, pos[2], v);
+            } else {   // p2g_values without humidity
+                const float v0 = (float)(0.25 * (double)at(a.p.vol, o4));
+                v[0] = v0;
 #pragma unroll
-        for (int f = 0; f < P2G_NF; ++f) csd[f] = have ? (double)(v[f] * sc[f]) : 0.0;   // exact: sc is a power of two
-        int cc[3];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) cc[d] = (int)floor((pos[d] - g.lower[d]) * g.dxi[d]);
-        // the four support points: target cell (box corner index, -1 when
-        // outside the neighbour cells) and cell fractions
-        // tgt: >= 0 box corner; -1 none; < -1 a point beyond the neighbour
-        // cells, -2 - its cell offsets (7 bits each, biased by 64)
-        int tgt[4];
-        float fr[4][3];
-        unsigned farm = 0;   // bit jp: point jp lies beyond the neighbour cells
-#pragma unroll
-        for (int jp = 0; jp < 4; ++jp) {
-            const double csn = support_cos(jp), snn = support_sin(jp);
-            int off[3];
+                for (int c = 0; c < 3; ++c) v[1 + c] = v0 * at(a.p.vor[c], o4);
+                v[4] = v[5] = v0 * at(a.p.buoy, o4);
+                v[6] = 0.0f;
+            }
+            int cc[3];
+            double xr[3], su[3], sw[3];   // position in the cell and point offsets, in cells
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
-                const double pt = pos[d] + ve[d] * csn + vt[d] * snn;
-                const double xyz = (pt - g.lower[d]) * g.dxi[d];
-                const double fl = floor(xyz);
-                off[d] = (int)fl - cc[d];
-                fr[jp][d] = (float)(xyz - fl);
+                const double x = (pos[d] - g.lower[d]) * g.dxi[d], fl = floor(x);
+                cc[d] = (int)fl;
+                xr[d] = x - fl;
+                support_offsets(ve[d], vt[d], EPIC_RT2I * g.dxi[d], su[d], sw[d]);
             }
-            tgt[jp] = -1;
-            if (cc[2] + off[2] < -1 || cc[2] + off[2] > g.nz) {   // beyond the halo layers (the reference fails too)
-                if (have) err |= ERR_OUT_OF_GRID;
-            } else if (off[0] < -1 || off[0] > 1 || off[1] < -1 || off[1] > 1 || off[2] < -1 || off[2] > 1) {
-                if (have && off[0] >= -64 && off[0] < 64 && off[1] >= -64 && off[1] < 64 && off[2] >= -64 && off[2] < 64) {
-                    farm |= 1u << jp;   // beyond the neighbour cells: global accumulator, below
-                    tgt[jp] = -2 - (((off[2] + 64) << 14) | ((off[1] + 64) << 7) | (off[0] + 64));
-                } else if (have) {
-                    err |= ERR_OUT_OF_GRID;   // more than 64 cells away
-                }
-            } else {   // lower corner of the point's cell in the box
-                tgt[jp] = (lz + off[2] + 1) * lplane + (cy + off[1] + 1) * lp + cx + off[0] + 1;
+            int cx = wrap(cc[0], g.nx) - i0, cy = wrap(cc[1], g.ny) - j0, lz = cc[2] - k0;
+            if ((unsigned)cx >= (unsigned)P2G_TX || (unsigned)cy >= (unsigned)P2G_TY || (unsigned)lz >= (unsigned)tz) {
+                err |= ERR_CELL_MISMATCH;   // not in the cell it was sorted into: left out
+                have = false;
+                cx = cy = lz = 0;
             }
-        }
-        // support points beyond the neighbour cells (strongly stretched
-        // parcels, rare): each point's 8 x 7 fixed-point terms go to the
-        // member's global accumulator by 64-bit atomics (exact integer sums,
-        // so still independent of the order), which the finalize adds
-        if (farm) {
-            s_far = 1;
-            const int64_t FS = field_stride(g);
+            const int cown = __mul24(lz + 1, lplane) + __mul24(cy + 1, lp) + cx + 1;   // own cell's lower corner
+            float cs[P2G_NF];
+#pragma unroll
+            for (int f = 0; f < P2G_NF; ++f) cs[f] = have ? v[f] * sc[f] : 0.0f;   // exact: sc is a power of two
+            // the four support points: target cell (box corner index, -1 when
+            // outside the neighbour cells) and cell fractions
+            // tgt: >= 0 box corner; -1 none; < -1 a point beyond the neighbour
+            // cells, -2 - its cell offsets (7 bits each, biased by 64)
+            int tgt[4];
+            float fr[4][3];
+            unsigned farm = 0;   // bit jp: point jp lies beyond the neighbour cells
 #pragma unroll
             for (int jp = 0; jp < 4; ++jp) {
-                if (!((farm >> jp) & 1u)) continue;
-                const int code = -2 - tgt[jp];
-                const int gi[3] = {cc[0] + (code & 127) - 64, cc[1] + ((code >> 7) & 127) - 64, cc[2] + (code >> 14) - 64};
-                const float *f3 = fr[jp];
-                const float wxy[4] = {(1.0f - f3[1]) * (1.0f - f3[0]), (1.0f - f3[1]) * f3[0], f3[1] * (1.0f - f3[0]),
-                                      f3[1] * f3[0]};
+                int off[3];
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    const double r = support_coord(jp, xr[d], su[d], sw[d]), fl = floor(r);
+                    off[d] = (int)fl;
+                    fr[jp][d] = (float)(r - fl);
+                }
+                tgt[jp] = -1;
+                if (cc[2] + off[2] < -1 || cc[2] + off[2] > g.nz) {   // beyond the halo layers (the reference fails too)
+                    if (have) err |= ERR_OUT_OF_GRID;
+                } else if (off[0] < -1 || off[0] > 1 || off[1] < -1 || off[1] > 1 || off[2] < -1 || off[2] > 1) {
+                    if (have && off[0] >= -64 && off[0] < 64 && off[1] >= -64 && off[1] < 64 && off[2] >= -64 && off[2] < 64) {
+                        farm |= 1u << jp;   // beyond the neighbour cells: global accumulator, below
+                        tgt[jp] = -2 - (((off[2] + 64) << 14) | ((off[1] + 64) << 7) | (off[0] + 64));
+                    } else if (have) {
+                        err |= ERR_OUT_OF_GRID;   // more than 64 cells away
+                    }
+                } else {   // lower corner of the point's cell in the box
+                    tgt[jp] = cown + __mul24(off[2], lplane) + __mul24(off[1], lp) + off[0];
+                }
+            }
+            // support points beyond the neighbour cells (strongly stretched
+            // parcels, rare): each point's 8 x 7 fixed-point terms go to the
+            // member's global accumulator by 64-bit atomics (exact integer sums,
+            // so still independent of the order), which the finalize adds
+            if (farm) {
+                s_far = 1;
+                const int64_t FS = field_stride(g);
+#pragma unroll
+                for (int jp = 0; jp < 4; ++jp) {
+                    if (!((farm >> jp) & 1u)) continue;
+                    const int code = -2 - tgt[jp];
+                    const int gi[3] = {cc[0] + (code & 127) - 64, cc[1] + ((code >> 7) & 127) - 64, cc[2] + (code >> 14) - 64};
+                    const float *f3 = fr[jp];
+                    const float wxy[4] = {(1.0f - f3[1]) * (1.0f - f3[0]), (1.0f - f3[1]) * f3[0], f3[1] * (1.0f - f3[0]),
+                                          f3[1] * f3[0]};
 #pragma unroll 1
-                for (int c = 0; c < 8; ++c) {
-                    const int ii = wrap(gi[0] + (c & 1), g.nx), jj = wrap(gi[1] + ((c >> 1) & 1), g.ny);
-                    const int kk = gi[2] + (c >> 2);   // in [-1, nz + 1]
-                    const int64_t node = ((int64_t)(kk + 1) * g.ny + jj) * g.nx + ii;
-                    const double wd = (double)(((c & 4) ? f3[2] : 1.0f - f3[2]) * wxy[c & 3]);
+                    for (int c = 0; c < 8; ++c) {
+                        const int ii = wrap(gi[0] + (c & 1), g.nx), jj = wrap(gi[1] + ((c >> 1) & 1), g.ny);
+                        const int kk = gi[2] + (c >> 2);   // in [-1, nz + 1]
+                        const int64_t node = ((int64_t)(kk + 1) * g.ny + jj) * g.nx + ii;
+                        const double wd = (double)(((c & 4) ? f3[2] : 1.0f - f3[2]) * wxy[c & 3]);
 #pragma unroll
-                    for (int f = 0; f < P2G_NF; ++f) atomicAdd(a.far_acc + f * FS + node, fixed_term(wd, csd[f]));
+                        for (int f = 0; f < P2G_NF; ++f) atomicAdd(a.far_acc + f * FS + node, fixed_term(wd, (double)cs[f]));
+                    }
                 }
             }
-        }
-        // own cell: the summed weights (in point order) of the points in it,
-        // on this lane's four corners and on the other lane's four
-        {
-            float wn[4] = {0.0f, 0.0f, 0.0f, 0.0f}, wf[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-            bool any = false;
+            // own cell: the summed weights (in point order) of the points in it
+            // by corner, [plane][row][x], this lane's plane and row first
+            {
+                float w[2][2][2] = {};
+#pragma unroll
+                for (int jp = 0; jp < 4; ++jp) {
+                    const float *f3 = fr[jp];
+                    // near and far weight of each axis: f or 1 - f, as one FMA
+                    const float wy[2] = {fmaf(ysg, f3[1], ynr), fmaf(-ysg, f3[1], yfr)};
+                    float wz[2] = {fmaf(zsg, f3[2], znr), fmaf(-zsg, f3[2], zfr)};
+                    const float xl = 1.0f - f3[0], xu = f3[0];
+                    if (tgt[jp] != cown) wz[0] = wz[1] = 0.0f;   // adds exact zeros
+#pragma unroll
+                    for (int cy_ = 0; cy_ < 2; ++cy_) {
+                        const float wxy[2] = {wy[cy_] * xl, wy[cy_] * xu};
+#pragma unroll
+                        for (int cz_ = 0; cz_ < 2; ++cz_)
+#pragma unroll
+                            for (int c = 0; c < 2; ++c) w[cz_][cy_][c] = fmaf(wz[cz_], wxy[c], w[cz_][cy_][c]);
+                    }
+                }
+                // node of [plane][row][0]
+                const int dzn = zup ? lplane : 0, dzf = lplane - dzn, dyn = yup ? lp : 0, dyf = lp - dyn;
+                if (quad_perm<QP_FIRST>(cown) == quad_perm<QP_LAST>(cown)) {   // (a cell's slots are consecutive)
+                    const int nn = cown + dzn + dyn;
+#pragma unroll
+                    for (int f = 0; f < P2G_NF; ++f) {
+                        if (!HUMID ? f > 4 : f == 5 && !own5) continue;   // uniform over the work-group
+                        const double q = (double)cs[f];
+#pragma unroll
+                        for (int c = 0; c < 2; ++c) {
+                            const int tn = fixed_term32((double)w[0][0][c], q) + quad_perm<QP_PAIR>(fixed_term32((double)w[1][0][c], q));
+                            const int tf = fixed_term32((double)w[0][1][c], q) + quad_perm<QP_PAIR>(fixed_term32((double)w[1][1][c], q));
+                            atomicAdd(&acc[f * lfield + nn + c], fixed_wide(tn + quad_perm<QP_CROSS>(tf)));
+                        }
+                    }
+                } else {
+                    const bool match = quad_perm<QP_PAIR>(cown) == cown;
+                    const int mm = match ? -1 : 0;
+#pragma unroll
+                    for (int f = 0; f < P2G_NF; ++f) {
+                        if (!HUMID ? f > 4 : f == 5 && !own5) continue;
+                        const double q = (double)cs[f];
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const int dy = (r >> 1) ? dyf : dyn, c = r & 1;
+                            const int tf = fixed_term32((double)w[1][r >> 1][c], q);
+                            const int tn = fixed_term32((double)w[0][r >> 1][c], q);
+                            atomicAdd(&acc[f * lfield + cown + dzn + dy + c], fixed_wide(tn + (quad_perm<QP_PAIR>(tf) & mm)));
+                            if (!match) atomicAdd(&acc[f * lfield + cown + dzf + dy + c], fixed_wide(tf));
+                        }
+                    }
+                }
+            }
+            // every other cell the points reach: its 8 corners take the summed
+            // weights of its points (in point order), 8 x 7 atomics per cell.
+            // These (lane, cell) items, about one for every second parcel, are
+            // shared out over the wave: item P[k] + (rank of the lane among the
+            // lanes with more than k items) is a lane's k-th; the lanes take 64
+            // items per pass, find their source lane through a per-wave list and
+            // read its fractions, targets and values by ds_bpermute, so the
+            // atomics run with nearly every lane active (one pass per round as a
+            // rule, where a loop over the four points ran up to four sparse ones).
+            // Each item's weights and terms are the same arithmetic as in its
+            // source lane.
+            unsigned leadm = 0;   // bit jp: point jp opens a cell other than its own and earlier points'
 #pragma unroll
             for (int jp = 0; jp < 4; ++jp) {
-                if (tgt[jp] != cown) continue;
-                const float *f3 = fr[jp];
-                const float wxy[4] = {(1.0f - f3[1]) * (1.0f - f3[0]), (1.0f - f3[1]) * f3[0], f3[1] * (1.0f - f3[0]),
-                                      f3[1] * f3[0]};
-                const float zl = 1.0f - f3[2], zu = f3[2];
-                const float zn = odd ? zu : zl, zf = odd ? zl : zu;
+                bool lead = tgt[jp] >= 0 && tgt[jp] != cown && have;
 #pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    wn[c] = any ? wn[c] + zn * wxy[c] : zn * wxy[c];
-                    wf[c] = any ? wf[c] + zf * wxy[c] : zf * wxy[c];
-                }
-                any = true;
+                for (int jq = 0; jq < jp; ++jq) lead = lead && (tgt[jq] != tgt[jp]);
+                leadm |= (lead ? 1u : 0u) << jp;
             }
+            const int ni = __popc(leadm);
+            unsigned long long lb[4];
+            int pk[5];
+            pk[0] = 0;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const int node = nown + ((c >> 1) & 1) * lp + (c & 1);
-                const double wnd = (double)wn[c], wfd = (double)wf[c];
-#pragma unroll
-                for (int f = 0; f < P2G_NF; ++f) {
-                    if ((f == 5 && !own5) || (f == 6 && !own6)) continue;   // uniform over the work-group
-                    // this lane's parcel on its plane plus the other lane's parcel on it
-                    const unsigned long long t = fixed_term(wnd, csd[f]) + pair_swap64(fixed_term(wfd, csd[f]));
-                    atomicAdd(&acc[f * lfield + node], t);
-                }
+            for (int k = 0; k < 4; ++k) {
+                lb[k] = __ballot(ni > k);
+                pk[k + 1] = pk[k] + __popcll(lb[k]);
             }
-        }
-        // every other cell the points reach: its 8 corners take the summed
-        // weights of its points (in point order), 8 x 7 atomics per cell.
-        // These (lane, cell) items, about one for every second parcel, are
-        // shared out over the wave: item P[k] + (rank of the lane among the
-        // lanes with more than k items) is a lane's k-th; the lanes take 64
-        // items per pass, find their source lane through a per-wave list and
-        // read its fractions, targets and values by ds_bpermute, so the
-        // atomics run with nearly every lane active (one pass per round as a
-        // rule, where a loop over the four points ran up to four sparse ones).
-        // Each item's weights and terms are the same arithmetic as in its
-        // source lane.
-        unsigned leadm = 0;   // bit jp: point jp opens a cell other than its own and earlier points'
+            const int total = pk[4];   // uniform over the wave
+            if (total > 0) {
+                // box corners in 16 bits each; no target (also a far point) as -1
+                int tb[4];
 #pragma unroll
-        for (int jp = 0; jp < 4; ++jp) {
-            bool lead = tgt[jp] >= 0 && tgt[jp] != cown && have;
+                for (int jq = 0; jq < 4; ++jq) tb[jq] = tgt[jq] >= 0 ? tgt[jq] : -1;
+                const int t01 = (tb[0] & 0xffff) | (tb[1] << 16), t23 = (tb[2] & 0xffff) | (tb[3] << 16);
+                for (int r = 0; r < total; r += 64) {
+                    unsigned lm = leadm;
 #pragma unroll
-            for (int jq = 0; jq < jp; ++jq) lead = lead && (tgt[jq] != tgt[jp]);
-            leadm |= (lead ? 1u : 0u) << jp;
-        }
-        const int ni = __popc(leadm);
-        unsigned long long lb[4];
-        int pk[5];
-        pk[0] = 0;
+                    for (int k = 0; k < 4; ++k) {
+                        const int jp = __ffs(lm) - 1;   // the lane's k-th item: point jp
+                        lm &= lm - 1u;
+                        const int idx = pk[k] + __popcll(lb[k] & below) - r;
+                        if (k < ni && idx >= 0 && idx < 64) items[idx] = (unsigned short)(lane | (jp << 8));
+                    }
+                    __builtin_amdgcn_wave_barrier();
+                    const bool mine = r + lane < total;
+                    const unsigned e = mine ? (unsigned)items[lane] : 0u;
+                    const int sa = (int)(e & 63u) << 2, jp0 = (int)(e >> 8) & 3;
+                    float g[4][3];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            lb[k] = __ballot(ni > k);
-            pk[k + 1] = pk[k] + __popcll(lb[k]);
-        }
-        const int total = pk[4];   // uniform over the wave
-        if (total > 0) {
-            float csf[P2G_NF];
+                    for (int jq = 0; jq < 4; ++jq)
 #pragma unroll
-            for (int f = 0; f < P2G_NF; ++f) csf[f] = have ? v[f] * sc[f] : 0.0f;
-            // box corners in 16 bits each; no target (also a far point) as -1
-            int tb[4];
+                        for (int d = 0; d < 3; ++d) g[jq][d] = __int_as_float(__builtin_amdgcn_ds_bpermute(sa, __float_as_int(fr[jq][d])));
+                    float cf[P2G_NF];
 #pragma unroll
-            for (int jq = 0; jq < 4; ++jq) tb[jq] = tgt[jq] >= 0 ? tgt[jq] : -1;
-            const int t01 = (tb[0] & 0xffff) | (tb[1] << 16), t23 = (tb[2] & 0xffff) | (tb[3] << 16);
-            for (int r = 0; r < total; r += 64) {
-                unsigned lm = leadm;
+                    for (int f = 0; f < P2G_NF; ++f)
+                        cf[f] = (!HUMID ? f > 4 : f == 5 && !own5) ? 0.0f
+                                : __int_as_float(__builtin_amdgcn_ds_bpermute(sa, __float_as_int(cs[f])));
+                    const int u01 = __builtin_amdgcn_ds_bpermute(sa, t01), u23 = __builtin_amdgcn_ds_bpermute(sa, t23);
+                    __builtin_amdgcn_wave_barrier();   // the list is read before the next pass writes it
+                    if (mine) {
+                        const int tg[4] = {(int)(short)(u01 & 0xffff), u01 >> 16, (int)(short)(u23 & 0xffff), u23 >> 16};
+                        const int t = jp0 == 0 ? tg[0] : jp0 == 1 ? tg[1] : jp0 == 2 ? tg[2] : tg[3];
+                        float w[8];
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const int jp = __ffs(lm) - 1;   // the lane's k-th item: point jp
-                    lm &= lm - 1u;
-                    const int idx = pk[k] + __popcll(lb[k] & below) - r;
-                    if (k < ni && idx >= 0 && idx < 64) items[idx] = (unsigned short)(lane | (jp << 8));
-                }
-                __builtin_amdgcn_wave_barrier();
-                const bool mine = r + lane < total;
-                const unsigned e = mine ? (unsigned)items[lane] : 0u;
-                const int sa = (int)(e & 63u) << 2, jp0 = (int)(e >> 8) & 3;
-                float g[4][3];
+                        for (int c = 0; c < 8; ++c) w[c] = 0.0f;
 #pragma unroll
-                for (int jq = 0; jq < 4; ++jq)
+                        for (int jq = 0; jq < 4; ++jq) {
+                            const float *f3 = g[jq];
+                            // (no point before the leader has its target)
+                            const bool in = tg[jq] == t;
+                            const float wz[2] = {in ? 1.0f - f3[2] : 0.0f, in ? f3[2] : 0.0f};
+                            const float xl = 1.0f - f3[0], yl = 1.0f - f3[1];
+                            const float wxy[4] = {yl * xl, yl * f3[0], f3[1] * xl, f3[1] * f3[0]};
 #pragma unroll
-                    for (int d = 0; d < 3; ++d) g[jq][d] = __int_as_float(__builtin_amdgcn_ds_bpermute(sa, __float_as_int(fr[jq][d])));
-                float cf[P2G_NF];
-#pragma unroll
-                for (int f = 0; f < P2G_NF; ++f)
-                    cf[f] = ((f == 5 && !own5) || (f == 6 && !own6)) ? 0.0f
-                            : __int_as_float(__builtin_amdgcn_ds_bpermute(sa, __float_as_int(csf[f])));
-                const int u01 = __builtin_amdgcn_ds_bpermute(sa, t01), u23 = __builtin_amdgcn_ds_bpermute(sa, t23);
-                __builtin_amdgcn_wave_barrier();   // the list is read before the next pass writes it
-                if (mine) {
-                    const int tg[4] = {(int)(short)(u01 & 0xffff), u01 >> 16, (int)(short)(u23 & 0xffff), u23 >> 16};
-                    const int t = jp0 == 0 ? tg[0] : jp0 == 1 ? tg[1] : jp0 == 2 ? tg[2] : tg[3];
-                    float w[8];
-#pragma unroll
-                    for (int c = 0; c < 8; ++c) w[c] = 0.0f;
-#pragma unroll
-                    for (int jq = 0; jq < 4; ++jq) {
-                        if (jq < jp0 || (jq > jp0 && tg[jq] != t)) continue;
-                        const float *f3 = g[jq];
-                        const float wxy[4] = {(1.0f - f3[1]) * (1.0f - f3[0]), (1.0f - f3[1]) * f3[0],
-                                              f3[1] * (1.0f - f3[0]), f3[1] * f3[0]};
+                            for (int c = 0; c < 8; ++c) {
+                                const float wc = wz[c >> 2] * wxy[c & 3];
+                                w[c] = w[c] + wc;
+                            }
+                        }
 #pragma unroll
                         for (int c = 0; c < 8; ++c) {
-                            const float wc = ((c & 4) ? f3[2] : 1.0f - f3[2]) * wxy[c & 3];
-                            w[c] = (jq == jp0) ? wc : w[c] + wc;
-                        }
-                    }
+                            const int node = t + (c >> 2) * lplane + ((c >> 1) & 1) * lp + (c & 1);
+                            const double wd = (double)w[c];
 #pragma unroll
-                    for (int c = 0; c < 8; ++c) {
-                        const int node = t + (c >> 2) * lplane + ((c >> 1) & 1) * lp + (c & 1);
-                        const double wd = (double)w[c];
-#pragma unroll
-                        for (int f = 0; f < P2G_NF; ++f) {
-                            if ((f == 5 && !own5) || (f == 6 && !own6)) continue;   // uniform over the work-group
-                            atomicAdd(&acc[f * lfield + node], fixed_term(wd, (double)cf[f]));
+                            for (int f = 0; f < P2G_NF; ++f) {
+                                if (!HUMID ? f > 4 : f == 5 && !own5) continue;   // uniform over the work-group
+                                atomicAdd(&acc[f * lfield + node], fixed_term(wd, (double)cf[f]));
+                            }
                         }
                     }
                 }
             }
         }
-    }
+    };
+    if (own6) scatter(std::true_type{});
+    else scatter(std::false_type{});
     if (err) atomicOr(&s_err, err);
     __syncthreads();
 
@@ -922,8 +964,6 @@ __global__ __launch_bounds__(64) void k_far_reset(const FarClearArgs *__restrict
     if (threadIdx.x == 0) gl(tab[ib.item].far_flag)[0] = 0;
 }
 
-constexpr size_t P2G_LDS_FLOOR = 160 * 1024 / 4 + 256;   // admits three work-groups per CU, not four
-
 void add_p2g(Plan &P, int phase, const std::vector<P2GArgs> &tiles, const std::vector<FinalizeArgs> &fin,
              const std::vector<FarClearArgs> &far)
 {
@@ -942,12 +982,7 @@ void add_p2g(Plan &P, int phase, const std::vector<P2GArgs> &tiles, const std::v
             nb.push_back(a.ntx * a.nty * a.nchz);
         }
         const void *k = tz == 2 ? (const void *)k_p2g_tiles<2> : tz == 4 ? (const void *)k_p2g_tiles<4> : (const void *)k_p2g_tiles<8>;
-        // at least a third of the CU's LDS a work-group: with four work-groups
-        // of tz = 2 on a CU, the rows of parcels their waves touch leave the
-        // L2 between a wave's rounds (the tile scatter 1.6 % slower than with
-        // three); larger tz need more than that anyway
-        const size_t lds = std::max<size_t>(p2g_lds_bytes(tz), P2G_LDS_FLOOR);
-        P.add(k, 64 * tz * P2G_TPC, lds, phase == PH_P2G ? (int)PH_P2G_TILES : phase, items, nb);
+        P.add(k, 64 * tz * P2G_TPC, p2g_lds_bytes(tz), phase == PH_P2G ? (int)PH_P2G_TILES : phase, items, nb);
     }
     std::vector<int> nf;
     for (const FinalizeArgs &f : fin) nf.push_back((int)(((int64_t)f.g.nx * f.g.ny * (f.g.nz + 3) + 255) / 256));
