@@ -16,6 +16,7 @@
 #include "epic_gpu.h"
 #include "common.h"
 #include "fft.h"
+#include "hostio.h"
 #include "launch.h"
 #include "plan.h"
 
@@ -783,23 +784,29 @@ int field_slot(int which)
     }
 }
 
-template <typename T> int copy_field_out(epic_member *m, const T *dev, int ncomp, double *out)
+// the caller's parcel arrays and their device arrays (host pointers may be
+// null or, for an upload, point to constant data that is only read)
+std::vector<IoGroup> parcel_groups(epic_member *m, const double *position, const double *vorticity, const double *B,
+                                   const double *volume, const double *buoyancy, const double *humidity)
 {
-    const Grid &g = m->g;
-    const int64_t FS = field_stride(g);
-    std::vector<T> h((size_t)(FS * ncomp));
-    HIPOK(m, hipMemcpyAsync(h.data(), dev, sizeof(T) * h.size(), hipMemcpyDeviceToHost, m->s));
-    HIPOK(m, hipStreamSynchronize(m->s));
-    const int64_t H = (int64_t)(g.nz + 3) * (g.ny + 3) * (g.nx + 3);
-    for (int c = 0; c < ncomp; ++c)
-        for (int ix = -1; ix <= g.nx + 1; ++ix)
-            for (int iy = -1; iy <= g.ny + 1; ++iy) {
-                const int wx = (ix + g.nx) % g.nx, wy = (iy + g.ny) % g.ny;
-                double *o = out + c * H + ((int64_t)(ix + 1) * (g.ny + 3) + (iy + 1)) * (g.nz + 3);
-                const T *src = h.data() + c * FS + (int64_t)wy * g.nx + wx;
-                for (int iz = -1; iz <= g.nz + 1; ++iz) o[iz + 1] = (double)src[(int64_t)(iz + 1) * g.ny * g.nx];
-            }
-    return EPIC_OK;
+    const ParcelsDev &p = m->pd;
+    auto h = [](const double *a) { return const_cast<double *>(a); };
+    return {IoGroup{3, true, {p.x, p.y, p.z}, h(position)},
+            IoGroup{3, false, {p.vor[0], p.vor[1], p.vor[2]}, h(vorticity)},
+            IoGroup{5, false, {p.B[0], p.B[1], p.B[2], p.B[3], p.B[4]}, h(B)},
+            IoGroup{1, false, {p.vol}, h(volume)},
+            IoGroup{1, false, {p.buoy}, h(buoyancy)},
+            IoGroup{1, false, {p.hum}, h(humidity)}};
+}
+
+std::vector<IoGroup> tendency_groups(epic_member *m, const double *delta_pos, const double *delta_vor, const double *strain)
+{
+    const ParcelsDev &p = m->pd;
+    auto h = [](const double *a) { return const_cast<double *>(a); };
+    IoGroup st{8, false, {}, h(strain)};
+    for (int d = 0; d < 8; ++d) st.dev[d] = p.strain[d];
+    return {IoGroup{3, false, {p.dpos[0], p.dpos[1], p.dpos[2]}, h(delta_pos)},
+            IoGroup{3, false, {p.dvor[0], p.dvor[1], p.dvor[2]}, h(delta_vor)}, st};
 }
 
 }  // namespace
@@ -984,30 +991,12 @@ int epic_set_parcels(epic_handle m, int64_t n, const double *position, const dou
     if (n < 0 || n > m->cap) return fail(m, EPIC_E_CAPACITY, "epic_set_parcels: more parcels than max_parcels");
     if (n > 0 && (!position || !vorticity || !B || !volume || !buoyancy || !humidity))
         return fail(m, EPIC_E_INVALID, "epic_set_parcels: null array");
-    const int64_t c = m->cap;
-    std::vector<double> hp(3 * (size_t)n);
-    std::vector<float> ha((size_t)11 * n);
-    std::vector<int> ho(n);
-    host_parallel_for(n, [&](int64_t lo, int64_t hi) {
-        for (int64_t q = lo; q < hi; ++q) {
-            for (int d = 0; d < 3; ++d) hp[d * n + q] = position[3 * q + d];
-            for (int d = 0; d < 3; ++d) ha[d * n + q] = (float)vorticity[3 * q + d];
-            for (int d = 0; d < 5; ++d) ha[(3 + d) * n + q] = (float)B[5 * q + d];
-            ha[8 * n + q] = (float)volume[q];
-            ha[9 * n + q] = (float)buoyancy[q];
-            ha[10 * n + q] = (float)humidity[q];
-            ho[q] = (int)q;
-        }
-    });
     m->n = n;
     HIPOK(m, bind_parcels(m));
     m->counts_changed();
-    for (int d = 0; d < 3 && n; ++d)
-        HIPOK(m, hipMemcpyAsync(m->pos + d * c, hp.data() + d * n, sizeof(double) * n, hipMemcpyHostToDevice, m->s));
-    for (int a = 0; a < 11 && n; ++a)
-        HIPOK(m, hipMemcpyAsync(m->attr + a * c, ha.data() + a * n, sizeof(float) * n, hipMemcpyHostToDevice, m->s));
-    if (n) HIPOK(m, hipMemcpyAsync(m->orig, ho.data(), sizeof(int) * n, hipMemcpyHostToDevice, m->s));
-    HIPOK(m, hipStreamSynchronize(m->s));
+    HIPOK(m, launch_iota(n, m->orig, m->s));
+    HIPOK(m, upload_parcels(n, nullptr, nullptr, parcel_groups(m, position, vorticity, B, volume, buoyancy, humidity), m->s));
+    HIPOK(m, hipStreamSynchronize(m->s));   // (nothing was uploaded when n is 0)
     m->keys_valid = false;
     m->axes_dirty = true;
     m->tend_displaced = false;
@@ -1019,30 +1008,8 @@ int epic_get_parcels(epic_handle m, int64_t n, double *position, double *vortici
 {
     if (!m) return EPIC_E_INVALID;
     if (n != m->n) return fail(m, EPIC_E_INVALID, "epic_get_parcels: n differs from the stored parcel count");
-    const int64_t c = m->cap;
-    std::vector<double> hp(3 * (size_t)n);
-    std::vector<float> ha((size_t)11 * n);
-    std::vector<int> ho(n);
-    for (int d = 0; d < 3 && n; ++d)
-        HIPOK(m, hipMemcpyAsync(hp.data() + d * n, m->pos + d * c, sizeof(double) * n, hipMemcpyDeviceToHost, m->s));
-    for (int a = 0; a < 11 && n; ++a)
-        HIPOK(m, hipMemcpyAsync(ha.data() + a * n, m->attr + a * c, sizeof(float) * n, hipMemcpyDeviceToHost, m->s));
-    if (n) HIPOK(m, hipMemcpyAsync(ho.data(), m->orig, sizeof(int) * n, hipMemcpyDeviceToHost, m->s));
-    HIPOK(m, hipStreamSynchronize(m->s));
-    host_parallel_for(n, [&](int64_t lo, int64_t hi) {   // orig is a permutation: one writer per element
-        for (int64_t q = lo; q < hi; ++q) {
-            const int64_t o = ho[q];
-            if (position)
-                for (int d = 0; d < 3; ++d) position[3 * o + d] = hp[d * n + q];
-            if (vorticity)
-                for (int d = 0; d < 3; ++d) vorticity[3 * o + d] = ha[d * n + q];
-            if (B)
-                for (int d = 0; d < 5; ++d) B[5 * o + d] = ha[(3 + d) * n + q];
-            if (volume) volume[o] = ha[8 * n + q];
-            if (buoyancy) buoyancy[o] = ha[9 * n + q];
-            if (humidity) humidity[o] = ha[10 * n + q];
-        }
-    });
+    // perm is scratch between calls
+    HIPOK(m, download_parcels(n, m->orig, m->perm, parcel_groups(m, position, vorticity, B, volume, buoyancy, humidity), m->s));
     return EPIC_OK;
 }
 
@@ -1054,25 +1021,7 @@ int epic_get_parcel_tendencies(epic_handle m, int64_t n, double *delta_pos, doub
         const int rc = settle_tendencies(m);
         if (rc) return rc;
     }
-    const int64_t c = m->cap;
-    std::vector<float> h((size_t)14 * n);
-    std::vector<int> ho(n);
-    for (int a = 0; a < 6 && n; ++a)
-        HIPOK(m, hipMemcpyAsync(h.data() + a * n, m->attr + (11 + a) * c, sizeof(float) * n, hipMemcpyDeviceToHost, m->s));
-    for (int a = 0; a < 8 && n; ++a)
-        HIPOK(m, hipMemcpyAsync(h.data() + (6 + a) * n, m->attr + (28 + a) * c, sizeof(float) * n,
-                                hipMemcpyDeviceToHost, m->s));
-    if (n) HIPOK(m, hipMemcpyAsync(ho.data(), m->orig, sizeof(int) * n, hipMemcpyDeviceToHost, m->s));
-    HIPOK(m, hipStreamSynchronize(m->s));
-    for (int64_t q = 0; q < n; ++q) {
-        const int64_t o = ho[q];
-        for (int d = 0; d < 3; ++d) {
-            if (delta_pos) delta_pos[3 * o + d] = h[d * n + q];
-            if (delta_vor) delta_vor[3 * o + d] = h[(3 + d) * n + q];
-        }
-        if (strain)
-            for (int d = 0; d < 8; ++d) strain[8 * o + d] = h[(6 + d) * n + q];
-    }
+    HIPOK(m, download_parcels(n, m->orig, m->perm, tendency_groups(m, delta_pos, delta_vor, strain), m->s));
     return EPIC_OK;
 }
 
@@ -1084,19 +1033,9 @@ int epic_set_parcel_tendencies(epic_handle m, int64_t n, const double *delta_pos
         const int rc = settle_tendencies(m);
         if (rc) return rc;
     }
-    const int64_t c = m->cap;
-    std::vector<int> ho(n);
-    if (n) HIPOK(m, hipMemcpyAsync(ho.data(), m->orig, sizeof(int) * n, hipMemcpyDeviceToHost, m->s));
-    HIPOK(m, hipStreamSynchronize(m->s));
-    std::vector<float> h((size_t)6 * n);
-    for (int64_t q = 0; q < n; ++q)
-        for (int d = 0; d < 3; ++d) {
-            h[d * n + q] = delta_pos ? (float)delta_pos[3 * ho[q] + d] : 0.0f;
-            h[(3 + d) * n + q] = delta_vor ? (float)delta_vor[3 * ho[q] + d] : 0.0f;
-        }
-    for (int a = 0; a < 6 && n; ++a)
-        HIPOK(m, hipMemcpyAsync(m->attr + (11 + a) * c, h.data() + a * n, sizeof(float) * n, hipMemcpyHostToDevice, m->s));
-    HIPOK(m, hipStreamSynchronize(m->s));
+    std::vector<IoGroup> g = tendency_groups(m, delta_pos, delta_vor, nullptr);
+    g.pop_back();   // strain stays
+    HIPOK(m, upload_parcels(n, m->orig, m->perm, g, m->s));
     return EPIC_OK;
 }
 
@@ -1106,8 +1045,9 @@ int epic_get_field(epic_handle m, int which, double *out)
     const int nc = field_ncomp(which);
     if (nc == 0) return fail(m, EPIC_E_INVALID, "epic_get_field: unknown field");
     if (which == EPIC_FIELD_NPARG || which == EPIC_FIELD_NSPARG)
-        return copy_field_out(m, which == EPIC_FIELD_NPARG ? m->nparg : m->nsparg, 1, out);
-    return copy_field_out(m, m->fld + field_slot(which) * field_stride(m->g), nc, out);
+        HIPOK(m, download_field(m->g, which == EPIC_FIELD_NPARG ? m->nparg : m->nsparg, 1, out, m->s));
+    else HIPOK(m, download_field(m->g, m->fld + field_slot(which) * field_stride(m->g), nc, out, m->s));
+    return EPIC_OK;
 }
 
 int epic_get_field_int(epic_handle m, int which, int *out)
@@ -1115,12 +1055,7 @@ int epic_get_field_int(epic_handle m, int which, int *out)
     if (!m || !out) return EPIC_E_INVALID;
     if (which != EPIC_FIELD_NPARG && which != EPIC_FIELD_NSPARG)
         return fail(m, EPIC_E_INVALID, "epic_get_field_int: not an integer field");
-    const Grid &g = m->g;
-    const int64_t H = (int64_t)(g.nz + 3) * (g.ny + 3) * (g.nx + 3);
-    std::vector<double> tmp((size_t)H);
-    int rc = copy_field_out(m, which == EPIC_FIELD_NPARG ? m->nparg : m->nsparg, 1, tmp.data());
-    if (rc) return rc;
-    for (int64_t i = 0; i < H; ++i) out[i] = (int)tmp[i];
+    HIPOK(m, download_field(m->g, which == EPIC_FIELD_NPARG ? m->nparg : m->nsparg, 1, out, m->s));
     return EPIC_OK;
 }
 
@@ -1130,17 +1065,7 @@ int epic_set_field(epic_handle m, int which, const double *in)
     const int nc = field_ncomp(which);
     const int slot = field_slot(which);
     if (nc == 0 || slot < 0) return fail(m, EPIC_E_INVALID, "epic_set_field: unknown or read-only field");
-    const Grid &g = m->g;
-    const int64_t FS = field_stride(g), H = (int64_t)(g.nz + 3) * (g.ny + 3) * (g.nx + 3);
-    std::vector<float> h((size_t)(FS * nc));
-    for (int c = 0; c < nc; ++c)
-        for (int ix = 0; ix < g.nx; ++ix)
-            for (int iy = 0; iy < g.ny; ++iy)
-                for (int iz = -1; iz <= g.nz + 1; ++iz)
-                    h[c * FS + (int64_t)(iz + 1) * g.ny * g.nx + (int64_t)iy * g.nx + ix] =
-                        (float)in[c * H + ((int64_t)(ix + 1) * (g.ny + 3) + (iy + 1)) * (g.nz + 3) + (iz + 1)];
-    HIPOK(m, hipMemcpyAsync(m->fld + slot * FS, h.data(), sizeof(float) * h.size(), hipMemcpyHostToDevice, m->s));
-    HIPOK(m, hipStreamSynchronize(m->s));
+    HIPOK(m, upload_field(m->g, m->fld + slot * field_stride(m->g), nc, in, m->s));
     return EPIC_OK;
 }
 
