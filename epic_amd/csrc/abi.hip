@@ -54,7 +54,7 @@ struct epic_member {
     int *keys = nullptr, *cnt[3] = {}, *scnt[3] = {};
     int *cell_start = nullptr, *cursor = nullptr, *perm = nullptr, *bsum = nullptr;
     bool keys_valid = false;
-    int tz_p2g = 2, tz_g2p = 2;     // z chunk of the tile kernels (autotuned)
+    int tz_p2g = 2, tz_g2p = 2;     // z chunk of the tile kernels (p2g_default_tz, the autotuner)
     // fields
     float *fld = nullptr;
     int *nparg = nullptr, *nsparg = nullptr;
@@ -398,9 +398,8 @@ P2GLayout layout_tz(const Grid &g, int tz)
     return L;
 }
 
-// z chunks the autotuner may choose (par2grid: 64 tz P2G_TPC threads per work-group;
-// both stage a node box of tz + 3 planes in LDS); the staging buffer fits
-// every par2grid candidate
+// z chunks the autotuner may choose (both tile kernels hold a node box of
+// tz + 3 planes in LDS); the staging buffer fits every par2grid candidate
 const int TZ_P2G[3] = {2, 4, 8};
 const int TZ_G2P[3] = {2, 4, 8};
 
@@ -874,6 +873,7 @@ int epic_create(const epic_grid_t *grid, const epic_phys_t *phys, const epic_fla
     for (int i = 0; i < 3; ++i) g.f_cor[i] = phys->f_cor[i];
     m->rk_order = flags->rk_order;
     m->cap = std::max<int64_t>(max_parcels, 1);
+    m->tz_p2g = p2g_layout(g).tz;
     {   // a transform work-group holds ZB lines (or a column) in LDS
         int dev = 0, lds_max = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
@@ -907,7 +907,7 @@ int epic_create(const epic_grid_t *grid, const epic_phys_t *phys, const epic_fla
     const int64_t FS = field_stride(g);
     if (bad(dalloc(&m->fld, (int64_t)F_COUNT * FS, m->s)) || bad(dalloc(&m->nparg, FS, m->s)) || bad(dalloc(&m->nsparg, FS, m->s)) ||
         bad(dalloc(&m->staging, staging_elems_max(g), m->s)) ||
-        bad(dalloc(&m->far_acc, (int64_t)P2G_NF * FS, m->s)) || bad(dalloc(&m->far_flag, 1, m->s)) ||
+        bad(dalloc(&m->far_acc, (int64_t)P2G_NF * FS, m->s)) || bad(dalloc(&m->far_flag, 2, m->s)) ||
         bad(dalloc(&m->far_scale, P2G_NF, m->s)))
         return EPIC_E_NOMEM;
     // vorticity_tendency's 3 (nz + 1) ny nx doubles: a spectrum holds more than nx/2 (nz + 1) ny of them
@@ -1444,7 +1444,7 @@ int64_t epic_member_bytes(const epic_grid_t *grid, int64_t max_parcels)
     b += 4 * (6 * nc + (nc + 1) + nc);                                        // histograms, cell_start, cursor
     b += 4 * scan_scratch_ints(std::max<int64_t>(std::max<int64_t>(nc, c), (int64_t)(g.nx + 3) * (g.ny + 3) * (g.nz + 2)));
     b += 4 * ((int64_t)F_COUNT * FS + 2 * FS) + 8 * staging_elems_max(g);   // fields, counts, staging
-    b += 8 * (int64_t)P2G_NF * FS + 4 + 8 * P2G_NF;                          // far-point sums
+    b += 8 * (int64_t)P2G_NF * FS + 8 + 8 * P2G_NF;                          // far-point sums
     b += 20 * c + 4096;                                                       // merge scratch (its first phase)
     b += (int64_t)NSPEC * 8 * spec_size(g);                                  // spectra
     return b;

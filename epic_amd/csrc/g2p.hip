@@ -135,10 +135,10 @@ __global__ __launch_bounds__(256) void k_grid2par(const G2PArgs *__restrict__ ta
 // parcel is loaded one round ahead, and parcel arrays are addressed as a
 // table pointer plus a 32-bit byte offset.
 // ---------------------------------------------------------------------------
-constexpr int G2P_THREADS = 256;
 size_t g2p_lds_bytes(int tz) { return (3 * sizeof(float4) + sizeof(float2)) * (tz + 3) * P2G_BOX * P2G_BOX; }
 
-__global__ __launch_bounds__(G2P_THREADS, 4) void k_g2p_tiles(const G2PTileArgs *__restrict__ tab, const int2 *__restrict__ bmap)
+template <int NT>
+__global__ __launch_bounds__(NT, 4) void k_g2p_tiles(const G2PTileArgs *__restrict__ tab, const int2 *__restrict__ bmap)
 {
     const ItemBlock ib = item_block(bmap);
     const G2PTileArgs &a = tab[ib.item];
@@ -163,19 +163,19 @@ __global__ __launch_bounds__(G2P_THREADS, 4) void k_g2p_tiles(const G2PTileArgs 
     if (tid <= P2G_NF) s_pmax[tid] = 0u;   // ordered by the barrier after the box is staged
 
     // ---- stage the node box (plane P = k0 - 1 + lp) ----
-    // thread = (node of the 11 x 11 box column, half of the 14 fields): the
-    // wrapped column offset is found once, then the thread walks the planes
-    // with its 7 loads in flight at a time
-    static_assert(NN <= 128 && G2P_THREADS == 256, "two threads per box node column");
+    // thread = (node of the 11 x 11 box column, half of the 14 fields, every
+    // NT / 256-th plane): the wrapped column offset is found once, then the
+    // thread walks its planes with its 7 loads in flight at a time
+    static_assert(NN <= 128 && NT % 256 == 0, "two threads per box node column");
     {
-        const int node = tid & 127, half = tid >> 7;
+        const int node = tid & 127, half = (tid >> 7) & 1;
         if (node < NN) {
             const int ly = node / P2G_BOX, lx = node - ly * P2G_BOX;
             int gi = i0 - 1 + lx, gj = j0 - 1 + ly;   // in [-1, n + 9]
             gi = (gi < 0) ? gi + g.nx : (gi >= g.nx ? gi - g.nx : gi);
             gj = (gj < 0) ? gj + g.ny : (gj >= g.ny ? gj - g.ny : gj);
             const EPIC_GLOBAL float *col = gl(a.fld) + (int64_t)(F_VELOG + half) * FS + (int64_t)gj * g.nx + gi;
-            for (int lp = 0; lp < nbox; ++lp) {
+            for (int lp = tid >> 8; lp < nbox; lp += NT / 256) {
                 const int P = k0 - 1 + lp;
                 const bool in = (P >= -1 && P <= g.nz + 1);
                 const int64_t po = (int64_t)(P + 1) * PS;
@@ -216,12 +216,12 @@ __global__ __launch_bounds__(G2P_THREADS, 4) void k_g2p_tiles(const G2PTileArgs 
         pi_nx = gl(a.perm)[first + tid];
         prefetch(pi_nx);
     }
-    for (int base = 0; base < total; base += G2P_THREADS) {   // uniform rounds: the ballot needs every lane
+    for (int base = 0; base < total; base += NT) {   // uniform rounds: the ballot needs every lane
         const int q = base + tid;
         const int pi = pi_nx;
         const unsigned o4 = (unsigned)pi * 4u;   // byte offset (pi < 2^30): scalar base + 32-bit offset addressing
-        const bool more = q + G2P_THREADS < total;
-        if (more) pi_nx = gl(a.perm)[first + q + G2P_THREADS];
+        const bool more = q + NT < total;
+        if (more) pi_nx = gl(a.perm)[first + q + NT];
         double pos[3] = {pn[0], pn[1], pn[2]};
         const double ve[3] = {an[0], an[1], an[2]};
         const double vt[3] = {an[3], an[4], an[5]};
@@ -418,11 +418,15 @@ void add_rk_stage_tiles(Plan &P, int phase, const std::vector<G2PTileArgs> &item
 {
     std::vector<int> nb;
     size_t lds = 0;
+    int64_t total = 0;
     for (const G2PTileArgs &a : items) {
         nb.push_back(a.ntx * a.nty * a.nchz);
+        total += nb.back();
         lds = std::max(lds, g2p_lds_bytes(a.tz));
     }
-    P.add((const void *)k_g2p_tiles, G2P_THREADS, lds, phase, items, nb);
+    const int nt = tile_threads(total);
+    const void *k = nt == 1024 ? (const void *)k_g2p_tiles<1024> : nt == 512 ? (const void *)k_g2p_tiles<512> : (const void *)k_g2p_tiles<256>;
+    P.add(k, nt, lds, phase, items, nb);
 }
 
 void add_grid2par(Plan &P, int phase, const std::vector<G2PArgs> &items)

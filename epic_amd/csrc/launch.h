@@ -13,6 +13,14 @@ namespace epic {
 // parcels of one item are processed PER_BLOCK at a time by a 256-thread block
 constexpr int PER_BLOCK = 1024;
 
+// Threads of a tile kernel's work-group (about 1024 parcels at tz = 2) in a
+// launch of n of them.  Four 256-thread work-groups fill a CU and overlap
+// their phases; while there are fewer than that, larger ones take a tile's
+// parcels in fewer rounds.  Push per step at 256, 512, 1024 threads, in us:
+// 36 work-groups (16^3) 270, 193, 158; 117 (24^3) 295, 214, 176; 272 (32^3)
+// 315, 231, 263; 612 (48x48x32) 386, 400, 437; 2112 (64^3) 1027, 1109, 1315.
+inline int tile_threads(int64_t n) { return n <= 256 ? 1024 : n <= 512 ? 512 : 256; }
+
 // ---- cell sort (p2g.hip) ----
 struct KeysArgs {
     Grid g;
@@ -33,9 +41,10 @@ struct PlaceArgs {
     int64_t cap = 0;   // grid size in parcels (0: n)
     const int64_t *n_dev = nullptr;   // when set, the count is read from here instead of n
 };
+constexpr int64_t SCAN_FUSED_BLOCKS = 8192;
 int64_t scan_scratch_ints(int64_t n);
 void add_cell_keys(Plan &P, int phase, const std::vector<KeysArgs> &items);
-void add_exclusive_scan(Plan &P, int phase, const std::vector<ScanArgs> &items);   // three launches
+void add_exclusive_scan(Plan &P, int phase, const std::vector<ScanArgs> &items);   // two or three launches
 void add_place(Plan &P, int phase, const std::vector<PlaceArgs> &items);
 // order of every cell by caller index (epic_cell_sort only; a direct launch)
 void launch_cell_order(int64_t nc, const int *cell_start, const int *perm_tmp, const int *orig, int *perm,
@@ -47,6 +56,11 @@ struct AxesArgs {
     float *ax[6];   // Veta (3), Vtau (3)
     int *err;
 };
+// default z chunk of the tile scatter: 4 layers where that still leaves four
+// work-groups of 1024 parcels per CU.  Boxes of 7 planes for 4 layers stage
+// 30 % less than of 5 for 2 (par2grid per step: 5.46 -> 5.20 ms at 128^3, 0.94
+// -> 0.90 at 64^3); smaller grids need the work-groups (32^3: 0.42 -> 0.43).
+inline int p2g_default_tz(int ntx, int nty, int nz) { return (int64_t)ntx * nty * ((nz + 5) / 4) >= 1024 ? 4 : 2; }
 struct P2GLayout {
     int tz, ntx, nty, nchz;
     int64_t staging_elems;   // FP64 values
@@ -98,7 +112,7 @@ struct FinalizeArgs {
 // clears far_acc and then far_flag after a finalize that read them
 struct FarClearArgs {
     unsigned long long *far_acc;
-    int *far_flag;
+    int *far_flag;                     // [0] the flag, [1] the clearing blocks' count, kept at 0
     int64_t n;                         // P2G_NF * field_stride
 };
 void add_axes(Plan &P, int phase, const std::vector<AxesArgs> &items);

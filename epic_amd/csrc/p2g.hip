@@ -75,32 +75,39 @@ __global__ __launch_bounds__(256) void k_cell_keys(const KeysArgs *__restrict__ 
 }
 
 // ---------------------------------------------------------------------------
-// 2. exclusive scan (three passes, 1024 elements per block)
+// 2. exclusive scan: block sums, then every block's own prefix.  A block of
+// the second pass adds up the sums before it itself, so there is no launch
+// for the sums' scan (up to SCAN_FUSED_BLOCKS of them: 32 KB each re-reads)
 // ---------------------------------------------------------------------------
 constexpr int SCAN_T = 256;
-constexpr int SCAN_PER = 4;
+constexpr int SCAN_PER = 8;
 constexpr int SCAN_BLOCK = SCAN_T * SCAN_PER;
 
 __device__ inline int block_excl_scan(int v, int *lds, int &total)
 {
-    const int t = threadIdx.x;
-    lds[t] = v;
-    __syncthreads();
-    for (int off = 1; off < SCAN_T; off <<= 1) {
-        int a = (t >= off) ? lds[t - off] : 0;
-        __syncthreads();
-        lds[t] += a;
-        __syncthreads();
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int incl = v;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int a = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += a;
     }
-    total = lds[SCAN_T - 1];
-    const int incl = lds[t];
+    if (lane == 63) lds[w] = incl;
     __syncthreads();
-    return incl - v;
+    int base = 0;
+    total = 0;
+#pragma unroll
+    for (int u = 0; u < SCAN_T / 64; ++u) {
+        if (u < w) base += lds[u];
+        total += lds[u];
+    }
+    __syncthreads();
+    return base + incl - v;
 }
 
 __global__ __launch_bounds__(SCAN_T) void k_scan_reduce(const ScanArgs *__restrict__ tab, const int2 *__restrict__ bmap)
 {
-    __shared__ int lds[SCAN_T];
+    __shared__ int lds[SCAN_T / 64];
     const ItemBlock ib = item_block(bmap);
     const ScanArgs &a = tab[ib.item];
     const int64_t base = ib.blk * (int64_t)SCAN_BLOCK + threadIdx.x * SCAN_PER;
@@ -116,7 +123,7 @@ __global__ __launch_bounds__(SCAN_T) void k_scan_reduce(const ScanArgs *__restri
 // one block per item: exclusive scan of the item's block sums in place
 __global__ __launch_bounds__(SCAN_T) void k_scan_blocks(const ScanArgs *__restrict__ tab, const int2 *__restrict__ bmap)
 {
-    __shared__ int lds[SCAN_T];
+    __shared__ int lds[SCAN_T / 64];
     const ItemBlock ib = item_block(bmap);
     const ScanArgs &a = tab[ib.item];
     const int nb = (int)((a.n + SCAN_BLOCK - 1) / SCAN_BLOCK);
@@ -143,10 +150,12 @@ __global__ __launch_bounds__(SCAN_T) void k_scan_blocks(const ScanArgs *__restri
 }
 
 // out[c] = exclusive prefix, out[n] = total; clears gl(a.clear)[c] (the
-// placement cursors) on the way
+// placement cursors) on the way.  FUSED: bsum holds the blocks' sums, not yet
+// their prefixes
+template <bool FUSED>
 __global__ __launch_bounds__(SCAN_T) void k_scan_apply(const ScanArgs *__restrict__ tab, const int2 *__restrict__ bmap)
 {
-    __shared__ int lds[SCAN_T];
+    __shared__ int lds[SCAN_T / 64];
     const ItemBlock ib = item_block(bmap);
     const ScanArgs &a = tab[ib.item];
     const int64_t n = a.n;
@@ -158,7 +167,16 @@ __global__ __launch_bounds__(SCAN_T) void k_scan_apply(const ScanArgs *__restric
         s += v[u];
     }
     int total;
-    int run = block_excl_scan(s, lds, total) + gl(a.bsum)[ib.blk];
+    int run = block_excl_scan(s, lds, total);
+    if constexpr (FUSED) {
+        int before = 0;
+        for (int b = threadIdx.x; b < ib.blk; b += SCAN_T) before += gl(a.bsum)[b];
+        int all;
+        (void)block_excl_scan(before, lds, all);
+        run += all;
+    } else {
+        run += gl(a.bsum)[ib.blk];
+    }
 #pragma unroll
     for (int u = 0; u < SCAN_PER; ++u) {
         if (base + u < n) {
@@ -179,8 +197,12 @@ void add_exclusive_scan(Plan &P, int phase, const std::vector<ScanArgs> &items)
         one.push_back(1);
     }
     P.add((const void *)k_scan_reduce, SCAN_T, 0, phase, items, nb);
+    if (*std::max_element(nb.begin(), nb.end()) <= SCAN_FUSED_BLOCKS) {
+        P.add((const void *)k_scan_apply<true>, SCAN_T, 0, phase, items, nb);
+        return;
+    }
     P.add((const void *)k_scan_blocks, SCAN_T, 0, phase, items, one);
-    P.add((const void *)k_scan_apply, SCAN_T, 0, phase, items, nb);
+    P.add((const void *)k_scan_apply<false>, SCAN_T, 0, phase, items, nb);
 }
 
 int64_t scan_scratch_ints(int64_t n) { return (n + SCAN_BLOCK - 1) / SCAN_BLOCK + 1; }
@@ -388,7 +410,7 @@ __global__ __launch_bounds__(256) void k_p2g_max(const P2GMaxArgs *__restrict__ 
 // 455 B read a parcel): 0.91 -> 0.69 ms a launch at 128^3 without humidity,
 // four work-groups per CU (three: 0.79).
 template <int TZ>
-__global__ __launch_bounds__(64 * TZ * P2G_TPC, 4) void k_p2g_tiles(const P2GArgs *__restrict__ tab, const int2 *__restrict__ bmap)
+__global__ __launch_bounds__(1024, 4) void k_p2g_tiles(const P2GArgs *__restrict__ tab, const int2 *__restrict__ bmap)
 {
     const ItemBlock ib = item_block(bmap);
     const P2GArgs &a = tab[ib.item];
@@ -406,7 +428,7 @@ __global__ __launch_bounds__(64 * TZ * P2G_TPC, 4) void k_p2g_tiles(const P2GArg
     constexpr int lfield = nbox * lplane;         // words per field
     extern __shared__ unsigned long long acc[];   // [field][plane][y][x]
     __shared__ int s_err, s_far;
-    __shared__ unsigned short s_items[2 * TZ][64];   // per wave: the pass's items (source lane, first point)
+    __shared__ unsigned short s_items[16][64];   // per wave: the pass's items (source lane, first point)
 
     for (int u = tid; u < P2G_NF * lfield; u += blockDim.x) acc[u] = 0ull;
     if (tid == 0) s_err = s_far = 0;
@@ -719,6 +741,30 @@ __global__ __launch_bounds__(64 * TZ * P2G_TPC, 4) void k_p2g_tiles(const P2GArg
 // ---------------------------------------------------------------------------
 // 6. staging sum + folds + normalisation (one thread per (i, j) column)
 // ---------------------------------------------------------------------------
+// tile d = -1, 0, 1 beside the one of node i (of n, nt >= 3 tiles of 8, the
+// last one shorter when n is not a multiple of 8): its number t and the node's
+// place l in its box; false when the box does not hold the node
+__device__ inline bool box_place(int d, int i, int n, int nt, int &t, int &l)
+{
+    const int own = i >> 3, r = i & 7;
+    t = own + d;
+    l = r + 1;
+    if (d < 0) {
+        if (r > 1) return false;
+        l = r + 9;
+        if (own == 0) {
+            t = nt - 1;
+            l = i + n - 8 * t + 1;
+            return l < P2G_BOX;
+        }
+    } else if (d > 0) {
+        l = 0;
+        if (i == n - 1) t = 0;
+        else if (r != 7) return false;
+    }
+    return true;
+}
+
 // adds the staged sums of node (i, j, k) to out[], and its far-point sums
 // when there are any (far)
 __device__ inline void stage_add(const FinalizeArgs &a, int i, int j, int k, double out[P2G_NF], bool far)
@@ -732,6 +778,25 @@ __device__ inline void stage_add(const FinalizeArgs &a, int i, int j, int k, dou
     }
     const int nbox = a.tz + 3;
     const int cza = (k + 1) / a.tz;
+    if (a.ntx >= 3 && a.nty >= 3) {   // no box meets itself: each neighbour holds a node once or not
+        for (int dcz = -1; dcz <= 1; ++dcz) {
+            const int cz = cza + dcz, lp = k - (cz * a.tz - 2);
+            if (cz < 0 || cz >= a.nchz || lp < 0 || lp >= nbox) continue;
+            for (int dty = -1; dty <= 1; ++dty) {
+                int ty, ly;
+                if (!box_place(dty, j, g.ny, a.nty, ty, ly)) continue;
+                for (int dtx = -1; dtx <= 1; ++dtx) {
+                    int tx, lx;
+                    if (!box_place(dtx, i, g.nx, a.ntx, tx, lx)) continue;
+                    const int wg = (cz * a.nty + ty) * a.ntx + tx;
+                    const EPIC_GLOBAL double *s = gl(a.staging) + ((int64_t)wg * nbox + lp) * PLANE + (ly * P2G_BOX + lx) * P2G_NF;
+#pragma unroll
+                    for (int f = 0; f < P2G_NF; ++f) out[f] += s[f];
+                }
+            }
+        }
+        return;
+    }
     const int txa = i / P2G_TX, tya = j / P2G_TY;
     for (int dcz = -1; dcz <= 1; ++dcz) {
         const int cz = cza + dcz;
@@ -933,11 +998,11 @@ void launch_cell_order(int64_t nc, const int *cell_start, const int *perm_tmp, c
 P2GLayout p2g_layout(const Grid &g)
 {
     P2GLayout L;
-    L.tz = 2;
     // the last tile of a row or column is partial when nx or ny is not a
     // multiple of 8: its cells beyond the grid hold no parcels
     L.ntx = (g.nx + P2G_TX - 1) / P2G_TX;
     L.nty = (g.ny + P2G_TY - 1) / P2G_TY;
+    L.tz = p2g_default_tz(L.ntx, L.nty, g.nz);
     L.nchz = (g.nz + 2 + L.tz - 1) / L.tz;
     L.staging_elems = (int64_t)L.ntx * L.nty * L.nchz * (L.tz + 3) * P2G_BOX * P2G_BOX * P2G_NF;
     return L;
@@ -953,43 +1018,46 @@ __global__ __launch_bounds__(256) void k_far_clear(const FarClearArgs *__restric
 {
     const ItemBlock ib = item_block(bmap);
     const FarClearArgs &a = tab[ib.item];
-    if (*a.far_flag == 0) return;   // uniform over the launch
+    // the flag changes only once every block has counted itself below, so the
+    // blocks of an item agree on it
+    if (*a.far_flag == 0) return;
     for (int64_t q = (int64_t)ib.blk * 256 + threadIdx.x; q < a.n; q += (int64_t)FAR_CLEAR_BLOCKS * 256)
         gl(a.far_acc)[q] = 0ull;
-}
-
-__global__ __launch_bounds__(64) void k_far_reset(const FarClearArgs *__restrict__ tab, const int2 *__restrict__ bmap)
-{
-    const ItemBlock ib = item_block(bmap);
-    if (threadIdx.x == 0) gl(tab[ib.item].far_flag)[0] = 0;
+    __syncthreads();
+    if (threadIdx.x == 0 && atomicAdd(a.far_flag + 1, 1) == FAR_CLEAR_BLOCKS - 1) {
+        a.far_flag[1] = 0;
+        a.far_flag[0] = 0;
+    }
 }
 
 void add_p2g(Plan &P, int phase, const std::vector<P2GArgs> &tiles, const std::vector<FinalizeArgs> &fin,
              const std::vector<FarClearArgs> &far)
 {
-    // one grouped launch per z chunk (the work-group size is 64 tz P2G_TPC),
-    // the kernel specialised on it (epic_set_tiling and the autotuner admit
-    // 2, 4 and 8 only)
+    // one grouped launch per z chunk, the kernel specialised on it
+    // (epic_set_tiling and the autotuner admit 2, 4 and 8 only)
     std::vector<int> tzs;
     for (const P2GArgs &a : tiles)
         if (std::find(tzs.begin(), tzs.end(), a.tz) == tzs.end()) tzs.push_back(a.tz);
     for (int tz : tzs) {
         std::vector<P2GArgs> items;
         std::vector<int> nb;
+        int64_t total = 0;
         for (P2GArgs a : tiles) {
             if (a.tz != tz) continue;
             items.push_back(a);
             nb.push_back(a.ntx * a.nty * a.nchz);
+            total += nb.back();
         }
+        // 128 threads a layer keep four waves per SIMD within the box's LDS
+        const int nt = std::max(tile_threads(total), 128 * tz);
         const void *k = tz == 2 ? (const void *)k_p2g_tiles<2> : tz == 4 ? (const void *)k_p2g_tiles<4> : (const void *)k_p2g_tiles<8>;
-        P.add(k, 64 * tz * P2G_TPC, p2g_lds_bytes(tz), phase == PH_P2G ? (int)PH_P2G_TILES : phase, items, nb);
+        P.add(k, nt, p2g_lds_bytes(tz), phase == PH_P2G ? (int)PH_P2G_TILES : phase, items, nb);
     }
     std::vector<int> nf;
     for (const FinalizeArgs &f : fin) nf.push_back((int)(((int64_t)f.g.nx * f.g.ny * (f.g.nz + 3) + 255) / 256));
     P.add((const void *)k_p2g_finalize, 256, 0, phase, fin, nf);
-    std::vector<int> nc(far.size(), FAR_CLEAR_BLOCKS), nr(far.size(), 1);
+    std::vector<int> nc(far.size(), FAR_CLEAR_BLOCKS);
     P.add((const void *)k_far_clear, 256, 0, phase, far, nc);
-    P.add((const void *)k_far_reset, 64, 0, phase, far, nr);
 }
 
 }  // namespace epic
