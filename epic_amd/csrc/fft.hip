@@ -9,6 +9,10 @@
 //
 // The parcel correction's source volg / vcell - 1 is formed in the forward x
 // pass's loader.
+//
+// Lines lie one point apart from a multiple of 32 banks in LDS where they are
+// read or written across (16 z of one point): at power-of-two lengths those
+// accesses met one bank 16 ways.
 #include "common.h"
 #include "fft.h"
 #include "launch.h"
@@ -36,7 +40,7 @@ template <int KIND> __device__ inline float phys_value(const FftXArgs &a, int64_
 }
 
 // ZB rows of nx reals (planes zp0.., row j) packed as m = nx/2 complex
-// values per row into buf[r m + q]; planes above nz are zero
+// values per row into buf[r (m + 1) + q]; planes above nz are zero
 template <int KIND> __device__ inline void stage_rows(const FftXArgs &a, float2 *buf, int j, int zp0, int m)
 {
     const Grid &g = a.g;
@@ -54,15 +58,15 @@ template <int KIND> __device__ inline void stage_rows(const FftXArgs &a, float2 
         }
 #pragma unroll
         for (int u = 0; u < LOAD_BATCH; ++u) {
-            const int t = t0 + u * blockDim.x;
-            if (t < total) buf[t] = (zp0 + fdiv(t, a.plan.n1) <= nz) ? z[u] : float2{0, 0};
+            const int t = t0 + u * blockDim.x, r = fdiv(min(t, total - 1), a.plan.n1);
+            if (t < total) buf[t + r] = (zp0 + r <= nz) ? z[u] : float2{0, 0};
         }
     }
 }
 
-// ZB z-contiguous spectra columns: buf[r * len + c] = in[(c * stride + col) * nzp + zp0 + r]
+// ZB z-contiguous spectra columns: buf[r * ls + c] = in[(c * stride + col) * nzp + zp0 + r]
 // for c < len
-__device__ inline void stage_columns(const float2 *in, float2 *buf, int len, int64_t stride, int col, const Grid &g, int zp0)
+__device__ inline void stage_columns(const float2 *in, float2 *buf, int len, int ls, int64_t stride, int col, const Grid &g, int zp0)
 {
     const int total = ZB * len;
     for (int t0 = threadIdx.x; t0 < total; t0 += LOAD_BATCH * blockDim.x) {
@@ -76,7 +80,7 @@ __device__ inline void stage_columns(const float2 *in, float2 *buf, int len, int
 #pragma unroll
         for (int u = 0; u < LOAD_BATCH; ++u) {
             const int t = t0 + u * blockDim.x, c = t / ZB, r = t - c * ZB;
-            if (t < total) buf[r * len + c] = v[u];
+            if (t < total) buf[r * ls + c] = v[u];
         }
     }
 }
@@ -96,13 +100,13 @@ __global__ __launch_bounds__(256) void k_fft_xf(const FftXArgs *__restrict__ tab
     if (a.mode == 3) stage_rows<XF_PHI>(a, bufa, j, zp0, m);
     else stage_rows<XF_FIELD>(a, bufa, j, zp0, m);
     __syncthreads();
-    float2 *Z = lds_fft(bufa, bufb, ZB, a.plan, tw, 2, false, m);
+    float2 *Z = lds_fft(bufa, bufb, ZB, a.plan, tw, 2, false, m + 1);
     float2 *other = (Z == bufa) ? bufb : bufa;
     // untangle the packed real transform: X_k, k = 0..m
     for (int t = threadIdx.x; t < ZB * (m + 1); t += blockDim.x) {
         const int kx = t / ZB, r = t - kx * ZB;
-        const float2 zk = Z[r * m + (kx == m ? 0 : kx)];              // kx mod m, kx in [0, m]
-        const float2 zc = cconj(Z[r * m + (kx == 0 ? 0 : m - kx)]);   // (m - kx) mod m
+        const float2 zk = Z[r * (m + 1) + (kx == m ? 0 : kx)];              // kx mod m, kx in [0, m]
+        const float2 zc = cconj(Z[r * (m + 1) + (kx == 0 ? 0 : m - kx)]);   // (m - kx) mod m
         const float2 w = tw[kx];   // e^{-2 pi i kx / nx}
         const float2 s = cadd(zk, zc), d = csub(zk, zc);
         const float2 wd = cmul(w, d);
@@ -131,15 +135,15 @@ __global__ __launch_bounds__(256) void k_fft_y(const FftYArgs *__restrict__ tab,
     const int zp0 = (ib.blk / g.nxh) * ZB;
     const int ny = g.ny, nxh = g.nxh;
     extern __shared__ float2 lds[];
-    float2 *bufa = lds, *bufb = lds + ZB * ny;
-    float2 *tw = bufb + ZB * ny;   // twiddles staged in LDS
+    float2 *bufa = lds, *bufb = lds + ZB * (ny + 1);
+    float2 *tw = bufb + ZB * (ny + 1);   // twiddles staged in LDS
     for (int t = threadIdx.x; t < ny; t += blockDim.x) tw[t] = gl(a.tw)[t];
-    stage_columns(a.in, bufa, ny, nxh, kx, g, zp0);
+    stage_columns(a.in, bufa, ny, ny + 1, nxh, kx, g, zp0);
     __syncthreads();
-    float2 *Rb = lds_fft(bufa, bufb, ZB, a.plan, tw, 1, a.mode != 0, ny);
+    float2 *Rb = lds_fft(bufa, bufb, ZB, a.plan, tw, 1, a.mode != 0, ny + 1);
     for (int t = threadIdx.x; t < ZB * ny; t += blockDim.x) {
         const int jy = t / ZB, r = t - jy * ZB;
-        gl(a.out)[((int64_t)jy * nxh + kx) * g.nzp + zp0 + r] = Rb[r * ny + jy];
+        gl(a.out)[((int64_t)jy * nxh + kx) * g.nzp + zp0 + r] = Rb[r * (ny + 1) + jy];
     }
 }
 
@@ -158,7 +162,7 @@ __global__ __launch_bounds__(256) void k_fft_xi(const FftXArgs *__restrict__ tab
     float2 *bufa = lds, *bufb = lds + ZB * (m + 1);
     float2 *tw = bufb + ZB * (m + 1);   // twiddles staged in LDS
     for (int t = threadIdx.x; t < g.nx; t += blockDim.x) tw[t] = gl(a.tw)[t];
-    stage_columns(a.in, bufb, nxh, 1, j * nxh, g, zp0);
+    stage_columns(a.in, bufb, nxh, nxh, 1, j * nxh, g, zp0);
     __syncthreads();
     for (int t = threadIdx.x; t < ZB * m; t += blockDim.x) {
         const int r = fdiv(t, a.plan.n1), k = t - r * m;
@@ -185,11 +189,15 @@ __global__ __launch_bounds__(256) void k_fft_xi(const FftXArgs *__restrict__ tab
 // host side
 // ---------------------------------------------------------------------------
 static size_t x_lds(const Grid &g) { return (2 * ZB * (size_t)(g.nx / 2 + 1) + g.nx) * sizeof(float2); }
-static size_t y_lds(const Grid &g) { return (2 * ZB * (size_t)g.ny + g.ny) * sizeof(float2); }
+static size_t y_lds(const Grid &g) { return (2 * ZB * (size_t)(g.ny + 1) + g.ny) * sizeof(float2); }
 
-// The grids accepted are those whose ZB lines fit a work-group's LDS at FP64:
-// twice the FP32 passes here, and more than vorticity_tendency's FP64 lines
-size_t transform_lds_bytes(const Grid &g) { return std::max({2 * x_lds(g), 2 * y_lds(g), col_lds_bytes(g)}); }
+// The grids accepted are those whose ZB lines of nx/2 + 1 and of ny points fit
+// a work-group's LDS twice at FP64: more than any of the transforms takes
+size_t transform_lds_bytes(const Grid &g)
+{
+    const size_t x = 2 * ZB * (size_t)(g.nx / 2 + 1) + g.nx, y = 2 * ZB * (size_t)g.ny + g.ny;
+    return std::max(std::max(x, y) * sizeof(double2), col_lds_bytes(g));
+}
 
 void add_fft_xf(Plan &P, int phase, const std::vector<FftXArgs> &items)
 {

@@ -1,0 +1,65 @@
+"""The stage operators at the sizes where their kernels change form: column
+lengths around the register slots of the vertical solve, lines around the
+block sizes of the tendency's transforms, tiles and z chunks with remainders,
+and launches of each work-group size; against the FP64 oracle at the
+repository's bar (max-rel 1e-5; counts exact)."""
+import numpy as np
+import pytest
+
+from epic_amd import workloads as W
+from epic_amd.core import Member
+from tests._util import maxrel, oracle_state
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1.0e-5
+
+GRIDS = [
+    (8, 8, 4),        # one tile, two-point-wide blocks, shortest column
+    (10, 8, 60),      # 61 values of a column: one slot
+    (8, 10, 64),      # 65: two slots
+    (8, 8, 125),      # 126: two slots, radix 5 in z
+    (8, 8, 128),      # 129: three slots
+    (8, 8, 192),      # 193: the LDS form
+    (24, 30, 8),      # three and four tiles, the last one partial
+    (18, 24, 10),     # a two-cell last tile in x
+    (128, 8, 6),      # long rows beside short y lines
+    (8, 128, 6),
+    (64, 64, 16),     # 576 work-groups: 256 threads; 2^16 nodes
+    (64, 40, 15),     # 360 work-groups: 512 threads
+]
+
+
+@pytest.mark.parametrize("grid", GRIDS, ids=lambda g: "x".join(map(str, g)))
+def test_stage_operators(grid):
+    nx, ny, nz = grid
+    print(f"operator edges: {grid}", flush=True)
+    mem = W.rising_thermal(nx, seed=11 + nx + ny + nz, ny=ny, nz=nz)
+    mem.f_cor = (0.1, -0.2, 0.3)
+    mem.zeta_zero = (True, False)
+    st = oracle_state(mem)
+    gm = Member.from_workload(mem)
+    st.par2grid()
+    gm.par2grid()
+    sl = (Ellipsis, slice(1, nx + 1), slice(1, ny + 1), slice(None))
+    for f in ("volg", "vortg", "tbuoyg"):
+        assert maxrel(gm.get_field(f)[sl], getattr(st, f)[sl]) <= TOL, f
+    assert np.array_equal(gm.get_field("nparg")[sl], st.nparg[sl])
+    # the same input to the inversion on both sides
+    for f in ("vortg", "tbuoyg"):
+        gm.set_field(f, np.asarray(getattr(st, f)).astype(np.float32).astype(np.float64))
+        getattr(st, f)[...] = np.asarray(getattr(st, f)).astype(np.float32).astype(np.float64)
+    st.vor2vel()
+    gm.vor2vel()
+    st.vorticity_tendency()
+    gm.vorticity_tendency()
+    for f in ("vortg", "velog", "velgradg", "vtend"):
+        assert maxrel(gm.get_field(f)[sl], getattr(st, f)[sl]) <= TOL, f
+    # and one step, through the tile kernels
+    st, gm = oracle_state(mem), Member.from_workload(mem)
+    st.ls_rk_step(0.0, 0.005)
+    gm.ls_rk_step(0.0, 0.005)
+    p = gm.get_parcels()
+    assert np.abs(p["position"] - st.position).max() <= TOL * max(mem.dx)
+    for k in ("vorticity", "B"):
+        assert maxrel(p[k], getattr(st, k)) <= TOL, k
