@@ -109,7 +109,7 @@ struct epic_member {
     bool tend_displaced = false;
     int *tend_src = nullptr;
     Plan pl_settle;
-    // p2g's fixed-point maxima (P2G_NF + 1)
+    // p2g's fixed-point maxima (P2G_MAXIMA)
     float *pmax_out = nullptr;
     Plan pl_resort;
     // the parcel count in device memory (and its pinned host staging word)
@@ -445,7 +445,8 @@ struct P2GSel {
     const int *use_alt;
     int rd;
     int clr;                  // -1: none
-    bool max_from_push = false;   // the previous push stored the fixed-point maxima: no k_p2g_max
+    bool max_from_push = false;   // the previous push and stages left the fixed-point maxima: no k_p2g_max
+    bool push_next = false;       // a push that fills the vorticity's maxima follows: the others stay
 };
 
 void build_p2g(Plan &P, const Members &ms, const std::vector<P2GSel> &sel)
@@ -475,6 +476,7 @@ void build_p2g(Plan &P, const Members &ms, const std::vector<P2GSel> &sel)
         a.staging = m->staging;
         a.err = m->err_d;
         a.tmax = m->pmax_out;
+        a.bounds = q.max_from_push ? 1 : 0;
         a.far_acc = m->far_acc;
         a.far_flag = m->far_flag;
         a.far_scale = m->far_scale;
@@ -494,6 +496,7 @@ void build_p2g(Plan &P, const Members &ms, const std::vector<P2GSel> &sel)
         f.clear_count = q.clr >= 0 ? m->cnt[q.clr] : nullptr;
         f.clear_scount = q.clr >= 0 ? m->scnt[q.clr] : nullptr;
         f.clear_tmax = m->pmax_out;
+        f.clear_all = q.push_next ? 0 : 1;
         f.far_acc = m->far_acc;
         f.far_flag = m->far_flag;
         f.far_scale = m->far_scale;
@@ -640,7 +643,7 @@ void build_step(Plan &P, const std::vector<StepItem> &items)
             float *const *a = last ? m->ax_stale : m->ax_cur;
             ax.push_back(a);
             const int rd = (s - 1) % 3, wr = last ? 0 : (s % 3);
-            sel.push_back(P2GSel{a, m->ax_stale, s == 1 ? it->reuse : nullptr, rd, wr, s > 1});
+            sel.push_back(P2GSel{a, m->ax_stale, s == 1 ? it->reuse : nullptr, rd, wr, s > 1, !last});
         }
         if (s == 1) build_axes(P, ms, ax);   // later stages: stored by the previous push
         build_p2g(P, ms, sel);
@@ -667,7 +670,7 @@ void build_step(Plan &P, const std::vector<StepItem> &items)
             for (int c = 0; c < 6; ++c) a.axes[c] = ax[i][c];
             if (!last) {
                 for (int c = 0; c < 6; ++c) a.axes_next[c] = (s + 1 == ns) ? m->ax_stale[c] : m->ax_cur[c];
-                a.tmax_next = m->pmax_out;   // cleared by this stage's finalize
+                a.tmax_next = m->pmax_out;   // its vorticity entries cleared by this stage's finalize
             }
             a.perm = m->perm;
             a.cell_start = m->cell_start;
@@ -915,7 +918,7 @@ int epic_create(const epic_grid_t *grid, const epic_phys_t *phys, const epic_fla
     if (bad(dalloc(&m->spec[0], NSPEC * spec_size(g), m->s))) return EPIC_E_NOMEM;
     for (int i = 1; i < NSPEC; ++i) m->spec[i] = m->spec[0] + i * spec_size(g);
     if (bad(dalloc(&m->err_d, 4, m->s)) || bad(dalloc(&m->flags_d, 4, m->s)) || bad(dalloc(&m->tm_d, 1, m->s))) return EPIC_E_NOMEM;
-    if (bad(dalloc(&m->pmax_out, P2G_NF + 1, m->s))) return EPIC_E_NOMEM;
+    if (bad(dalloc(&m->pmax_out, P2G_MAXIMA, m->s))) return EPIC_E_NOMEM;
     if (bad(hipHostMalloc((void **)&m->err_h, sizeof(int) * 4, hipHostMallocDefault)) ||
         bad(hipHostMalloc((void **)&m->tm_h, sizeof(StepTime), hipHostMallocDefault)))
         return EPIC_E_NOMEM;

@@ -167,6 +167,18 @@ template <class T> __device__ inline const EPIC_GLOBAL T &at(const T *p, unsigne
     return *(const EPIC_GLOBAL T *)((const EPIC_GLOBAL char *)p + off);
 }
 
+// The same offset as a new value of the current basic block.  Instruction
+// selection folds the 32-bit offset into an access only where it sees the
+// offset's extension in the same block; an offset formed in an earlier block
+// arrives as a 64-bit register pair, and every access adds its base to it.
+__device__ inline unsigned block_offset(unsigned off)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    asm volatile("" : "+v"(off));
+#endif
+    return off;
+}
+
 __host__ __device__ inline int64_t field_stride(const Grid &g) { return (int64_t)(g.nz + 3) * g.ny * g.nx; }
 __host__ __device__ inline int64_t plane_stride(const Grid &g) { return (int64_t)g.ny * g.nx; }
 __host__ __device__ inline int64_t spec_size(const Grid &g) { return (int64_t)g.ny * g.nxh * g.nzp; }

@@ -244,20 +244,6 @@ __device__ inline bool support_axes(const double B[5], double vol, double veta[3
     return true;
 }
 
-// The four support points in cell units: with x the centre's grid coordinate
-// along one axis, u = rt2i dxi (Veta + Vtau) and w = rt2i dxi (Veta - Vtau),
-// point j is at x + u, x - w, x - u, x + w (j = 0..3): eight FP64 operations
-// an axis, where scaling each point's position took sixteen.
-__device__ inline void support_offsets(double veta, double vtau, double rt2i_dxi, double &u, double &w)
-{
-    u = (veta + vtau) * rt2i_dxi;
-    w = (veta - vtau) * rt2i_dxi;
-}
-__device__ inline double support_coord(int j, double x, double u, double w)
-{
-    return j == 0 ? x + u : j == 1 ? x - w : j == 2 ? x - u : x + w;
-}
-
 // cos and sin of (2j+1) pi/4 for j = 0..3
 __device__ inline double support_cos(int j) { return (j == 0 || j == 3) ? EPIC_RT2I : -EPIC_RT2I; }
 __device__ inline double support_sin(int j) { return (j < 2) ? EPIC_RT2I : -EPIC_RT2I; }

@@ -134,16 +134,23 @@ __global__ __launch_bounds__(256) void k_grid2par(const G2PArgs *__restrict__ ta
 // half axes cached for this stage.  The permutation entry of a thread's next
 // parcel is loaded one round ahead, and parcel arrays are addressed as a
 // table pointer plus a 32-bit byte offset.
+//
+// What bounds it: HBM traffic (about 380 B a parcel at 4.8 TB/s, a large
+// copy's rate here) together with VALU issue; both only overlap as far as no
+// round waits for memory before its gather.  With the deltas taken into the
+// sums after the gather, constant LDS strides, offsets folded into the
+// accesses and the fields that a step does not change out of the maxima, no
+// register spills and a launch takes 1.20 ms at 128^3 (1.46 before).
 // ---------------------------------------------------------------------------
 size_t g2p_lds_bytes(int tz) { return (3 * sizeof(float4) + sizeof(float2)) * (tz + 3) * P2G_BOX * P2G_BOX; }
 
-template <int NT>
+template <int NT, int TZ>
 __global__ __launch_bounds__(NT, 4) void k_g2p_tiles(const G2PTileArgs *__restrict__ tab, const int2 *__restrict__ bmap)
 {
     const ItemBlock ib = item_block(bmap);
     const G2PTileArgs &a = tab[ib.item];
     const Grid &g = a.g;
-    const int tz = a.tz;
+    constexpr int tz = TZ;   // = a.tz
     const int tx = ib.blk % a.ntx;
     const int ty = (ib.blk / a.ntx) % a.nty;
     const int cz = ib.blk / (a.ntx * a.nty);
@@ -153,14 +160,14 @@ __global__ __launch_bounds__(NT, 4) void k_g2p_tiles(const G2PTileArgs *__restri
     const int tid = threadIdx.x;
     const int64_t PS = plane_stride(g), FS = field_stride(g);
     constexpr int NN = P2G_BOX * P2G_BOX;
-    const int nbox = tz + 3;
+    constexpr int nbox = tz + 3;
 
     extern __shared__ float4 box[];                 // [group][plane][y][x]: 3 float4 groups, then a float2 group
-    const int NB = nbox * NN;                       // nodes in the box
+    constexpr int NB = nbox * NN;                   // nodes in the box
     float2 *box2 = (float2 *)(box + 3 * NB);
-    __shared__ unsigned int s_pmax[P2G_NF + 1];     // the next par2grid's maxima (float bits)
+    __shared__ unsigned int s_pmax[3];              // the next par2grid's vorticity maxima (float bits)
     int e = 0;
-    if (tid <= P2G_NF) s_pmax[tid] = 0u;   // ordered by the barrier after the box is staged
+    if (tid < 3) s_pmax[tid] = 0u;   // ordered by the barrier after the box is staged
 
     // ---- stage the node box (plane P = k0 - 1 + lp) ----
     // thread = (node of the 11 x 11 box column, half of the 14 fields, every
@@ -204,8 +211,9 @@ __global__ __launch_bounds__(NT, 4) void k_g2p_tiles(const G2PTileArgs *__restri
     int pi_nx = 0;
     double pn[3] = {0.0, 0.0, 0.0};
     float an[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    const bool acc_prev = a.stage > 1;
     auto prefetch = [&](int pj) {
-        const unsigned oj = (unsigned)pj * 4u;
+        const unsigned oj = block_offset((unsigned)pj * 4u);
         pn[0] = gl(a.p.x)[pj];
         pn[1] = gl(a.p.y)[pj];
         pn[2] = gl(a.p.z)[pj];
@@ -223,16 +231,24 @@ __global__ __launch_bounds__(NT, 4) void k_g2p_tiles(const G2PTileArgs *__restri
         const bool more = q + NT < total;
         if (more) pi_nx = gl(a.perm)[first + q + NT];
         double pos[3] = {pn[0], pn[1], pn[2]};
-        const double ve[3] = {an[0], an[1], an[2]};
-        const double vt[3] = {an[3], an[4], an[5]};
         int key = -1;
         bool small = false;
         auto process = [&]() {
             if (q >= total) return;
-            double B[5];
+            // requested here and used after the gather
+            float Bf[5];
 #pragma unroll
-            for (int c = 0; c < 5; ++c) B[c] = (double)at(a.p.B[c], o4);
-            const double vol = (double)at(a.p.vol, o4);
+            for (int c = 0; c < 5; ++c) Bf[c] = at(a.p.B[c], o4);
+            const float volf = at(a.p.vol, o4);
+            float dp[3] = {}, dv[3] = {};
+            if (acc_prev) {
+                const unsigned o = block_offset(o4);
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    dp[c] = at(a.p.dpos[c], o);
+                    dv[c] = at(a.p.dvor[c], o);
+                }
+            }
             int cc[3];
 #pragma unroll
             for (int d = 0; d < 3; ++d) cc[d] = (int)floor((pos[d] - g.lower[d]) * g.dxi[d]);
@@ -243,38 +259,38 @@ __global__ __launch_bounds__(NT, 4) void k_g2p_tiles(const G2PTileArgs *__restri
                 if (more) prefetch(pi_nx);
                 return;
             }
-            const bool acc_prev = a.stage > 1;
-            float dp[3], dv[3], st[8];
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                dp[c] = acc_prev ? at(a.p.dpos[c], o4) : 0.0f;
-                dv[c] = acc_prev ? at(a.p.dvor[c], o4) : 0.0f;
-            }
+            const int own = __mul24(k - k0 + 1, NN) + __mul24(cy + 1, P2G_BOX) + cx + 1;   // own cell's lower corner in the box
+            // coordinate of support point jp along axis d, in cells
+            auto coord = [&](int jp, int d) {
+                const double pt = pos[d] + (double)an[d] * support_cos(jp) + (double)an[3 + d] * support_sin(jp);
+                return (pt - g.lower[d]) * g.dxi[d];
+            };
+            // A point's gathered velocity and tendency wait in sd until the
+            // deltas that they are added to have arrived.
+            float st[8], sd[4][6];
 #pragma unroll
             for (int c = 0; c < 8; ++c) st[c] = 0.0f;
 #pragma unroll
             for (int jp = 0; jp < 4; ++jp) {
-                const double cs = support_cos(jp), sn = support_sin(jp);
                 int off[3];
                 float w[3];
 #pragma unroll
                 for (int d = 0; d < 3; ++d) {
-                    const double pt = pos[d] + ve[d] * cs + vt[d] * sn;
-                    const double xyz = (pt - g.lower[d]) * g.dxi[d];
-                    const double fl = floor(xyz);
+                    const double xyz = coord(jp, d), fl = floor(xyz);
                     off[d] = (int)fl - cc[d];
                     w[d] = (float)(xyz - fl);
                 }
-                if (k + off[2] < -1 || k + off[2] > g.nz) {   // beyond the halo layers (the reference fails too)
+                // box corner; -2: beyond the neighbour cells; -1: beyond the
+                // halo layers (the reference fails too)
+                int n0 = own + __mul24(off[2], NN) + __mul24(off[1], P2G_BOX) + off[0];
+                if ((unsigned)(off[0] + 1) > 2u || (unsigned)(off[1] + 1) > 2u || (unsigned)(off[2] + 1) > 2u) n0 = -2;
+                if (k + off[2] < -1 || k + off[2] > g.nz) {
                     e |= ERR_OUT_OF_GRID;
-                    continue;
+                    n0 = -1;
                 }
-                // a point beyond the neighbour cells (strongly stretched
-                // parcels, rare) gathers its corners from the global fields,
-                // in the same order, so the sums are the same bits
-                const bool far = off[0] < -1 || off[0] > 1 || off[1] < -1 || off[1] > 1 || off[2] < -1 || off[2] > 1;
-                // box coordinates of the point's lower corner
-                const int lx = cx + off[0] + 1, ly = cy + off[1] + 1, lp = k + off[2] - (k0 - 1);
+#pragma unroll
+                for (int c = 0; c < 6; ++c) sd[jp][c] = 0.0f;
+                if (n0 == -1) continue;
                 const float pxc = 1.0f - w[0], pyc = 1.0f - w[1], pzc = 1.0f - w[2];
                 const float w00 = pyc * pxc, w10 = pyc * w[0], w01 = w[1] * pxc, w11 = w[1] * w[0];
                 // corners in Fortran element order of ww(0:1,0:1,0:1): k fastest
@@ -283,11 +299,11 @@ __global__ __launch_bounds__(NT, 4) void k_g2p_tiles(const G2PTileArgs *__restri
                 float s[14];
 #pragma unroll
                 for (int f = 0; f < 14; ++f) s[f] = 0.0f;
-                if (!far) {
+                if (n0 >= 0) {
 #pragma unroll
                     for (int m = 0; m < 8; ++m) {
                         const int dz = m & 1, dy = (m >> 1) & 1, dx = (m >> 2) & 1;
-                        const int nd = (lp + dz) * NN + (ly + dy) * P2G_BOX + (lx + dx);
+                        const int nd = n0 + dz * NN + dy * P2G_BOX + dx;
                         const float4 q0 = box[nd], q1 = box[NB + nd], q2 = box[2 * NB + nd];
                         const float2 q3 = box2[nd];
                         const float vv[14] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w,
@@ -296,26 +312,53 @@ __global__ __launch_bounds__(NT, 4) void k_g2p_tiles(const G2PTileArgs *__restri
                         for (int f = 0; f < 14; ++f) s[f] += wt[m] * vv[f];
                     }
                 } else {
+                    // strongly stretched parcels, rare: the corners from the
+                    // global fields, in the same order, so the sums are the
+                    // same bits (the cell again from its coordinates: offsets
+                    // kept to here would spill registers of the gather)
+                    const int ci = (int)floor(coord(jp, 0)), cj = (int)floor(coord(jp, 1)), ck = (int)floor(coord(jp, 2));
 #pragma unroll 1
                     for (int m = 0; m < 8; ++m) {
                         const int dz = m & 1, dy = (m >> 1) & 1, dx = (m >> 2) & 1;
-                        const int ii = wrap(cc[0] + off[0] + dx, g.nx), jj = wrap(cc[1] + off[1] + dy, g.ny);
-                        const int64_t o = (int64_t)(k + off[2] + dz + 1) * PS + (int64_t)jj * g.nx + ii;
+                        const int ii = wrap(ci + dx, g.nx), jj = wrap(cj + dy, g.ny);
+                        const int64_t o = (int64_t)(ck + dz + 1) * PS + (int64_t)jj * g.nx + ii;
                         const EPIC_GLOBAL float *f0 = gl(a.fld) + (int64_t)F_VELOG * FS + o;
 #pragma unroll
                         for (int f = 0; f < 14; ++f) s[f] += wt[m] * f0[(int64_t)f * FS];
                     }
                 }
 #pragma unroll
-                for (int c = 0; c < 3; ++c) dp[c] += 0.25f * s[c];
-#pragma unroll
                 for (int c = 0; c < 8; ++c) st[c] += 0.25f * s[3 + c];
 #pragma unroll
-                for (int c = 0; c < 3; ++c) dv[c] += 0.25f * s[11 + c];
+                for (int c = 0; c < 3; ++c) {
+                    sd[jp][c] = s[c];
+                    sd[jp][3 + c] = s[11 + c];
+                }
             }
+#pragma unroll
+            for (int jp = 0; jp < 4; ++jp)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    dp[c] += 0.25f * sd[jp][c];
+                    dv[c] += 0.25f * sd[jp][3 + c];
+                }
             if (more) prefetch(pi_nx);   // the next round's position and axes, in flight during the rest
+            float vor[3], dBo[5] = {};
+            {
+                const unsigned o = block_offset(o4);
+#pragma unroll
+                for (int c = 0; c < 3; ++c) vor[c] = at(a.p.vor[c], o);
+            }
+            if (acc_prev) {
+                const unsigned o = block_offset(o4);
+#pragma unroll
+                for (int c = 0; c < 5; ++c) dBo[c] = at(a.p.dB[c], o);
+            }
             // dB/dt (FP64, B33 from the volume constraint)
-            double S[8], dB[5];
+            const double vol = (double)volf;
+            double B[5], S[8], dB[5];
+#pragma unroll
+            for (int c = 0; c < 5; ++c) B[c] = (double)Bf[c];
 #pragma unroll
             for (int c = 0; c < 8; ++c) S[c] = (double)st[c];
             if (!dBdt(B, S, vol, dB)) {
@@ -324,13 +367,13 @@ __global__ __launch_bounds__(NT, 4) void k_g2p_tiles(const G2PTileArgs *__restri
             }
             float db[5];
 #pragma unroll
-            for (int c = 0; c < 5; ++c) db[c] = acc_prev ? at(a.p.dB[c], o4) + (float)dB[c] : (float)dB[c];
+            for (int c = 0; c < 5; ++c) db[c] = dBo[c] + (float)dB[c];
             // push (ls_rk.f90:183-191), periodic wrap (parcel_bc.f90:17-21)
             const double cbdt = a.cb * (*a.dt);
 #pragma unroll
             for (int c = 0; c < 3; ++c) pos[c] = pos[c] + cbdt * (double)dp[c];
 #pragma unroll
-            for (int c = 0; c < 3; ++c) at(a.p.vor[c], o4) = (float)((double)at(a.p.vor[c], o4) + cbdt * (double)dv[c]);
+            for (int c = 0; c < 3; ++c) vor[c] = (float)((double)vor[c] + cbdt * (double)dv[c]);
 #pragma unroll
             for (int c = 0; c < 5; ++c) B[c] = B[c] + cbdt * (double)db[c];
             pos[0] = pos[0] - g.extent[0] * trunc((pos[0] - g.center[0]) * g.hli[0]);
@@ -349,17 +392,23 @@ __global__ __launch_bounds__(NT, 4) void k_g2p_tiles(const G2PTileArgs *__restri
             gl(a.p.x)[pi] = pos[0];
             gl(a.p.y)[pi] = pos[1];
             gl(a.p.z)[pi] = pos[2];
+            {
+                const unsigned o = block_offset(o4);
 #pragma unroll
-            for (int c = 0; c < 5; ++c) at(a.p.B[c], o4) = (float)B[c];
+                for (int c = 0; c < 3; ++c) at(a.p.vor[c], o) = vor[c];
+#pragma unroll
+                for (int c = 0; c < 5; ++c) at(a.p.B[c], o) = (float)B[c];
+            }
             if (a.stage < a.nstages) {
                 const float ca = (float)a.ca;
+                const unsigned o = block_offset(o4);
 #pragma unroll
                 for (int c = 0; c < 3; ++c) {
-                    at(a.p.dpos[c], o4) = ca * dp[c];
-                    at(a.p.dvor[c], o4) = ca * dv[c];
+                    at(a.p.dpos[c], o) = ca * dp[c];
+                    at(a.p.dvor[c], o) = ca * dv[c];
                 }
 #pragma unroll
-                for (int c = 0; c < 5; ++c) at(a.p.dB[c], o4) = ca * db[c];
+                for (int c = 0; c < 5; ++c) at(a.p.dB[c], o) = ca * db[c];
             }
             // cell of the new position for the next stage's sort
             const int ni = (int)floor((pos[0] - g.lower[0]) * g.dxi[0]);
@@ -367,7 +416,7 @@ __global__ __launch_bounds__(NT, 4) void k_g2p_tiles(const G2PTileArgs *__restri
             const int nk = (int)floor((pos[2] - g.lower[2]) * g.dxi[2]);
             if (nk < -1 || nk > g.nz) e |= ERR_PARCEL_COUNT;
             else key = cell_index(g, wrap(ni, g.nx), wrap(nj, g.ny), nk);
-            at(a.keys, o4) = key;
+            at(a.keys, block_offset(o4)) = key;
             small = (vol <= g.vmin);
             if (a.axes_next[0]) {   // the next stage's support axes, from B as stored
                 double Bs[5], ve2[3], vt2[3];
@@ -377,56 +426,59 @@ __global__ __launch_bounds__(NT, 4) void k_g2p_tiles(const G2PTileArgs *__restri
                     e |= ERR_B33;
                     ve2[0] = ve2[1] = ve2[2] = vt2[0] = vt2[1] = vt2[2] = 0.0;
                 }
+                const unsigned o = block_offset(o4);
 #pragma unroll
                 for (int d = 0; d < 3; ++d) {
-                    at(a.axes_next[d], o4) = (float)ve2[d];
-                    at(a.axes_next[3 + d], o4) = (float)vt2[d];
+                    at(a.axes_next[d], o) = (float)ve2[d];
+                    at(a.axes_next[3 + d], o) = (float)vt2[d];
                 }
             }
             if (a.tmax_next) {
-                // bounds of the next par2grid's |contributions| of this
-                // parcel, from what it stored: the condensate is at most the
-                // humidity, so |tbuoy| <= |buoy| + glat hum and |tbuoy - buoy|
-                // <= glat hum (exact when there is no humidity); a scale from
-                // a bound is at most one power of two coarser, and the
-                // fixed-point sums keep a factor 2 of headroom for rounding
-                const float v0 = (float)(0.25 * vol), h = at(a.p.hum, o4);
-                const float hb = fabsf(v0 * (float)g.glat * h);
-                const float b5 = fabsf(v0 * at(a.p.buoy, o4));
-                const float m[P2G_NF + 1] = {fabsf(v0), fabsf(v0 * at(a.p.vor[0], o4)), fabsf(v0 * at(a.p.vor[1], o4)),
-                                             fabsf(v0 * at(a.p.vor[2], o4)), b5 + hb, b5, fabsf(v0 * h), hb};
-                // into the work-group's maxima (bits of non-negative floats);
-                // a lane below the running maximum skips the atomic
+                // the next par2grid's largest vorticity contributions, from
+                // what was stored (the other fields' values do not change in a
+                // step), into the work-group's maxima (bits of non-negative
+                // floats); a lane below the running maximum skips the atomic
+                const float v0 = (float)(0.25 * vol);
 #pragma unroll
-                for (int f = 0; f <= P2G_NF; ++f)
-                    if (m[f] > __uint_as_float(s_pmax[f])) atomicMax(&s_pmax[f], __float_as_uint(m[f]));
+                for (int c = 0; c < 3; ++c) {
+                    const float m = fabsf(v0 * vor[c]);
+                    if (m > __uint_as_float(s_pmax[c])) atomicMax(&s_pmax[c], __float_as_uint(m));
+                }
             }
         };
         process();
         // next stage's cell histogram, one atomic per run of equal keys
         wave_run_add(key, gl(a.count));
-        wave_run_add(small ? key : -1, gl(a.scount));
+        if (__any(small)) wave_run_add(small ? key : -1, gl(a.scount));
     }
     if (a.tmax_next) {
         __syncthreads();
-        if (tid <= P2G_NF && s_pmax[tid]) atomicMax((unsigned int *)a.tmax_next + tid, s_pmax[tid]);
+        if (tid < 3 && s_pmax[tid]) atomicMax((unsigned int *)a.tmax_next + 1 + tid, s_pmax[tid]);
     }
     if (e) atomicOr(a.err, e);
 }
 
-void add_rk_stage_tiles(Plan &P, int phase, const std::vector<G2PTileArgs> &items)
+template <int TZ> static const void *tiles_kernel(int nt)
 {
-    std::vector<int> nb;
-    size_t lds = 0;
-    int64_t total = 0;
-    for (const G2PTileArgs &a : items) {
-        nb.push_back(a.ntx * a.nty * a.nchz);
-        total += nb.back();
-        lds = std::max(lds, g2p_lds_bytes(a.tz));
+    return nt == 1024 ? (const void *)k_g2p_tiles<1024, TZ> : nt == 512 ? (const void *)k_g2p_tiles<512, TZ> : (const void *)k_g2p_tiles<256, TZ>;
+}
+
+void add_rk_stage_tiles(Plan &P, int phase, const std::vector<G2PTileArgs> &all)
+{
+    for (int tz : {2, 4, 8}) {   // one grouped launch per z chunk, the kernel specialised on it
+        std::vector<G2PTileArgs> items;
+        std::vector<int> nb;
+        int64_t total = 0;
+        for (const G2PTileArgs &a : all) {
+            if (a.tz != tz) continue;
+            items.push_back(a);
+            nb.push_back(a.ntx * a.nty * a.nchz);
+            total += nb.back();
+        }
+        if (items.empty()) continue;
+        const int nt = tile_threads(total);
+        P.add(tz == 2 ? tiles_kernel<2>(nt) : tz == 4 ? tiles_kernel<4>(nt) : tiles_kernel<8>(nt), nt, g2p_lds_bytes(tz), phase, items, nb);
     }
-    const int nt = tile_threads(total);
-    const void *k = nt == 1024 ? (const void *)k_g2p_tiles<1024> : nt == 512 ? (const void *)k_g2p_tiles<512> : (const void *)k_g2p_tiles<256>;
-    P.add(k, nt, lds, phase, items, nb);
 }
 
 void add_grid2par(Plan &P, int phase, const std::vector<G2PArgs> &items)

@@ -76,7 +76,8 @@ struct P2GArgs {
     const int *cell_start;
     double *staging;            // exact partial node sums (scaled integers)
     int *err;
-    const float *tmax;          // P2G_NF + 1 maxima from k_p2g_max (fixed-point scales)
+    const float *tmax;          // P2G_MAXIMA maxima (fixed-point scales)
+    int bounds;                 // take the moist fields' bounds: their maxima are an earlier stage's
     // support points beyond the neighbour cells of their parcel's cell: their
     // fixed-point terms go to far_acc ([field][plane k+1][j][i], 64-bit) by
     // global atomics; far_flag is set when there are any, far_scale receives
@@ -86,13 +87,15 @@ struct P2GArgs {
     double *far_scale;
     int tz, ntx, nty, nchz;
 };
-// largest |contribution| per field (and |tbuoy - buoy|) over a member's parcels
+// largest |contribution| per field, |tbuoy - buoy|, and the bounds of the total
+// buoyancy's and of that difference over a member's parcels
+constexpr int P2G_MAX_BOUND = P2G_NF + 1, P2G_MAXIMA = P2G_NF + 3;
 constexpr int P2G_MAX_BLOCKS = 4096;
 struct P2GMaxArgs {
     Grid g;
     ParcelsDev p;
     int nblk;                   // p2g_max_blocks(p.n)
-    float *out;                 // P2G_NF + 1, zero on entry; cleared again by the finalize kernel
+    float *out;                 // P2G_MAXIMA, zero on entry; cleared again by the finalize kernel
 };
 int p2g_max_blocks(int64_t n);
 void add_p2g_max(Plan &P, int phase, const std::vector<P2GMaxArgs> &items);
@@ -103,7 +106,8 @@ struct FinalizeArgs {
     float *fld;     // F_VOLG .. F_HUMG
     int *nparg, *nsparg;
     int *clear_count, *clear_scount;   // histograms cleared for the next push (may be null)
-    float *clear_tmax;                 // the tile kernel's maxima, zeroed for the next k_p2g_max (may be null)
+    float *clear_tmax;                 // the tile kernel's maxima, zeroed for the next k_p2g_max
+    int clear_all;                     // 0: only the vorticity's, which the stage's push fills
     const unsigned long long *far_acc; // the tile kernel's far-point sums (read when *far_flag)
     const int *far_flag;
     const double *far_scale;
@@ -132,7 +136,7 @@ struct G2PTileArgs {
     ParcelsDev p;
     const float *axes[6];
     float *axes_next[6];         // null, or where the half axes of the pushed B go (the next stage's)
-    float *tmax_next;            // null, or the next par2grid's maxima (atomicMax; zero on entry)
+    float *tmax_next;            // null, or the maxima whose vorticity entries the push fills (atomicMax; zero on entry)
     const int *perm;
     const int *cell_start;
     const float *fld;

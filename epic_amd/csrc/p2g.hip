@@ -368,16 +368,21 @@ __device__ inline void p2g_values(const Grid &g, const ParcelsDev &p, unsigned o
 // of the same par2grid clears it once the tile kernel has taken its scales
 // from it (a value left by an interrupted sequence would only be larger, a
 // coarser but still valid scale).  Inside an RK step only the first stage
-// runs this pass: each later stage's maxima come from the previous push,
-// which has the parcels' new values at hand and bounds the moist
-// contributions by the humidity (exact without humidity).
+// runs this pass: volume, buoyancy and humidity do not change in a step, so
+// their maxima stay for the later stages, the vorticity maxima come from the
+// previous push, and the moist contributions, which follow the height, are
+// bounded by the humidity: the condensate is at most the humidity, so |tbuoy|
+// <= |buoy| + glat hum and |tbuoy - buoy| <= glat hum (exact when there is no
+// humidity; P2G_MAX_BOUND onwards).  A scale from a bound is at most one power
+// of two coarser, and the fixed-point sums keep a factor 2 of headroom for
+// rounding.
 __global__ __launch_bounds__(256) void k_p2g_max(const P2GMaxArgs *__restrict__ tab, const int2 *__restrict__ bmap)
 {
     const ItemBlock ib = item_block(bmap);
     const P2GMaxArgs &a = tab[ib.item];
-    float mx[P2G_NF + 1];
+    float mx[P2G_MAXIMA];
 #pragma unroll
-    for (int f = 0; f <= P2G_NF; ++f) mx[f] = 0.0f;
+    for (int f = 0; f < P2G_MAXIMA; ++f) mx[f] = 0.0f;
     const int64_t n = parcel_count(a.p);
     for (int64_t q = (int64_t)ib.blk * 256 + threadIdx.x; q < n; q += (int64_t)a.nblk * 256) {
         float v[P2G_NF];
@@ -385,15 +390,18 @@ __global__ __launch_bounds__(256) void k_p2g_max(const P2GMaxArgs *__restrict__ 
 #pragma unroll
         for (int f = 0; f < P2G_NF; ++f) mx[f] = fmaxf(mx[f], fabsf(v[f]));
         mx[P2G_NF] = fmaxf(mx[P2G_NF], fabsf(v[4] - v[5]));
+        const float hb = fabsf(v[0] * (float)a.g.glat * at(a.p.hum, (unsigned)q * 4u));
+        mx[P2G_MAX_BOUND] = fmaxf(mx[P2G_MAX_BOUND], fabsf(v[5]) + hb);
+        mx[P2G_MAX_BOUND + 1] = fmaxf(mx[P2G_MAX_BOUND + 1], hb);
     }
-    __shared__ float wm[4][P2G_NF + 1];
+    __shared__ float wm[4][P2G_MAXIMA];
 #pragma unroll
-    for (int f = 0; f <= P2G_NF; ++f) {
+    for (int f = 0; f < P2G_MAXIMA; ++f) {
         for (int o = 32; o > 0; o >>= 1) mx[f] = fmaxf(mx[f], __shfl_xor(mx[f], o, 64));
         if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6][f] = mx[f];
     }
     __syncthreads();
-    if (threadIdx.x <= P2G_NF) {
+    if (threadIdx.x < P2G_MAXIMA) {
         const int f = threadIdx.x;
         const float m = fmaxf(fmaxf(wm[0][f], wm[1][f]), fmaxf(wm[2][f], wm[3][f]));
         if (m > 0.0f) atomicMax((unsigned int *)a.out + f, __float_as_uint(m));
@@ -444,6 +452,10 @@ __global__ __launch_bounds__(1024, 4) void k_p2g_tiles(const P2GArgs *__restrict
     float mx[P2G_NF + 1];
 #pragma unroll
     for (int f = 0; f <= P2G_NF; ++f) mx[f] = gl(a.tmax)[f];
+    if (a.bounds) {   // the later stages of a step
+        mx[4] = gl(a.tmax)[P2G_MAX_BOUND];
+        mx[P2G_NF] = gl(a.tmax)[P2G_MAX_BOUND + 1];
+    }
     float sc[P2G_NF];
 #pragma unroll
     for (int f = 0; f < P2G_NF; ++f) {
@@ -489,14 +501,8 @@ __global__ __launch_bounds__(1024, 4) void k_p2g_tiles(const P2GArgs *__restrict
                 v[6] = 0.0f;
             }
             int cc[3];
-            double xr[3], su[3], sw[3];   // position in the cell and point offsets, in cells
 #pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                const double x = (pos[d] - g.lower[d]) * g.dxi[d], fl = floor(x);
-                cc[d] = (int)fl;
-                xr[d] = x - fl;
-                support_offsets(ve[d], vt[d], EPIC_RT2I * g.dxi[d], su[d], sw[d]);
-            }
+            for (int d = 0; d < 3; ++d) cc[d] = (int)floor((pos[d] - g.lower[d]) * g.dxi[d]);
             int cx = wrap(cc[0], g.nx) - i0, cy = wrap(cc[1], g.ny) - j0, lz = cc[2] - k0;
             if ((unsigned)cx >= (unsigned)P2G_TX || (unsigned)cy >= (unsigned)P2G_TY || (unsigned)lz >= (unsigned)tz) {
                 err |= ERR_CELL_MISMATCH;   // not in the cell it was sorted into: left out
@@ -519,9 +525,11 @@ __global__ __launch_bounds__(1024, 4) void k_p2g_tiles(const P2GArgs *__restrict
                 int off[3];
 #pragma unroll
                 for (int d = 0; d < 3; ++d) {
-                    const double r = support_coord(jp, xr[d], su[d], sw[d]), fl = floor(r);
-                    off[d] = (int)fl;
-                    fr[jp][d] = (float)(r - fl);
+                    const double pt = pos[d] + ve[d] * support_cos(jp) + vt[d] * support_sin(jp);
+                    const double xyz = (pt - g.lower[d]) * g.dxi[d];
+                    const double fl = floor(xyz);
+                    off[d] = (int)fl - cc[d];
+                    fr[jp][d] = (float)(xyz - fl);
                 }
                 tgt[jp] = -1;
                 if (cc[2] + off[2] < -1 || cc[2] + off[2] > g.nz) {   // beyond the halo layers (the reference fails too)
@@ -835,7 +843,7 @@ __global__ __launch_bounds__(256) void k_p2g_finalize(const FinalizeArgs *__rest
     const int nz = g.nz;
     const int64_t ncol = (int64_t)g.nx * g.ny;
     const int64_t tq = ib.blk * (int64_t)blockDim.x + threadIdx.x;
-    if (a.clear_tmax && tq <= P2G_NF) gl(a.clear_tmax)[tq] = 0.0f;   // the tile kernel has read them
+    if (tq < P2G_MAXIMA && (a.clear_all || (tq >= 1 && tq <= 3))) gl(a.clear_tmax)[tq] = 0.0f;   // the tile kernel has read them
     if (tq >= ncol * (nz + 3)) return;
     const bool far = *a.far_flag != 0;   // k_far_clear resets it after this kernel
     const int k = (int)(tq / ncol) - 1;
