@@ -480,6 +480,7 @@ void build_p2g(Plan &P, const Members &ms, const std::vector<P2GSel> &sel)
         a.far_acc = m->far_acc;
         a.far_flag = m->far_flag;
         a.far_scale = m->far_scale;
+        a.staged = m->far_flag + 2;
         a.tz = L.tz;
         a.ntx = L.ntx;
         a.nty = L.nty;
@@ -500,6 +501,7 @@ void build_p2g(Plan &P, const Members &ms, const std::vector<P2GSel> &sel)
         f.far_acc = m->far_acc;
         f.far_flag = m->far_flag;
         f.far_scale = m->far_scale;
+        f.staged = m->far_flag + 2;
         far.push_back(FarClearArgs{m->far_acc, m->far_flag, (int64_t)P2G_NF * field_stride(m->g)});
         f.tz = L.tz;
         f.ntx = L.ntx;
@@ -910,7 +912,7 @@ int epic_create(const epic_grid_t *grid, const epic_phys_t *phys, const epic_fla
     const int64_t FS = field_stride(g);
     if (bad(dalloc(&m->fld, (int64_t)F_COUNT * FS, m->s)) || bad(dalloc(&m->nparg, FS, m->s)) || bad(dalloc(&m->nsparg, FS, m->s)) ||
         bad(dalloc(&m->staging, staging_elems_max(g), m->s)) ||
-        bad(dalloc(&m->far_acc, (int64_t)P2G_NF * FS, m->s)) || bad(dalloc(&m->far_flag, 2, m->s)) ||
+        bad(dalloc(&m->far_acc, (int64_t)P2G_NF * FS, m->s)) || bad(dalloc(&m->far_flag, 3, m->s)) ||
         bad(dalloc(&m->far_scale, P2G_NF, m->s)))
         return EPIC_E_NOMEM;
     // vorticity_tendency's 3 (nz + 1) ny nx doubles: a spectrum holds more than nx/2 (nz + 1) ny of them

@@ -85,6 +85,7 @@ struct P2GArgs {
     unsigned long long *far_acc;
     int *far_flag;
     double *far_scale;
+    int *staged;                // set to the fields staged per node, P2G_NF or P2G_DRY
     int tz, ntx, nty, nchz;
 };
 // largest |contribution| per field, |tbuoy - buoy|, and the bounds of the total
@@ -111,12 +112,13 @@ struct FinalizeArgs {
     const unsigned long long *far_acc; // the tile kernel's far-point sums (read when *far_flag)
     const int *far_flag;
     const double *far_scale;
+    const int *staged;
     int tz, ntx, nty, nchz;
 };
 // clears far_acc and then far_flag after a finalize that read them
 struct FarClearArgs {
     unsigned long long *far_acc;
-    int *far_flag;                     // [0] the flag, [1] the clearing blocks' count, kept at 0
+    int *far_flag;                     // [0] the flag, [1] the clearing blocks' count, kept at 0; ([2] is P2GArgs::staged)
     int64_t n;                         // P2G_NF * field_stride
 };
 void add_axes(Plan &P, int phase, const std::vector<AxesArgs> &items);

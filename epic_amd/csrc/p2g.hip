@@ -731,32 +731,51 @@ __global__ __launch_bounds__(1024, 4) void k_p2g_tiles(const P2GArgs *__restrict
     double inv[P2G_NF];
 #pragma unroll
     for (int f = 0; f < P2G_NF; ++f) inv[f] = (sc[f] > 0.0f) ? 1.0 / (double)sc[f] : 0.0;
-    constexpr int PLANE = P2G_BOX * P2G_BOX * P2G_NF;
-    EPIC_GLOBAL double *stage = gl(a.staging) + (int64_t)ib.blk * nbox * PLANE;
-    for (int u = tid; u < nbox * PLANE; u += blockDim.x) {
-        const int f = u % P2G_NF, nd = u / P2G_NF;
-        const int pz = nd / (P2G_BOX * P2G_BOX), yx = nd - pz * (P2G_BOX * P2G_BOX);
-        const int y = yx / P2G_BOX, x = yx - y * P2G_BOX;
-        const int fs = (f == 5 && !own5) ? 4 : f;   // a skipped field 5 is field 4
-        const long long q = (f == 6 && !own6) ? 0ll : fixed_sum(acc[fs * lfield + pz * lplane + y * lp + x]);
-        stage[u] = (double)q * inv[fs];
-    }
+    auto stage = [&](auto fields) {
+        constexpr int NS = decltype(fields)::value, PLANE = P2G_BOX * P2G_BOX * NS;
+        EPIC_GLOBAL double *out = gl(a.staging) + (int64_t)ib.blk * nbox * PLANE;
+        for (int u = tid; u < nbox * PLANE; u += blockDim.x) {
+            const int f = u % NS, nd = u / NS;
+            const int pz = nd / (P2G_BOX * P2G_BOX), yx = nd - pz * (P2G_BOX * P2G_BOX);
+            const int y = yx / P2G_BOX, x = yx - y * P2G_BOX;
+            const int fs = (f == 5 && !own5) ? 4 : f;   // a skipped field 5 is field 4
+            out[u] = (double)fixed_sum(acc[fs * lfield + pz * lplane + y * lp + x]) * inv[fs];
+        }
+    };
+    // without humidity only the fields with sums of their own: the staging is
+    // 400 MB at 128^3 otherwise, written here and read by the finalize
+    const bool dry = !own5 && !own6;
+    if (dry) stage(std::integral_constant<int, P2G_DRY>{});
+    else stage(std::integral_constant<int, P2G_NF>{});
     if (tid == 0 && s_err) atomicOr(a.err, s_err);
     if (tid == 0 && s_far) atomicOr(a.far_flag, 1);
-    if (ib.blk == 0 && tid < P2G_NF) a.far_scale[tid] = inv[tid];   // the same in every work-group
+    if (ib.blk == 0) {   // the same in every work-group
+        if (tid < P2G_NF) a.far_scale[tid] = inv[tid];
+        if (tid == 0) *a.staged = dry ? P2G_DRY : P2G_NF;
+    }
 }
 
 // ---------------------------------------------------------------------------
 // 6. staging sum + folds + normalisation (one thread per (i, j) column)
 // ---------------------------------------------------------------------------
-// tile d = -1, 0, 1 beside the one of node i (of n, nt >= 3 tiles of 8, the
-// last one shorter when n is not a multiple of 8): its number t and the node's
-// place l in its box; false when the box does not hold the node
+// tile d = -1, 0, 1 beside the one of node i (of n >= P2G_BOX nodes in nt >= 2
+// tiles of 8, the last one shorter when n is not a multiple of 8): its number t
+// and the node's place l in its box; false when the box does not hold the node.
+// No box of such a row meets itself, and of two tiles one is beside the other
+// once.
 __device__ inline bool box_place(int d, int i, int n, int nt, int &t, int &l)
 {
     const int own = i >> 3, r = i & 7;
     t = own + d;
     l = r + 1;
+    if (nt == 2) {
+        if (d > 0) return false;
+        if (d < 0) {
+            t = 1 - own;
+            l = wrap(i - (8 * t - 1), n);
+        }
+        return l < P2G_BOX;
+    }
     if (d < 0) {
         if (r > 1) return false;
         l = r + 9;
@@ -774,32 +793,71 @@ __device__ inline bool box_place(int d, int i, int n, int nt, int &t, int &l)
 }
 
 // adds the staged sums of node (i, j, k) to out[], and its far-point sums
-// when there are any (far)
+// when there are any (far).  NS fields are staged; of P2G_DRY, field 5 is
+// field 4 and field 6 zero.  A node lies in one box, or in two (three where
+// the last tile has a single node) along each direction.  The kernel was bound
+// by its waits, one per box; the up to four boxes of a z chunk are loaded
+// together instead: 19.3 -> 11.6 us at 16^3, 24.9 -> 20.9 at 64^3, 143 -> 103 at
+// 128^3 (290 MB of dry staging).  All nine combinations at once take 184
+// registers: 25 and 127 us; several lanes per node do not help.
+template <int NS>
 __device__ inline void stage_add(const FinalizeArgs &a, int i, int j, int k, double out[P2G_NF], bool far)
 {
-    constexpr int PLANE = P2G_BOX * P2G_BOX * P2G_NF;
+    constexpr int PLANE = P2G_BOX * P2G_BOX * NS;
     const Grid &g = a.g;
     if (far) {
         const int64_t FS = field_stride(g), o = ((int64_t)(k + 1) * g.ny + j) * g.nx + i;
 #pragma unroll
         for (int f = 0; f < P2G_NF; ++f) out[f] += (double)fixed_sum(a.far_acc[f * FS + o]) * a.far_scale[f];
     }
+    auto add = [&](auto v) {
+#pragma unroll
+        for (int f = 0; f < NS; ++f) out[f] += v[f];
+        if constexpr (NS == P2G_DRY) out[5] += v[4];
+    };
     const int nbox = a.tz + 3;
     const int cza = (k + 1) / a.tz;
-    if (a.ntx >= 3 && a.nty >= 3) {   // no box meets itself: each neighbour holds a node once or not
+    if (a.ntx >= 2 && a.nty >= 2 && g.nx >= P2G_BOX && g.ny >= P2G_BOX) {
+        // offsets of the boxes' tiles and places along x and y, -1 for none:
+        // its own tile's, a neighbour's, and (a last tile of one node only)
+        // the other neighbour's
+        int64_t ox[3], oy[3];
+        auto places = [&](int64_t o[3], int p, int n, int nt, int64_t tile, int node) {
+#pragma unroll
+            for (int d = -1; d <= 1; ++d) {
+                int t, l;
+                o[d == 0 ? 0 : d < 0 ? 1 : 2] = box_place(d, p, n, nt, t, l) ? t * tile + l * node : -1;
+            }
+            if (o[1] < 0) {
+                o[1] = o[2];
+                o[2] = -1;
+            }
+        };
+        places(ox, i, g.nx, a.ntx, nbox * PLANE, NS);
+        places(oy, j, g.ny, a.nty, (int64_t)a.ntx * nbox * PLANE, P2G_BOX * NS);
+#pragma unroll 1
         for (int dcz = -1; dcz <= 1; ++dcz) {
             const int cz = cza + dcz, lp = k - (cz * a.tz - 2);
             if (cz < 0 || cz >= a.nchz || lp < 0 || lp >= nbox) continue;
-            for (int dty = -1; dty <= 1; ++dty) {
-                int ty, ly;
-                if (!box_place(dty, j, g.ny, a.nty, ty, ly)) continue;
-                for (int dtx = -1; dtx <= 1; ++dtx) {
-                    int tx, lx;
-                    if (!box_place(dtx, i, g.nx, a.ntx, tx, lx)) continue;
-                    const int wg = (cz * a.nty + ty) * a.ntx + tx;
-                    const EPIC_GLOBAL double *s = gl(a.staging) + ((int64_t)wg * nbox + lp) * PLANE + (ly * P2G_BOX + lx) * P2G_NF;
+            const EPIC_GLOBAL double *s = gl(a.staging) + (int64_t)cz * a.nty * a.ntx * nbox * PLANE + lp * PLANE;
+            double v[4][NS];
 #pragma unroll
-                    for (int f = 0; f < P2G_NF; ++f) out[f] += s[f];
+            for (int q = 0; q < 4; ++q) {
+                const int64_t x = ox[q & 1], y = oy[q >> 1];
+#pragma unroll
+                for (int f = 0; f < NS; ++f) v[q][f] = 0.0;
+                if (x >= 0 && y >= 0) {
+#pragma unroll
+                    for (int f = 0; f < NS; ++f) v[q][f] = s[y + x + f];
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) add(v[q]);
+            if (ox[2] >= 0 || oy[2] >= 0) {
+#pragma unroll 1
+                for (int q = 0; q < 5; ++q) {
+                    const int64_t x = q < 3 ? ox[2] : q == 3 ? ox[0] : ox[1], y = q == 0 ? oy[0] : q == 1 ? oy[1] : oy[2];
+                    if (x >= 0 && y >= 0) add(s + y + x);
                 }
             }
         }
@@ -821,9 +879,11 @@ __device__ inline void stage_add(const FinalizeArgs &a, int i, int j, int k, dou
                     const int tx = wrap(txa + dtx, a.ntx);
                     for (int lx = wrap(i - (tx * P2G_TX - 1), g.nx); lx < P2G_BOX; lx += g.nx) {
                         const int wg = (cz * a.nty + ty) * a.ntx + tx;
-                        const EPIC_GLOBAL double *s = gl(a.staging) + ((int64_t)wg * nbox + lp) * PLANE + (ly * P2G_BOX + lx) * P2G_NF;
+                        const EPIC_GLOBAL double *s = gl(a.staging) + ((int64_t)wg * nbox + lp) * PLANE + (ly * P2G_BOX + lx) * NS;
+                        double v[NS];
 #pragma unroll
-                        for (int f = 0; f < P2G_NF; ++f) out[f] += s[f];
+                        for (int f = 0; f < NS; ++f) v[f] = s[f];
+                        add(v);
                     }
                 }
             }
@@ -856,15 +916,20 @@ __global__ __launch_bounds__(256) void k_p2g_finalize(const FinalizeArgs *__rest
     // the node value of plane kk (folds of parcel_interpl.f90:258-287); the
     // staged sums add exactly, the folds and the normalisation run in FP64
     // and each field is rounded to FP32 once, when it is stored
+    const bool dry = *a.staged == P2G_DRY;
+    auto staged = [&](int kk, double r[P2G_NF]) {
+        if (dry) stage_add<P2G_DRY>(a, i, j, kk, r, far);
+        else stage_add<P2G_NF>(a, i, j, kk, r, far);
+    };
     auto folded = [&](int kk, double r[P2G_NF]) {
 #pragma unroll
         for (int f = 0; f < P2G_NF; ++f) r[f] = 0.0;
-        stage_add(a, i, j, kk, r, far);
+        staged(kk, r);
         if (kk == 0 || kk == nz) {
 #pragma unroll
             for (int f = 0; f < P2G_NF; ++f) r[f] *= 2.0;
         } else if (kk == 1 || kk == nz - 1) {
-            stage_add(a, i, j, kk == 1 ? -1 : nz + 1, r, far);
+            staged(kk == 1 ? -1 : nz + 1, r);
         }
     };
     auto zero_zeta = [&](int kk) { return (kk == 0 && g.zeta_zero[0]) || (kk == nz && g.zeta_zero[1]); };
@@ -886,7 +951,7 @@ __global__ __launch_bounds__(256) void k_p2g_finalize(const FinalizeArgs *__rest
         double r[P2G_NF];
 #pragma unroll
         for (int f = 0; f < P2G_NF; ++f) r[f] = 0.0;
-        stage_add(a, i, j, k, r, far);
+        staged(k, r);
         F(F_VOLG, k) = (float)r[0];
         F(F_DBUOYG, k) = (float)r[5];
         F(F_HUMG, k) = (float)r[6];

@@ -23,6 +23,8 @@ GRIDS = [
     (8, 8, 192),      # 193: the LDS form
     (24, 30, 8),      # three and four tiles, the last one partial
     (18, 24, 10),     # a two-cell last tile in x
+    (12, 16, 10),     # two tiles a side
+    (16, 10, 12),     # two tiles, of which one box meets itself in y
     (128, 8, 6),      # long rows beside short y lines
     (8, 128, 6),
     (64, 64, 16),     # 576 work-groups: 256 threads; 2^16 nodes
