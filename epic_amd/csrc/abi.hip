@@ -76,11 +76,10 @@ struct epic_member {
     std::vector<int> ev_phase;
     double timers_ms[EPIC_NUM_TIMERS] = {};
     int timer_calls[EPIC_NUM_TIMERS] = {};
-    // errors; flags_d[0] = reuse the cached axes in the first par2grid of a step
-    int *err_d = nullptr;
-    int *err_h = nullptr;
-    int *flags_d = nullptr;
-    StepTime *tm_d = nullptr, *tm_h = nullptr;   // the step's time step (device, pinned host copy)
+    // the step's time step, axes flag and error word (device, pinned host
+    // copy): one copy there before a step and one back
+    StepTime *tm_d = nullptr, *tm_h = nullptr;
+    int *err_d = nullptr;   // tm_d->err
     std::string msg;
     // launch plans of the call surface (built on first use)
     Plan pl_keys, pl_p2g_fresh, pl_p2g_reuse, pl_vor2vel, pl_vtend, pl_g2p[2], pl_step, pl_step_adaptive;
@@ -272,12 +271,13 @@ int error_code(epic_member *m, int e, const char *where)
 }
 
 // drain the device error word; maps the first error bit to a code
-int check(epic_member *m, const char *where)
+// (copied: the caller enqueued the copy of the whole StepTime)
+int check(epic_member *m, const char *where, bool copied = false)
 {
-    HIPOK(m, hipMemcpyAsync(m->err_h, m->err_d, sizeof(int), hipMemcpyDeviceToHost, m->s));
+    if (!copied) HIPOK(m, hipMemcpyAsync(&m->tm_h->err, m->err_d, sizeof(int), hipMemcpyDeviceToHost, m->s));
     HIPOK(m, hipStreamSynchronize(m->s));
     HIPOK(m, hipGetLastError());
-    const int e = *m->err_h;
+    const int e = m->tm_h->err;
     collect_timers(m);
     if (e == 0) return EPIC_OK;
     HIPOK(m, hipMemsetAsync(m->err_d, 0, sizeof(int), m->s));
@@ -455,13 +455,13 @@ void build_p2g(Plan &P, const Members &ms, const std::vector<P2GSel> &sel)
     std::vector<PlaceArgs> pl;
     std::vector<P2GArgs> ti;
     std::vector<FinalizeArgs> fi;
-    std::vector<FarClearArgs> far;
     for (size_t i = 0; i < ms.size(); ++i) {
         epic_member *m = ms[i];
         const P2GSel &q = sel[i];
         const int64_t nc = ncells(m->g);
-        sc.push_back(ScanArgs{m->cnt[q.rd], nc, m->cell_start, m->bsum, m->cursor});
-        pl.push_back(PlaceArgs{m->n, m->keys, m->cell_start, m->cursor, m->perm, m->cap, m->n_dev});
+        sc.push_back(ScanArgs{m->cnt[q.rd], nc, m->cell_start, m->bsum, m->cursor, m->far_flag, m->far_acc,
+                              (int64_t)P2G_NF * field_stride(m->g)});
+        pl.push_back(PlaceArgs{m->n, m->keys, m->cell_start, m->cursor, m->perm, m->cap, m->n_dev, m->far_flag});
         const P2GLayout L = layout_tz(m->g, m->tz_p2g);
         P2GArgs a{};
         a.g = m->g;
@@ -502,7 +502,6 @@ void build_p2g(Plan &P, const Members &ms, const std::vector<P2GSel> &sel)
         f.far_flag = m->far_flag;
         f.far_scale = m->far_scale;
         f.staged = m->far_flag + 2;
-        far.push_back(FarClearArgs{m->far_acc, m->far_flag, (int64_t)P2G_NF * field_stride(m->g)});
         f.tz = L.tz;
         f.ntx = L.ntx;
         f.nty = L.nty;
@@ -515,7 +514,7 @@ void build_p2g(Plan &P, const Members &ms, const std::vector<P2GSel> &sel)
     if (!mx.empty()) add_p2g_max(P, PH_P2G, mx);
     add_exclusive_scan(P, PH_SORT, sc);
     add_place(P, PH_SORT, pl);
-    add_p2g(P, PH_P2G, ti, fi, far);
+    add_p2g(P, PH_P2G, ti, fi);
 }
 
 FftXArgs xargs(epic_member *m)
@@ -539,8 +538,9 @@ FftYArgs yargs(epic_member *m)
 }
 
 // vor2vel + vel2vgrad: 3 forward transforms, the column solve, 11 inverse
-// transforms, the physical-space completion
-void build_vor2vel(Plan &P, const Members &ms)
+// transforms, the physical-space completion (fix; a step leaves that to the
+// launch of its vorticity tendency)
+void build_vor2vel(Plan &P, const Members &ms, bool fix)
 {
     static const int slots[11] = {F_VORTG + 0, F_VORTG + 1, F_VORTG + 2, F_VELOG + 0, F_VELOG + 1, F_VELOG + 2,
                                   F_VELGRADG + DUDX, F_VELGRADG + DUDY, F_VELGRADG + DVDY, F_VELGRADG + DWDX,
@@ -588,12 +588,12 @@ void build_vor2vel(Plan &P, const Members &ms)
     add_vor2vel_columns(P, PH_VOR2VEL, co);
     add_fft_y(P, PH_VOR2VEL, yi);
     add_fft_xi(P, PH_VOR2VEL, xi);
-    add_vor2vel_fixup(P, PH_VOR2VEL, fx);
+    if (fix) add_vor2vel_fixup(P, PH_VOR2VEL, fx);
 }
 
 // vorticity_tendency; the FP64 x parts take the spectra, which are free
 // between two transforms
-void build_vtend(Plan &P, const Members &ms)
+void build_vtend(Plan &P, const Members &ms, bool fix)
 {
     std::vector<VtendArgs> items;
     for (epic_member *m : ms) {
@@ -607,20 +607,19 @@ void build_vtend(Plan &P, const Members &ms)
         a.dx = (double *)m->spec[0];
         items.push_back(a);
     }
-    add_vtend(P, PH_VTEND, items);
+    add_vtend(P, PH_VTEND, items, fix);
 }
 
 // one LS-RK step (ls_rk.f90:88-136) of every member.  Histograms: stage s
 // sorts by cnt[(s-1)%3] and its push fills cnt[s%3], the last push cnt[0]
 // (never the one the stage read, so par2grid can clear it in parallel).
 // Half axes: stages 1..ns-1 use ax_cur, the last stage ax_stale, which is
-// then the cache the next step's first par2grid takes when *reuse is set.
+// then the cache the next step's first par2grid takes when tm->reuse is set.
 // Stage 1 computes ax_cur from B; the push of stage s < ns stores the axes of
 // the B it writes, which are stage s+1's (ax_cur, or ax_stale for the last).
 struct StepItem {
     epic_member *m;
-    StepTime *tm;        // device: dt (written by the host, or by the adaptive time step)
-    const int *reuse;
+    StepTime *tm;        // device: dt (written by the host, or by the adaptive time step), axes flag
     bool adaptive;
 };
 
@@ -645,12 +644,12 @@ void build_step(Plan &P, const std::vector<StepItem> &items)
             float *const *a = last ? m->ax_stale : m->ax_cur;
             ax.push_back(a);
             const int rd = (s - 1) % 3, wr = last ? 0 : (s % 3);
-            sel.push_back(P2GSel{a, m->ax_stale, s == 1 ? it->reuse : nullptr, rd, wr, s > 1, !last});
+            sel.push_back(P2GSel{a, m->ax_stale, s == 1 ? &it->tm->reuse : nullptr, rd, wr, s > 1, !last});
         }
         if (s == 1) build_axes(P, ms, ax);   // later stages: stored by the previous push
         build_p2g(P, ms, sel);
-        build_vor2vel(P, ms);
-        build_vtend(P, ms);
+        build_vor2vel(P, ms, false);
+        build_vtend(P, ms, true);
         if (s == 1) {   // get_time_step after the first vorticity_tendency (ls_rk.f90:92-101)
             std::vector<TsArgs> ts;
             for (const StepItem *it : act)
@@ -919,10 +918,10 @@ int epic_create(const epic_grid_t *grid, const epic_phys_t *phys, const epic_fla
     static_assert(NSPEC >= 6, "the FP64 x parts of vorticity_tendency take six spectra");
     if (bad(dalloc(&m->spec[0], NSPEC * spec_size(g), m->s))) return EPIC_E_NOMEM;
     for (int i = 1; i < NSPEC; ++i) m->spec[i] = m->spec[0] + i * spec_size(g);
-    if (bad(dalloc(&m->err_d, 4, m->s)) || bad(dalloc(&m->flags_d, 4, m->s)) || bad(dalloc(&m->tm_d, 1, m->s))) return EPIC_E_NOMEM;
+    if (bad(dalloc(&m->tm_d, 1, m->s))) return EPIC_E_NOMEM;
+    m->err_d = &m->tm_d->err;
     if (bad(dalloc(&m->pmax_out, P2G_MAXIMA, m->s))) return EPIC_E_NOMEM;
-    if (bad(hipHostMalloc((void **)&m->err_h, sizeof(int) * 4, hipHostMallocDefault)) ||
-        bad(hipHostMalloc((void **)&m->tm_h, sizeof(StepTime), hipHostMallocDefault)))
+    if (bad(hipHostMalloc((void **)&m->tm_h, sizeof(StepTime), hipHostMallocDefault)))
         return EPIC_E_NOMEM;
     *m->tm_h = StepTime{};
     // twiddles (FP64-accurate roots of unity)
@@ -968,12 +967,11 @@ int epic_destroy(epic_handle m)
     if (m->merge_scratch.base) (void)hipFree(m->merge_scratch.base);
     void *ptrs[] = {m->pos, m->attr, m->orig, m->axbuf, m->keys, m->cnt[0], m->scnt[0], m->cnt[1], m->scnt[1],
                     m->cnt[2], m->scnt[2], m->cell_start, m->cursor, m->perm, m->bsum, m->fld, m->nparg, m->nsparg, m->staging,
-                    m->twx, m->twy, m->twz, m->twx64, m->twy64, m->err_d, m->flags_d, m->vw_d, m->tm_d, m->diag_d,
+                    m->twx, m->twy, m->twz, m->twx64, m->twy64, m->vw_d, m->tm_d, m->diag_d,
                     m->sort_tmp, m->pmax_out, m->tend_src, m->far_acc, m->far_flag, m->far_scale, m->n_dev};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (m->spec[0]) (void)hipFree(m->spec[0]);
-    if (m->err_h) (void)hipHostFree(m->err_h);
     if (m->vw_h) (void)hipHostFree(m->vw_h);
     if (m->tm_h) (void)hipHostFree(m->tm_h);
     if (m->diag_h) (void)hipHostFree(m->diag_h);
@@ -1099,7 +1097,7 @@ int epic_par2grid(epic_handle m, int l_reuse)
 int epic_vor2vel(epic_handle m)
 {
     if (!m) return EPIC_E_INVALID;
-    if (m->pl_vor2vel.empty()) build_vor2vel(m->pl_vor2vel, {m});
+    if (m->pl_vor2vel.empty()) build_vor2vel(m->pl_vor2vel, {m}, true);
     const int rc = run_plan(m, m->pl_vor2vel);
     if (rc) return rc;
     return check(m, "epic_vor2vel");
@@ -1108,7 +1106,7 @@ int epic_vor2vel(epic_handle m)
 int epic_vorticity_tendency(epic_handle m)
 {
     if (!m) return EPIC_E_INVALID;
-    if (m->pl_vtend.empty()) build_vtend(m->pl_vtend, {m});
+    if (m->pl_vtend.empty()) build_vtend(m->pl_vtend, {m}, false);
     const int rc = run_plan(m, m->pl_vtend);
     if (rc) return rc;
     return check(m, "epic_vorticity_tendency");
@@ -1250,20 +1248,19 @@ static int run_step(epic_member *m, double *t, double t_initial, bool adaptive, 
     uint64_t &pg = m->step_gen[adaptive ? 1 : 0];
     if (!P.empty() && pg != m->gen) {   // stale: new tables into the same graph, or a new plan
         Plan Q;
-        build_step(Q, {StepItem{m, m->tm_d, m->flags_d, adaptive}});
+        build_step(Q, {StepItem{m, m->tm_d, adaptive}});
         bool same = false;
         HIPOK(m, P.refresh_from(Q, m->s, &same));
         if (!same) P.swap(Q);   // Q now holds the old plan and releases it
     }
-    if (P.empty()) build_step(P, {StepItem{m, m->tm_d, m->flags_d, adaptive}});
+    if (P.empty()) build_step(P, {StepItem{m, m->tm_d, adaptive}});
     pg = m->gen;
     // the first par2grid of a step reuses the cached axes (ls_rk.f90:93)
-    m->err_h[1] = (*t > t_initial) ? 1 : 0;
+    m->tm_h->reuse = (*t > t_initial) ? 1 : 0;
     m->tm_h->t = *t;
     m->tm_h->adaptive = adaptive ? 1 : 0;
     m->tm_h->gmax_bits = m->tm_h->b2max_bits = 0ull;
-    HIPOK(m, hipMemcpyAsync(m->flags_d, m->err_h + 1, sizeof(int), hipMemcpyHostToDevice, m->s));
-    HIPOK(m, hipMemcpyAsync(m->tm_d, m->tm_h, sizeof(StepTime), hipMemcpyHostToDevice, m->s));
+    HIPOK(m, hipMemcpyAsync(m->tm_d, m->tm_h, offsetof(StepTime, err), hipMemcpyHostToDevice, m->s));
     if (m->profiling == 1) {
         rc = run_plan(m, P);
         if (rc) return rc;
@@ -1272,7 +1269,7 @@ static int run_step(epic_member *m, double *t, double t_initial, bool adaptive, 
     }
     HIPOK(m, hipMemcpyAsync(m->tm_h, m->tm_d, sizeof(StepTime), hipMemcpyDeviceToHost, m->s));
     m->tend_displaced = false;   // every stage rewrote the tendencies in place
-    rc = check(m, where);   // synchronises the stream
+    rc = check(m, where, true);   // synchronises the stream
     if (rc) return rc;
     if (m->profiling == 2) {
         rc = collect_graph_timers(m, P);
@@ -1336,13 +1333,13 @@ int epic_get_time_step(epic_handle m, double t, const epic_time_t *opts, double 
     h.precise_stop = opts->precise_stop ? 1 : 0;
     h.adaptive = 1;
     *m->tm_h = h;
-    HIPOK(m, hipMemcpyAsync(m->tm_d, m->tm_h, sizeof(StepTime), hipMemcpyHostToDevice, m->s));
+    HIPOK(m, hipMemcpyAsync(m->tm_d, m->tm_h, offsetof(StepTime, err), hipMemcpyHostToDevice, m->s));
     {
         Plan P;
         add_time_step(P, PH_OTHER, {TsArgs{m->g, m->fld, m->tm_d, m->err_d}});
         HIPOK(m, P.run(m->s));
         HIPOK(m, hipMemcpyAsync(m->tm_h, m->tm_d, sizeof(StepTime), hipMemcpyDeviceToHost, m->s));
-        const int rc = check(m, "epic_get_time_step");
+        const int rc = check(m, "epic_get_time_step", true);
         if (gmax) *gmax = m->tm_h->gmax;
         if (bmax) *bmax = m->tm_h->bmax;
         if (rc) return rc;
@@ -1383,8 +1380,7 @@ int epic_get_timers(epic_handle m, double *ms, int *calls, int reset)
 struct epic_batch {
     std::vector<epic_member *> ms;
     hipStream_t s = nullptr;
-    int *flags_d = nullptr, *errs_d = nullptr;
-    int *flags_h = nullptr, *errs_h = nullptr;
+    int *errs_d = nullptr, *errs_h = nullptr;
     StepTime *tms_d = nullptr, *tms_h = nullptr;   // one time step per member
     Plan plan;
     std::vector<uint64_t> gens;
@@ -1565,10 +1561,9 @@ int epic_batch_create(const epic_handle *members, int count, epic_batch_handle *
         return false;
     };
     if (bad(hipStreamCreateWithFlags(&b->s, hipStreamNonBlocking))) return EPIC_E_HIP;
-    if (bad(dalloc(&b->flags_d, count, b->s)) || bad(dalloc(&b->errs_d, count, b->s)) || bad(dalloc(&b->tms_d, count, b->s)))
+    if (bad(dalloc(&b->errs_d, count, b->s)) || bad(dalloc(&b->tms_d, count, b->s)))
         return EPIC_E_NOMEM;
-    if (bad(hipHostMalloc((void **)&b->flags_h, sizeof(int) * count, hipHostMallocDefault)) ||
-        bad(hipHostMalloc((void **)&b->errs_h, sizeof(int) * count, hipHostMallocDefault)) ||
+    if (bad(hipHostMalloc((void **)&b->errs_h, sizeof(int) * count, hipHostMallocDefault)) ||
         bad(hipHostMalloc((void **)&b->tms_h, sizeof(StepTime) * count, hipHostMallocDefault)))
         return EPIC_E_NOMEM;
     *out = b;
@@ -1580,9 +1575,7 @@ int epic_batch_destroy(epic_batch_handle b)
     if (!b) return EPIC_OK;
     if (b->s) (void)hipStreamSynchronize(b->s);
     b->plan.release();
-    if (b->flags_d) (void)hipFree(b->flags_d);
     if (b->errs_d) (void)hipFree(b->errs_d);
-    if (b->flags_h) (void)hipHostFree(b->flags_h);
     if (b->errs_h) (void)hipHostFree(b->errs_h);
     if (b->tms_d) (void)hipFree(b->tms_d);
     if (b->tms_h) (void)hipHostFree(b->tms_h);
@@ -1622,7 +1615,7 @@ static int batch_prepare(epic_batch *b)
         std::vector<StepItem> items;
         std::vector<ErrArgs> errs;
         for (int i = 0; i < nm; ++i) {
-            items.push_back(StepItem{b->ms[i], b->tms_d + i, b->flags_d + i, false});
+            items.push_back(StepItem{b->ms[i], b->tms_d + i, false});
             errs.push_back(ErrArgs{b->ms[i]->err_d, b->errs_d + i});
         }
         build_step(Q, items);
@@ -1655,12 +1648,11 @@ int epic_batch_launch(epic_batch_handle b, const double *t, const double *dt, co
     if (rc) return rc;
     // the first par2grid of a step reuses the cached axes (ls_rk.f90:93)
     for (int i = 0; i < nm; ++i) {
-        b->flags_h[i] = (t[i] > t_initial[i]) ? 1 : 0;
         b->tms_h[i] = StepTime{};
+        b->tms_h[i].reuse = (t[i] > t_initial[i]) ? 1 : 0;
         b->tms_h[i].dt = dt[i];
         b->tms_h[i].t = t[i];
     }
-    BHIPOK(b, hipMemcpyAsync(b->flags_d, b->flags_h, sizeof(int) * nm, hipMemcpyHostToDevice, b->s));
     BHIPOK(b, hipMemcpyAsync(b->tms_d, b->tms_h, sizeof(StepTime) * nm, hipMemcpyHostToDevice, b->s));
     BHIPOK(b, b->plan.run_graph(b->s));
     BHIPOK(b, hipMemcpyAsync(b->errs_h, b->errs_d, sizeof(int) * nm, hipMemcpyDeviceToHost, b->s));

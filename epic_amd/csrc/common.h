@@ -43,6 +43,8 @@ struct StepTime {
     double gmax, bmax;                          // maxima of the last adaptive step
     unsigned long long gmax_bits, b2max_bits;   // running maxima (non-negative doubles as bits), kept at 0
     int precise_stop, adaptive;
+    int reuse;   // the first par2grid of the step takes the cached axes
+    int err;     // a member's error word: set by kernels, never written from the host copy
 };
 
 // field slots inside Member::fld (FP32 node fields)

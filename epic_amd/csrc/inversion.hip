@@ -886,50 +886,6 @@ __global__ __launch_bounds__(64) void k_vor2vel_columns_seq(const ColArgs *__res
 #pragma clang diagnostic pop
 #undef ZSLOTS
 
-// ---------------------------------------------------------------------------
-// physical-space completion
-// ---------------------------------------------------------------------------
-// vor2vel: z halo of velocity (inversion.f90:241-248) and the derived
-// gradient components (:278-313); one thread per (column, plane k =
-// -1..nz+1).  A halo-plane thread forms its own halo values (linear
-// extrapolation, or antisymmetry for w and its horizontal derivatives) from
-// the interior planes before the derived components.
-__global__ __launch_bounds__(256) void k_vor2vel_fixup(const FixArgs *__restrict__ tab, const int2 *__restrict__ bmap)
-{
-    const ItemBlock ib = item_block(bmap);
-    const Grid &g = tab[ib.item].g;
-    float *const fld = tab[ib.item].fld;
-    const int nz = g.nz;
-    const int64_t ncol = (int64_t)g.nx * g.ny;
-    const int64_t tq = ib.blk * (int64_t)blockDim.x + threadIdx.x;
-    if (tq >= ncol * (nz + 3)) return;
-    const int k = (int)(tq / ncol) - 1;
-    const int64_t col = tq - (int64_t)(k + 1) * ncol;
-    const int64_t FS = field_stride(g), PS = plane_stride(g);
-    auto F = [&](int slot, int kk) -> EPIC_GLOBAL float & { return gl(fld)[slot * FS + (int64_t)(kk + 1) * PS + col]; };
-    float dwdx, dudy, dwdy;
-    if (k == -1 || k == nz + 1) {
-        const int kb = (k < 0) ? 0 : nz, kn = (k < 0) ? 1 : nz - 1;
-        auto lin = [&](int slot) { return F(slot, k) = 2.0f * F(slot, kb) - F(slot, kn); };
-        auto anti = [&](int slot) { return F(slot, k) = -F(slot, kn); };
-        lin(F_VELOG + 0);
-        lin(F_VELOG + 1);
-        anti(F_VELOG + 2);
-        lin(F_VELGRADG + DUDX);
-        dudy = lin(F_VELGRADG + DUDY);
-        dwdx = anti(F_VELGRADG + DWDX);
-        lin(F_VELGRADG + DVDY);
-        dwdy = anti(F_VELGRADG + DWDY);
-    } else {
-        dwdx = F(F_VELGRADG + DWDX, k);
-        dudy = F(F_VELGRADG + DUDY, k);
-        dwdy = F(F_VELGRADG + DWDY, k);
-    }
-    F(F_VELGRADG + DUDZ, k) = dwdx + F(F_VORTG + 1, k);
-    F(F_VELGRADG + DVDX, k) = dudy + F(F_VORTG + 2, k);
-    F(F_VELGRADG + DVDZ, k) = dwdy - F(F_VORTG + 0, k);
-}
-
 // register slots per lane for a column of nz + 1 values (0: the LDS form)
 static int col_slots(const Grid &g)
 {
@@ -966,13 +922,6 @@ void add_vor2vel_columns(Plan &P, int phase, const std::vector<ColArgs> &items)
         }
         if (!sel.empty()) P.add(kern[ns], 64, lds, phase, sel, nb);
     }
-}
-
-void add_vor2vel_fixup(Plan &P, int phase, const std::vector<FixArgs> &items)
-{
-    std::vector<int> nb;
-    for (const FixArgs &a : items) nb.push_back((int)(((int64_t)a.g.nx * a.g.ny * (a.g.nz + 3) + 255) / 256));
-    P.add((const void *)k_vor2vel_fixup, 256, 0, phase, items, nb);
 }
 
 }  // namespace epic

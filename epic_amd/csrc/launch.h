@@ -33,6 +33,10 @@ struct ScanArgs {
     int *out;      // n + 1 entries: exclusive prefix and total
     int *bsum;     // scan_scratch_ints(n)
     int *clear;    // n entries set to zero on the way (may be null)
+    // far-point sums of the par2grid before, set to zero when *far_flag (may be null)
+    const int *far_flag = nullptr;
+    unsigned long long *far_acc = nullptr;
+    int64_t far_n = 0;
 };
 struct PlaceArgs {
     int64_t n;
@@ -40,11 +44,13 @@ struct PlaceArgs {
     int *cursor, *perm;
     int64_t cap = 0;   // grid size in parcels (0: n)
     const int64_t *n_dev = nullptr;   // when set, the count is read from here instead of n
+    int *far_flag = nullptr;          // set to zero (may be null)
 };
+constexpr int SCAN_SOLO_BLOCKS = 8;
 constexpr int64_t SCAN_FUSED_BLOCKS = 8192;
 int64_t scan_scratch_ints(int64_t n);
 void add_cell_keys(Plan &P, int phase, const std::vector<KeysArgs> &items);
-void add_exclusive_scan(Plan &P, int phase, const std::vector<ScanArgs> &items);   // two or three launches
+void add_exclusive_scan(Plan &P, int phase, const std::vector<ScanArgs> &items);   // one to three launches
 void add_place(Plan &P, int phase, const std::vector<PlaceArgs> &items);
 // order of every cell by caller index (epic_cell_sort only; a direct launch)
 void launch_cell_order(int64_t nc, const int *cell_start, const int *perm_tmp, const int *orig, int *perm,
@@ -115,15 +121,8 @@ struct FinalizeArgs {
     const int *staged;
     int tz, ntx, nty, nchz;
 };
-// clears far_acc and then far_flag after a finalize that read them
-struct FarClearArgs {
-    unsigned long long *far_acc;
-    int *far_flag;                     // [0] the flag, [1] the clearing blocks' count, kept at 0; ([2] is P2GArgs::staged)
-    int64_t n;                         // P2G_NF * field_stride
-};
 void add_axes(Plan &P, int phase, const std::vector<AxesArgs> &items);
-void add_p2g(Plan &P, int phase, const std::vector<P2GArgs> &tiles, const std::vector<FinalizeArgs> &fin,
-             const std::vector<FarClearArgs> &far);
+void add_p2g(Plan &P, int phase, const std::vector<P2GArgs> &tiles, const std::vector<FinalizeArgs> &fin);
 
 // ---- grid2par + push (g2p.hip) ----
 struct G2PArgs {
@@ -203,8 +202,9 @@ struct VtendArgs {
     double *dx;                // scratch: the x parts, 3 (nz + 1) ny nx
     int comp;                  // component, set by add_vtend with the two below
     int lines, planes;         // row pairs per k_flux_dx block, planes per k_flux_dy block
+    int dx_blocks;             // blocks of the x parts; those beyond complete vor2vel
 };
-void add_vtend(Plan &P, int phase, const std::vector<VtendArgs> &members);
+void add_vtend(Plan &P, int phase, const std::vector<VtendArgs> &members, bool fix);
 
 // ---- parcel splitting (split.hip) ----
 struct SplitArgs {

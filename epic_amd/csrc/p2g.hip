@@ -77,7 +77,10 @@ __global__ __launch_bounds__(256) void k_cell_keys(const KeysArgs *__restrict__ 
 // ---------------------------------------------------------------------------
 // 2. exclusive scan: block sums, then every block's own prefix.  A block of
 // the second pass adds up the sums before it itself, so there is no launch
-// for the sums' scan (up to SCAN_FUSED_BLOCKS of them: 32 KB each re-reads)
+// for the sums' scan (up to SCAN_FUSED_BLOCKS of them: 32 KB each re-reads);
+// of at most SCAN_SOLO_BLOCKS a block adds up the entries before it, and the
+// scan is one launch (three blocks at 16^3: 8.8 us in two, 5.4 in one; eight
+// at 24^3: 9.3 and 7.5)
 // ---------------------------------------------------------------------------
 constexpr int SCAN_T = 256;
 constexpr int SCAN_PER = 8;
@@ -105,6 +108,15 @@ __device__ inline int block_excl_scan(int v, int *lds, int &total)
     return base + incl - v;
 }
 
+// the previous par2grid's far-point sums back to zero, when there were any
+// (k_place then resets the flag)
+__device__ inline void clear_far(const ScanArgs &a, int blk)
+{
+    if (!a.far_flag || *a.far_flag == 0) return;
+    const int64_t step = (a.n + SCAN_BLOCK - 1) / SCAN_BLOCK * SCAN_T;
+    for (int64_t q = (int64_t)blk * SCAN_T + threadIdx.x; q < a.far_n; q += step) gl(a.far_acc)[q] = 0ull;
+}
+
 __global__ __launch_bounds__(SCAN_T) void k_scan_reduce(const ScanArgs *__restrict__ tab, const int2 *__restrict__ bmap)
 {
     __shared__ int lds[SCAN_T / 64];
@@ -118,6 +130,7 @@ __global__ __launch_bounds__(SCAN_T) void k_scan_reduce(const ScanArgs *__restri
     int total;
     block_excl_scan(s, lds, total);
     if (threadIdx.x == 0) gl(a.bsum)[ib.blk] = total;
+    clear_far(a, ib.blk);
 }
 
 // one block per item: exclusive scan of the item's block sums in place
@@ -150,9 +163,13 @@ __global__ __launch_bounds__(SCAN_T) void k_scan_blocks(const ScanArgs *__restri
 }
 
 // out[c] = exclusive prefix, out[n] = total; clears gl(a.clear)[c] (the
-// placement cursors) on the way.  FUSED: bsum holds the blocks' sums, not yet
-// their prefixes
-template <bool FUSED>
+// placement cursors) on the way
+enum ScanForm {
+    SCAN_PREFIXES,   // bsum holds the prefixes of the blocks' sums
+    SCAN_SUMS,       // the sums
+    SCAN_ALONE       // nothing yet
+};
+template <ScanForm FORM>
 __global__ __launch_bounds__(SCAN_T) void k_scan_apply(const ScanArgs *__restrict__ tab, const int2 *__restrict__ bmap)
 {
     __shared__ int lds[SCAN_T / 64];
@@ -168,9 +185,17 @@ __global__ __launch_bounds__(SCAN_T) void k_scan_apply(const ScanArgs *__restric
     }
     int total;
     int run = block_excl_scan(s, lds, total);
-    if constexpr (FUSED) {
+    if constexpr (FORM != SCAN_PREFIXES) {
         int before = 0;
-        for (int b = threadIdx.x; b < ib.blk; b += SCAN_T) before += gl(a.bsum)[b];
+        if constexpr (FORM == SCAN_SUMS) {
+            for (int b = threadIdx.x; b < ib.blk; b += SCAN_T) before += gl(a.bsum)[b];
+        } else {
+            for (int b = 0; b < ib.blk; ++b) {
+#pragma unroll
+                for (int u = 0; u < SCAN_PER; ++u) before += gl(a.in)[b * SCAN_BLOCK + u * SCAN_T + threadIdx.x];
+            }
+            clear_far(a, ib.blk);
+        }
         int all;
         (void)block_excl_scan(before, lds, all);
         run += all;
@@ -196,13 +221,20 @@ void add_exclusive_scan(Plan &P, int phase, const std::vector<ScanArgs> &items)
         nb.push_back((int)((a.n + SCAN_BLOCK - 1) / SCAN_BLOCK));
         one.push_back(1);
     }
+    const int most = *std::max_element(nb.begin(), nb.end());
+    bool apart = true;   // blocks read what others may have scanned already
+    for (const ScanArgs &a : items) apart = apart && a.in != a.out && a.in != a.clear;
+    if (apart && most <= SCAN_SOLO_BLOCKS) {
+        P.add((const void *)k_scan_apply<SCAN_ALONE>, SCAN_T, 0, phase, items, nb);
+        return;
+    }
     P.add((const void *)k_scan_reduce, SCAN_T, 0, phase, items, nb);
-    if (*std::max_element(nb.begin(), nb.end()) <= SCAN_FUSED_BLOCKS) {
-        P.add((const void *)k_scan_apply<true>, SCAN_T, 0, phase, items, nb);
+    if (most <= SCAN_FUSED_BLOCKS) {
+        P.add((const void *)k_scan_apply<SCAN_SUMS>, SCAN_T, 0, phase, items, nb);
         return;
     }
     P.add((const void *)k_scan_blocks, SCAN_T, 0, phase, items, one);
-    P.add((const void *)k_scan_apply<false>, SCAN_T, 0, phase, items, nb);
+    P.add((const void *)k_scan_apply<SCAN_PREFIXES>, SCAN_T, 0, phase, items, nb);
 }
 
 int64_t scan_scratch_ints(int64_t n) { return (n + SCAN_BLOCK - 1) / SCAN_BLOCK + 1; }
@@ -221,6 +253,7 @@ __global__ __launch_bounds__(256) void k_place(const PlaceArgs *__restrict__ tab
     constexpr int NR = PER_BLOCK / 256;   // every lane of a wave runs the same rounds
     const int lane = threadIdx.x & 63;
     const int64_t n = a.n_dev ? *a.n_dev : a.n;
+    if (a.far_flag && ib.blk == 0 && threadIdx.x == 0) *a.far_flag = 0;   // its sums were cleared by the scan
     int key[NR], start[NR], head_lane[NR], got[NR];
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
@@ -905,7 +938,7 @@ __global__ __launch_bounds__(256) void k_p2g_finalize(const FinalizeArgs *__rest
     const int64_t tq = ib.blk * (int64_t)blockDim.x + threadIdx.x;
     if (tq < P2G_MAXIMA && (a.clear_all || (tq >= 1 && tq <= 3))) gl(a.clear_tmax)[tq] = 0.0f;   // the tile kernel has read them
     if (tq >= ncol * (nz + 3)) return;
-    const bool far = *a.far_flag != 0;   // k_far_clear resets it after this kernel
+    const bool far = *a.far_flag != 0;   // reset by the next sort
     const int k = (int)(tq / ncol) - 1;
     const int64_t col = tq - (int64_t)(k + 1) * ncol;
     const int i = (int)(col % g.nx), j = (int)(col / g.nx);
@@ -1084,27 +1117,7 @@ P2GLayout p2g_layout(const Grid &g)
 
 size_t p2g_lds_bytes(int tz) { return sizeof(unsigned long long) * P2G_NF * box_planes(tz) * P2G_BOX * p2g_lpitch(tz); }
 
-// after a finalize: the far-point accumulator back to zero (only when the
-// tile kernel put terms there), then the flag
-constexpr int FAR_CLEAR_BLOCKS = 1024;
-__global__ __launch_bounds__(256) void k_far_clear(const FarClearArgs *__restrict__ tab, const int2 *__restrict__ bmap)
-{
-    const ItemBlock ib = item_block(bmap);
-    const FarClearArgs &a = tab[ib.item];
-    // the flag changes only once every block has counted itself below, so the
-    // blocks of an item agree on it
-    if (*a.far_flag == 0) return;
-    for (int64_t q = (int64_t)ib.blk * 256 + threadIdx.x; q < a.n; q += (int64_t)FAR_CLEAR_BLOCKS * 256)
-        gl(a.far_acc)[q] = 0ull;
-    __syncthreads();
-    if (threadIdx.x == 0 && atomicAdd(a.far_flag + 1, 1) == FAR_CLEAR_BLOCKS - 1) {
-        a.far_flag[1] = 0;
-        a.far_flag[0] = 0;
-    }
-}
-
-void add_p2g(Plan &P, int phase, const std::vector<P2GArgs> &tiles, const std::vector<FinalizeArgs> &fin,
-             const std::vector<FarClearArgs> &far)
+void add_p2g(Plan &P, int phase, const std::vector<P2GArgs> &tiles, const std::vector<FinalizeArgs> &fin)
 {
     // one grouped launch per z chunk, the kernel specialised on it
     // (epic_set_tiling and the autotuner admit 2, 4 and 8 only)
@@ -1129,8 +1142,6 @@ void add_p2g(Plan &P, int phase, const std::vector<P2GArgs> &tiles, const std::v
     std::vector<int> nf;
     for (const FinalizeArgs &f : fin) nf.push_back((int)(((int64_t)f.g.nx * f.g.ny * (f.g.nz + 3) + 255) / 256));
     P.add((const void *)k_p2g_finalize, 256, 0, phase, fin, nf);
-    std::vector<int> nc(far.size(), FAR_CLEAR_BLOCKS);
-    P.add((const void *)k_far_clear, 256, 0, phase, far, nc);
 }
 
 }  // namespace epic

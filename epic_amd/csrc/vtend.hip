@@ -63,6 +63,63 @@ __device__ inline void times_ik(double2 *Z, int L, int ls, const FftPlan &pl, do
     __syncthreads();
 }
 
+// ---------------------------------------------------------------------------
+// physical-space completion
+// ---------------------------------------------------------------------------
+// vor2vel: z halo of velocity (inversion.f90:241-248) and the derived
+// gradient components (:278-313); one thread per (column, plane k =
+// -1..nz+1).  A halo-plane thread forms its own halo values (linear
+// extrapolation, or antisymmetry for w and its horizontal derivatives) from
+// the interior planes before the derived components.  In a step these are
+// further blocks of k_flux_dx, which reads neither the halo planes nor the
+// gradient (a launch of 4 to 5 us less on small grids).
+__device__ inline void vor2vel_fixup(const Grid &g, float *fld, int64_t tq)
+{
+    const int nz = g.nz;
+    const int64_t ncol = (int64_t)g.nx * g.ny;
+    if (tq >= ncol * (nz + 3)) return;
+    const int k = (int)(tq / ncol) - 1;
+    const int64_t col = tq - (int64_t)(k + 1) * ncol;
+    const int64_t FS = field_stride(g), PS = plane_stride(g);
+    auto F = [&](int slot, int kk) -> EPIC_GLOBAL float & { return gl(fld)[slot * FS + (int64_t)(kk + 1) * PS + col]; };
+    float dwdx, dudy, dwdy;
+    if (k == -1 || k == nz + 1) {
+        const int kb = (k < 0) ? 0 : nz, kn = (k < 0) ? 1 : nz - 1;
+        auto lin = [&](int slot) { return F(slot, k) = 2.0f * F(slot, kb) - F(slot, kn); };
+        auto anti = [&](int slot) { return F(slot, k) = -F(slot, kn); };
+        lin(F_VELOG + 0);
+        lin(F_VELOG + 1);
+        anti(F_VELOG + 2);
+        lin(F_VELGRADG + DUDX);
+        dudy = lin(F_VELGRADG + DUDY);
+        dwdx = anti(F_VELGRADG + DWDX);
+        lin(F_VELGRADG + DVDY);
+        dwdy = anti(F_VELGRADG + DWDY);
+    } else {
+        dwdx = F(F_VELGRADG + DWDX, k);
+        dudy = F(F_VELGRADG + DUDY, k);
+        dwdy = F(F_VELGRADG + DWDY, k);
+    }
+    F(F_VELGRADG + DUDZ, k) = dwdx + F(F_VORTG + 1, k);
+    F(F_VELGRADG + DVDX, k) = dudy + F(F_VORTG + 2, k);
+    F(F_VELGRADG + DVDZ, k) = dwdy - F(F_VORTG + 0, k);
+}
+
+__global__ __launch_bounds__(256) void k_vor2vel_fixup(const FixArgs *__restrict__ tab, const int2 *__restrict__ bmap)
+{
+    const ItemBlock ib = item_block(bmap);
+    vor2vel_fixup(tab[ib.item].g, tab[ib.item].fld, ib.blk * (int64_t)256 + threadIdx.x);
+}
+
+static int fixup_blocks(const Grid &g) { return (int)(((int64_t)g.nx * g.ny * (g.nz + 3) + 255) / 256); }
+
+void add_vor2vel_fixup(Plan &P, int phase, const std::vector<FixArgs> &items)
+{
+    std::vector<int> nb;
+    for (const FixArgs &a : items) nb.push_back(fixup_blocks(a.g));
+    P.add((const void *)k_vor2vel_fixup, 256, 0, phase, items, nb);
+}
+
 // x derivative of the x flux of one component on planes 0..nz, rows (plane,
 // j) taken in pairs; a.lines pairs per block
 __global__ __launch_bounds__(256) void k_flux_dx(const VtendArgs *__restrict__ tab, const int2 *__restrict__ bmap)
@@ -70,6 +127,10 @@ __global__ __launch_bounds__(256) void k_flux_dx(const VtendArgs *__restrict__ t
     const ItemBlock ib = item_block(bmap);
     const VtendArgs &a = tab[ib.item];
     const Grid &g = a.g;
+    if (ib.blk >= a.dx_blocks) {   // uniform over the block
+        vor2vel_fixup(g, a.fld, (ib.blk - a.dx_blocks) * (int64_t)256 + threadIdx.x);
+        return;
+    }
     const int n = g.nx, L = a.lines, ls = n + 1;
     const int64_t rows = (int64_t)(g.nz + 1) * g.ny, r0 = (int64_t)ib.blk * 2 * L;
     extern __shared__ double2 lds[];
@@ -223,7 +284,7 @@ static int block_points(const Grid &g) { return (int64_t)g.nx * g.ny * (g.nz + 1
 static int dx_lines(const Grid &g) { return std::max(1, block_points(g) / g.nx); }
 static int dy_planes(const Grid &g) { return std::max(1, block_points(g) / (VT_PAIRS * g.ny)); }
 
-void add_vtend(Plan &P, int phase, const std::vector<VtendArgs> &members)
+void add_vtend(Plan &P, int phase, const std::vector<VtendArgs> &members, bool fix)
 {
     std::vector<VtendArgs> items;
     std::vector<int> bx, by;
@@ -237,8 +298,9 @@ void add_vtend(Plan &P, int phase, const std::vector<VtendArgs> &members)
         ly = std::max(ly, sizeof(double2) * (2 * (size_t)VT_PAIRS * a.planes * (g.ny + 1) + g.ny));
         for (int c = 0; c < 3; ++c) {
             a.comp = c;
+            a.dx_blocks = (int)((rows + 2 * a.lines - 1) / (2 * a.lines));
             items.push_back(a);
-            bx.push_back((int)((rows + 2 * a.lines - 1) / (2 * a.lines)));
+            bx.push_back(a.dx_blocks + (fix && c == 0 ? fixup_blocks(g) : 0));
             by.push_back((g.nx + VT_COLS - 1) / VT_COLS * ((g.nz + 3 + a.planes - 1) / a.planes));
         }
     }

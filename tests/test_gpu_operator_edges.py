@@ -27,6 +27,8 @@ GRIDS = [
     (16, 10, 12),     # two tiles, of which one box meets itself in y
     (128, 8, 6),      # long rows beside short y lines
     (8, 128, 6),
+    (16, 32, 30),     # 8 x 2048 cells: the one-launch scan, and one block more
+    (16, 32, 32),
     (64, 64, 16),     # 576 work-groups: 256 threads; 2^16 nodes
     (64, 40, 15),     # 360 work-groups: 512 threads
 ]
