@@ -115,13 +115,16 @@ __device__ inline int fdiv(int x, const FastDiv &f) { return f.d == 1 ? x : (int
 // The index arithmetic of the transforms stays below 2^16 (at most ZB lines
 // of FFT_MAX_N points).
 constexpr int FFT_MAX_N = 2048;
+struct FftStage {   // (together, so that a stage's numbers are one scalar load)
+    int radix;
+    int tstep;    // n / (ns radix), the twiddle stride
+    FastDiv nb;   // n / radix
+    FastDiv ns;   // the product of the earlier radices
+};
 struct FftPlan {
     int n;          // complex length
     int nst;        // number of stages
-    int radix[16];
-    FastDiv nb[16];   // per stage: n / radix
-    FastDiv ns[16];   // per stage: the product of the earlier radices
-    int tstep[16];    // per stage: n / (ns radix), the twiddle stride
+    FftStage st[16];
     FastDiv n1, n2;   // n and 2 n
 };
 

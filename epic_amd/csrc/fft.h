@@ -112,12 +112,15 @@ template <typename T2, typename TW>
 __device__ T2 *lds_fft_tw(T2 *a, T2 *b, int L, const FftPlan &pl, const TW &tw, bool inv, int ls)
 {
     T2 *in = a, *out = b;
-    for (int st = 0; st < pl.nst; ++st) {
-        const int R = pl.radix[st];
-        if (R == 4) fft_stage<4>(in, out, L, ls, pl.nb[st], pl.ns[st], pl.tstep[st], tw, inv);
-        else if (R == 2) fft_stage<2>(in, out, L, ls, pl.nb[st], pl.ns[st], pl.tstep[st], tw, inv);
-        else if (R == 3) fft_stage<3>(in, out, L, ls, pl.nb[st], pl.ns[st], pl.tstep[st], tw, inv);
-        else fft_stage<5>(in, out, L, ls, pl.nb[st], pl.ns[st], pl.tstep[st], tw, inv);
+    const int nst = pl.nst;
+    FftStage next = pl.st[0];
+    for (int st = 0; st < nst; ++st) {
+        const FftStage g = next;
+        next = pl.st[min(st + 1, nst - 1)];   // requested a stage ahead
+        if (g.radix == 4) fft_stage<4>(in, out, L, ls, g.nb, g.ns, g.tstep, tw, inv);
+        else if (g.radix == 2) fft_stage<2>(in, out, L, ls, g.nb, g.ns, g.tstep, tw, inv);
+        else if (g.radix == 3) fft_stage<3>(in, out, L, ls, g.nb, g.ns, g.tstep, tw, inv);
+        else fft_stage<5>(in, out, L, ls, g.nb, g.ns, g.tstep, tw, inv);
         __syncthreads();
         T2 *tmp = in;
         in = out;
@@ -138,20 +141,21 @@ inline FftPlan make_plan(int n)
     FftPlan p{};
     p.n = n;
     int m = n;
-    while (m % 4 == 0) { p.radix[p.nst++] = 4; m /= 4; }
-    while (m % 2 == 0) { p.radix[p.nst++] = 2; m /= 2; }
-    while (m % 3 == 0) { p.radix[p.nst++] = 3; m /= 3; }
-    while (m % 5 == 0) { p.radix[p.nst++] = 5; m /= 5; }
+    while (m % 4 == 0) { p.st[p.nst++].radix = 4; m /= 4; }
+    while (m % 2 == 0) { p.st[p.nst++].radix = 2; m /= 2; }
+    while (m % 3 == 0) { p.st[p.nst++].radix = 3; m /= 3; }
+    while (m % 5 == 0) { p.st[p.nst++].radix = 5; m /= 5; }
     if (m != 1 || n > FFT_MAX_N) {   // unsupported length
         p.nst = -1;
         return p;
     }
     int ns = 1;
     for (int st = 0; st < p.nst; ++st) {
-        p.nb[st] = make_fastdiv(n / p.radix[st]);
-        p.ns[st] = make_fastdiv(ns);
-        p.tstep[st] = n / (ns * p.radix[st]);
-        ns *= p.radix[st];
+        FftStage &g = p.st[st];
+        g.nb = make_fastdiv(n / g.radix);
+        g.ns = make_fastdiv(ns);
+        g.tstep = n / (ns * g.radix);
+        ns *= g.radix;
     }
     p.n1 = make_fastdiv(n);
     p.n2 = make_fastdiv(2 * n);

@@ -16,11 +16,13 @@ TOL = 1.0e-5
 
 GRIDS = [
     (8, 8, 4),        # one tile, two-point-wide blocks, shortest column
-    (10, 8, 60),      # 61 values of a column: one slot
-    (8, 10, 64),      # 65: two slots
-    (8, 8, 125),      # 126: two slots, radix 5 in z
-    (8, 8, 128),      # 129: three slots
-    (8, 8, 192),      # 193: the LDS form
+    (10, 8, 60),      # 59 inner values of a column: one slot
+    (8, 10, 64),      # 63: one slot, the longest line
+    (8, 8, 72),       # two slots, radix 3 in z
+    (8, 8, 125),      # two slots, radix 5
+    (8, 8, 128),      # two slots, the longest line
+    (8, 8, 135),      # three slots
+    (8, 8, 192),      # the LDS form
     (24, 30, 8),      # three and four tiles, the last one partial
     (18, 24, 10),     # a two-cell last tile in x
     (12, 16, 10),     # two tiles a side
