@@ -424,7 +424,9 @@ void build_keys(Plan &P, const Members &ms)
     add_cell_keys(P, PH_SORT, k);
 }
 
-void build_axes(Plan &P, const Members &ms, const std::vector<float *const *> &ax)
+P2GMaxArgs max_args(epic_member *m) { return P2GMaxArgs{m->g, m->pd, p2g_max_blocks(m->cap), m->pmax_out}; }
+
+void build_axes(Plan &P, const Members &ms, const std::vector<float *const *> &ax, bool maxima)
 {
     std::vector<AxesArgs> v;
     for (size_t i = 0; i < ms.size(); ++i) {
@@ -432,9 +434,11 @@ void build_axes(Plan &P, const Members &ms, const std::vector<float *const *> &a
         a.p = ms[i]->pd;
         for (int c = 0; c < 6; ++c) a.ax[c] = ax[i][c];
         a.err = ms[i]->err_d;
+        a.max = max_args(ms[i]);
         v.push_back(a);
     }
-    add_axes(P, PH_AXES, v);
+    if (maxima) add_axes_max(P, PH_AXES, v);
+    else add_axes(P, PH_AXES, v);
 }
 
 // sort by the histogram rd, scatter with the axes ax (ax_alt when *use_alt),
@@ -446,6 +450,7 @@ struct P2GSel {
     int rd;
     int clr;                  // -1: none
     bool max_from_push = false;   // the previous push and stages left the fixed-point maxima: no k_p2g_max
+    bool max_done = false;        // k_axes_max has taken them
     bool push_next = false;       // a push that fills the vorticity's maxima follows: the others stay
 };
 
@@ -510,7 +515,7 @@ void build_p2g(Plan &P, const Members &ms, const std::vector<P2GSel> &sel)
     }
     std::vector<P2GMaxArgs> mx;
     for (size_t i = 0; i < ms.size(); ++i)
-        if (!sel[i].max_from_push) mx.push_back(P2GMaxArgs{ms[i]->g, ms[i]->pd, p2g_max_blocks(ms[i]->cap), ms[i]->pmax_out});
+        if (!sel[i].max_from_push && !sel[i].max_done) mx.push_back(max_args(ms[i]));
     if (!mx.empty()) add_p2g_max(P, PH_P2G, mx);
     add_exclusive_scan(P, PH_SORT, sc);
     add_place(P, PH_SORT, pl);
@@ -644,9 +649,9 @@ void build_step(Plan &P, const std::vector<StepItem> &items)
             float *const *a = last ? m->ax_stale : m->ax_cur;
             ax.push_back(a);
             const int rd = (s - 1) % 3, wr = last ? 0 : (s % 3);
-            sel.push_back(P2GSel{a, m->ax_stale, s == 1 ? &it->tm->reuse : nullptr, rd, wr, s > 1, !last});
+            sel.push_back(P2GSel{a, m->ax_stale, s == 1 ? &it->tm->reuse : nullptr, rd, wr, s > 1, s == 1, !last});
         }
-        if (s == 1) build_axes(P, ms, ax);   // later stages: stored by the previous push
+        if (s == 1) build_axes(P, ms, ax, true);   // later stages: stored by the previous push
         build_p2g(P, ms, sel);
         build_vor2vel(P, ms, false);
         build_vtend(P, ms, true);
@@ -749,7 +754,7 @@ int ensure_keys(epic_member *m)
 int ensure_axes(epic_member *m)
 {
     if (!m->axes_dirty) return EPIC_OK;
-    if (m->pl_axes.empty()) build_axes(m->pl_axes, {m}, {m->ax_stale});
+    if (m->pl_axes.empty()) build_axes(m->pl_axes, {m}, {m->ax_stale}, false);
     const int rc = run_plan(m, m->pl_axes);
     if (rc == EPIC_OK) m->axes_dirty = false;
     return rc;
@@ -1081,8 +1086,8 @@ int epic_par2grid(epic_handle m, int l_reuse)
     // with l_reuse the stored ones are taken
     Plan &P = (l_reuse == 1) ? m->pl_p2g_reuse : m->pl_p2g_fresh;
     if (P.empty()) {
-        if (l_reuse != 1) build_axes(P, {m}, {m->ax_stale});
-        build_p2g(P, {m}, {P2GSel{m->ax_stale, nullptr, nullptr, 0, -1}});
+        if (l_reuse != 1) build_axes(P, {m}, {m->ax_stale}, true);
+        build_p2g(P, {m}, {P2GSel{m->ax_stale, nullptr, nullptr, 0, -1, false, l_reuse != 1}});
     }
     if (l_reuse == 1) {
         rc = ensure_axes(m);
@@ -1458,7 +1463,7 @@ int epic_autotune(epic_handle m, int *tz_p2g, int *tz_g2p)
     if (rc) return rc;
     {
         Plan P;
-        build_axes(P, {m}, {m->ax_cur});
+        build_axes(P, {m}, {m->ax_cur}, false);
         HIPOK(m, P.run(m->s));
     }
     float best_p = 1e30f, best_g = 1e30f;

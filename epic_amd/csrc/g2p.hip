@@ -453,7 +453,10 @@ __global__ __launch_bounds__(NT, 4) void k_g2p_tiles(const G2PTileArgs *__restri
     }
     if (a.tmax_next) {
         __syncthreads();
-        if (tid < 3 && s_pmax[tid]) atomicMax((unsigned int *)a.tmax_next + 1 + tid, s_pmax[tid]);
+        if (tid < 3) {   // only what is above the maximum there (atomics on one address take turns)
+            unsigned int *out = (unsigned int *)a.tmax_next + 1 + tid;
+            if (s_pmax[tid] > __hip_atomic_load(out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(out, s_pmax[tid]);
+        }
     }
     if (e) atomicOr(a.err, e);
 }

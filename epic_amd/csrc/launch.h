@@ -57,11 +57,6 @@ void launch_cell_order(int64_t nc, const int *cell_start, const int *perm_tmp, c
                        hipStream_t s);
 
 // ---- support-point half axes + par2grid (p2g.hip) ----
-struct AxesArgs {
-    ParcelsDev p;
-    float *ax[6];   // Veta (3), Vtau (3)
-    int *err;
-};
 // default z chunk of the tile scatter: 4 layers where that still leaves four
 // work-groups of 1024 parcels per CU.  Boxes of 7 planes for 4 layers stage
 // 30 % less than of 5 for 2 (par2grid per step: 5.46 -> 5.20 ms at 128^3, 0.94
@@ -104,6 +99,12 @@ struct P2GMaxArgs {
     int nblk;                   // p2g_max_blocks(p.n)
     float *out;                 // P2G_MAXIMA, zero on entry; cleared again by the finalize kernel
 };
+struct AxesArgs {
+    ParcelsDev p;
+    float *ax[6];   // Veta (3), Vtau (3)
+    int *err;
+    P2GMaxArgs max;   // k_axes_max only
+};
 int p2g_max_blocks(int64_t n);
 void add_p2g_max(Plan &P, int phase, const std::vector<P2GMaxArgs> &items);
 struct FinalizeArgs {
@@ -122,6 +123,7 @@ struct FinalizeArgs {
     int tz, ntx, nty, nchz;
 };
 void add_axes(Plan &P, int phase, const std::vector<AxesArgs> &items);
+void add_axes_max(Plan &P, int phase, const std::vector<AxesArgs> &items);
 void add_p2g(Plan &P, int phase, const std::vector<P2GArgs> &tiles, const std::vector<FinalizeArgs> &fin);
 
 // ---- grid2par + push (g2p.hip) ----

@@ -409,24 +409,22 @@ __device__ inline void p2g_values(const Grid &g, const ParcelsDev &p, unsigned o
 // humidity; P2G_MAX_BOUND onwards).  A scale from a bound is at most one power
 // of two coarser, and the fixed-point sums keep a factor 2 of headroom for
 // rounding.
-__global__ __launch_bounds__(256) void k_p2g_max(const P2GMaxArgs *__restrict__ tab, const int2 *__restrict__ bmap)
+__device__ inline void take_maxima(const Grid &g, const ParcelsDev &p, int64_t q, float mx[P2G_MAXIMA])
 {
-    const ItemBlock ib = item_block(bmap);
-    const P2GMaxArgs &a = tab[ib.item];
-    float mx[P2G_MAXIMA];
+    float v[P2G_NF];
+    p2g_values(g, p, (unsigned)q * 4u, gl(p.z)[q], v);
 #pragma unroll
-    for (int f = 0; f < P2G_MAXIMA; ++f) mx[f] = 0.0f;
-    const int64_t n = parcel_count(a.p);
-    for (int64_t q = (int64_t)ib.blk * 256 + threadIdx.x; q < n; q += (int64_t)a.nblk * 256) {
-        float v[P2G_NF];
-        p2g_values(a.g, a.p, (unsigned)q * 4u, gl(a.p.z)[q], v);
-#pragma unroll
-        for (int f = 0; f < P2G_NF; ++f) mx[f] = fmaxf(mx[f], fabsf(v[f]));
-        mx[P2G_NF] = fmaxf(mx[P2G_NF], fabsf(v[4] - v[5]));
-        const float hb = fabsf(v[0] * (float)a.g.glat * at(a.p.hum, (unsigned)q * 4u));
-        mx[P2G_MAX_BOUND] = fmaxf(mx[P2G_MAX_BOUND], fabsf(v[5]) + hb);
-        mx[P2G_MAX_BOUND + 1] = fmaxf(mx[P2G_MAX_BOUND + 1], hb);
-    }
+    for (int f = 0; f < P2G_NF; ++f) mx[f] = fmaxf(mx[f], fabsf(v[f]));
+    mx[P2G_NF] = fmaxf(mx[P2G_NF], fabsf(v[4] - v[5]));
+    const float hb = fabsf(v[0] * (float)g.glat * at(p.hum, (unsigned)q * 4u));
+    mx[P2G_MAX_BOUND] = fmaxf(mx[P2G_MAX_BOUND], fabsf(v[5]) + hb);
+    mx[P2G_MAX_BOUND + 1] = fmaxf(mx[P2G_MAX_BOUND + 1], hb);
+}
+// the block's maxima to out[] (256 threads).  A block whose maximum is not
+// above the one already there leaves it: atomics on one address take turns
+// across the chip
+__device__ inline void put_maxima(float mx[P2G_MAXIMA], float *out)
+{
     __shared__ float wm[4][P2G_MAXIMA];
 #pragma unroll
     for (int f = 0; f < P2G_MAXIMA; ++f) {
@@ -437,8 +435,20 @@ __global__ __launch_bounds__(256) void k_p2g_max(const P2GMaxArgs *__restrict__ 
     if (threadIdx.x < P2G_MAXIMA) {
         const int f = threadIdx.x;
         const float m = fmaxf(fmaxf(wm[0][f], wm[1][f]), fmaxf(wm[2][f], wm[3][f]));
-        if (m > 0.0f) atomicMax((unsigned int *)a.out + f, __float_as_uint(m));
+        if (m > __hip_atomic_load(out + f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            atomicMax((unsigned int *)out + f, __float_as_uint(m));
     }
+}
+__global__ __launch_bounds__(256) void k_p2g_max(const P2GMaxArgs *__restrict__ tab, const int2 *__restrict__ bmap)
+{
+    const ItemBlock ib = item_block(bmap);
+    const P2GMaxArgs &a = tab[ib.item];
+    float mx[P2G_MAXIMA];
+#pragma unroll
+    for (int f = 0; f < P2G_MAXIMA; ++f) mx[f] = 0.0f;
+    const int64_t n = parcel_count(a.p);
+    for (int64_t q = (int64_t)ib.blk * 256 + threadIdx.x; q < n; q += (int64_t)a.nblk * 256) take_maxima(a.g, a.p, q, mx);
+    put_maxima(mx, a.out);
 }
 
 // TZ (= a.tz) is a template parameter, so the LDS strides are constants and
@@ -1025,29 +1035,50 @@ __global__ __launch_bounds__(256) void k_p2g_finalize(const FinalizeArgs *__rest
 // ---------------------------------------------------------------------------
 // support-point half axes, once per parcel per stage (FP64 eigen-solve)
 // ---------------------------------------------------------------------------
+__device__ inline void store_axes(const ParcelsDev &p, float *const ax[6], int64_t q, int &e)
+{
+    const double B[5] = {gl(p.B[0])[q], gl(p.B[1])[q], gl(p.B[2])[q], gl(p.B[3])[q], gl(p.B[4])[q]};
+    double ve[3], vt[3];
+    if (!support_axes(B, (double)gl(p.vol)[q], ve, vt)) {
+        e |= ERR_B33;
+        ve[0] = ve[1] = ve[2] = vt[0] = vt[1] = vt[2] = 0.0;
+    }
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        gl(ax[d])[q] = (float)ve[d];
+        gl(ax[3 + d])[q] = (float)vt[d];
+    }
+}
 __global__ __launch_bounds__(256) void k_axes(const AxesArgs *__restrict__ tab, const int2 *__restrict__ bmap)
 {
     const ItemBlock ib = item_block(bmap);
     const AxesArgs &a = tab[ib.item];
-    const ParcelsDev &p = a.p;
-    const int64_t n = parcel_count(p);
+    const int64_t n = parcel_count(a.p);
     int e = 0;
 #pragma unroll
     for (int r = 0; r < PER_BLOCK / 256; ++r) {
         const int64_t q = (int64_t)ib.blk * PER_BLOCK + r * 256 + threadIdx.x;
         if (q >= n) break;
-        const double B[5] = {gl(p.B[0])[q], gl(p.B[1])[q], gl(p.B[2])[q], gl(p.B[3])[q], gl(p.B[4])[q]};
-        double ve[3], vt[3];
-        if (!support_axes(B, (double)gl(p.vol)[q], ve, vt)) {
-            e |= ERR_B33;
-            ve[0] = ve[1] = ve[2] = vt[0] = vt[1] = vt[2] = 0.0;
-        }
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            gl(a.ax[d])[q] = (float)ve[d];
-            gl(a.ax[3 + d])[q] = (float)vt[d];
-        }
+        store_axes(a.p, a.ax, q, e);
     }
+    if (e) atomicOr(a.err, e);
+}
+// the axes and k_p2g_max's maxima in one pass, where a par2grid needs both
+// (43 + 35 us at 64^3 in two, 62 in one; 288 + 111 and 349 at 128^3)
+__global__ __launch_bounds__(256) void k_axes_max(const AxesArgs *__restrict__ tab, const int2 *__restrict__ bmap)
+{
+    const ItemBlock ib = item_block(bmap);
+    const AxesArgs &a = tab[ib.item];
+    const int64_t n = parcel_count(a.p);
+    float mx[P2G_MAXIMA];
+#pragma unroll
+    for (int f = 0; f < P2G_MAXIMA; ++f) mx[f] = 0.0f;
+    int e = 0;
+    for (int64_t q = (int64_t)ib.blk * 256 + threadIdx.x; q < n; q += (int64_t)a.max.nblk * 256) {
+        take_maxima(a.max.g, a.p, q, mx);
+        store_axes(a.p, a.ax, q, e);
+    }
+    put_maxima(mx, a.max.out);
     if (e) atomicOr(a.err, e);
 }
 
@@ -1093,6 +1124,12 @@ void add_axes(Plan &P, int phase, const std::vector<AxesArgs> &items)
     std::vector<int64_t> n;
     for (const AxesArgs &a : items) n.push_back(grid_parcels(a.p));
     P.add((const void *)k_axes, 256, 0, phase, items, parcel_blocks_of(n));
+}
+void add_axes_max(Plan &P, int phase, const std::vector<AxesArgs> &items)
+{
+    std::vector<int> nb;
+    for (const AxesArgs &a : items) nb.push_back(a.max.nblk);
+    P.add((const void *)k_axes_max, 256, 0, phase, items, nb);
 }
 
 void launch_cell_order(int64_t nc, const int *cell_start, const int *perm_tmp, const int *orig, int *perm, hipStream_t s)
