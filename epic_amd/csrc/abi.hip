@@ -588,11 +588,9 @@ void build_vor2vel(Plan &P, const Members &ms, bool fix)
         }
         fx.push_back(FixArgs{m->g, m->fld});
     }
-    add_fft_xf(P, PH_VOR2VEL, xf);
-    add_fft_y(P, PH_VOR2VEL, yf);
+    add_fft_forward(P, PH_VOR2VEL, xf, yf);
     add_vor2vel_columns(P, PH_VOR2VEL, co);
-    add_fft_y(P, PH_VOR2VEL, yi);
-    add_fft_xi(P, PH_VOR2VEL, xi);
+    add_fft_inverse(P, PH_VOR2VEL, yi, xi);
     if (fix) add_vor2vel_fixup(P, PH_VOR2VEL, fx);
 }
 
@@ -708,12 +706,11 @@ void build_laplace(epic_member *m)
     FftXArgs x = xargs(m);
     x.mode = 3;
     x.out = m->spec[0];
-    add_fft_xf(m->pl_lap[0], PH_OTHER, {x});
     FftYArgs y = yargs(m);
     y.mode = 0;
     y.in = m->spec[0];
     y.out = m->spec[0];
-    add_fft_y(m->pl_lap[0], PH_OTHER, {y});
+    add_fft_forward(m->pl_lap[0], PH_OTHER, {x}, {y});
     std::vector<FftYArgs> yi;
     std::vector<FftXArgs> xi;
     for (int c = 0; c < 3; ++c) {
@@ -728,8 +725,7 @@ void build_laplace(epic_member *m)
         a.in = m->spec[1 + c];
         xi.push_back(a);
     }
-    add_fft_y(m->pl_lap[1], PH_OTHER, yi);
-    add_fft_xi(m->pl_lap[1], PH_OTHER, xi);
+    add_fft_inverse(m->pl_lap[1], PH_OTHER, yi, xi);
 }
 
 // enqueue a member plan on the member stream (event timers when profiling)

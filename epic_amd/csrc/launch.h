@@ -173,9 +173,14 @@ struct FftYArgs {
     const float2 *in;
     float2 *out;           // may equal in
 };
-void add_fft_xf(Plan &P, int phase, const std::vector<FftXArgs> &items);
-void add_fft_y(Plan &P, int phase, const std::vector<FftYArgs> &items);
-void add_fft_xi(Plan &P, int phase, const std::vector<FftXArgs> &items);
+struct FftPlaneArgs {      // both passes of one component
+    FftXArgs x;
+    FftYArgs y;
+    FastDiv nxh;
+};
+// x and y hold the two passes of each component, item by item
+void add_fft_forward(Plan &P, int phase, const std::vector<FftXArgs> &x, const std::vector<FftYArgs> &y);
+void add_fft_inverse(Plan &P, int phase, const std::vector<FftYArgs> &y, const std::vector<FftXArgs> &x);
 
 // ---- vertical column kernel + fix-ups (inversion.hip) ----
 struct ColArgs {

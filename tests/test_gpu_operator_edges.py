@@ -32,6 +32,8 @@ GRIDS = [
     (16, 32, 30),     # 8 x 2048 cells: the one-launch scan, and one block more
     (16, 32, 32),
     (64, 64, 16),     # 576 work-groups: 256 threads; 2^16 nodes
+    (72, 64, 6),      # about the largest planes of the one-launch transforms
+    (80, 72, 5),      # and beyond them
     (64, 40, 15),     # 360 work-groups: 512 threads
 ]
 
