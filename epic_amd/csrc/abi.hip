@@ -54,7 +54,8 @@ struct epic_member {
     int *keys = nullptr, *cnt[3] = {}, *scnt[3] = {};
     int *cell_start = nullptr, *cursor = nullptr, *perm = nullptr, *bsum = nullptr;
     bool keys_valid = false;
-    int tz_p2g = 2, tz_g2p = 2;     // z chunk of the tile kernels (p2g_default_tz, the autotuner)
+    int tz_p2g = 2, tz_g2p = 2;     // z chunk of the tile kernels (p2g_default_tz, g2p_default_tz, the autotuner)
+    bool tz_chosen = false;         // by the caller or the autotuner
     // fields
     float *fld = nullptr;
     int *nparg = nullptr, *nsparg = nullptr;
@@ -629,7 +630,12 @@ struct StepItem {
 void build_step(Plan &P, const std::vector<StepItem> &items)
 {
     int maxns = 0;
-    for (const StepItem &it : items) maxns = std::max(maxns, it.m->rk_order == 4 ? 5 : 3);
+    int64_t chunks = 0;
+    for (const StepItem &it : items) {
+        maxns = std::max(maxns, it.m->rk_order == 4 ? 5 : 3);
+        chunks += p2g_chunks4(it.m->g);
+    }
+    const int tz_g2p = g2p_default_tz(chunks);
     for (int s = 1; s <= maxns; ++s) {
         Members ms;
         std::vector<const StepItem *> act;
@@ -667,7 +673,7 @@ void build_step(Plan &P, const std::vector<StepItem> &items)
             const double *cb = (m->rk_order == 4) ? CBS4 : CBS3;
             const bool last = (s == ns);
             const int wr = last ? 0 : (s % 3);
-            const P2GLayout L = layout_tz(m->g, m->tz_g2p);
+            const P2GLayout L = layout_tz(m->g, m->tz_chosen ? m->tz_g2p : tz_g2p);
             G2PTileArgs a{};
             a.g = m->g;
             a.p = m->pd;
@@ -879,6 +885,7 @@ int epic_create(const epic_grid_t *grid, const epic_phys_t *phys, const epic_fla
     m->rk_order = flags->rk_order;
     m->cap = std::max<int64_t>(max_parcels, 1);
     m->tz_p2g = p2g_layout(g).tz;
+    m->tz_g2p = g2p_default_tz(p2g_chunks4(g));
     {   // a transform work-group holds ZB lines (or a column) in LDS
         int dev = 0, lds_max = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
@@ -1517,6 +1524,7 @@ int epic_autotune(epic_handle m, int *tz_p2g, int *tz_g2p)
         }
     }
     m->tz_g2p = tg;
+    m->tz_chosen = true;
     m->invalidate_plans();
     if (tz_p2g) *tz_p2g = m->tz_p2g;
     if (tz_g2p) *tz_g2p = m->tz_g2p;
@@ -1533,6 +1541,7 @@ int epic_set_tiling(epic_handle m, int tz_p2g, int tz_g2p)
         return fail(m, EPIC_E_INVALID, "epic_set_tiling: z chunks must be 2, 4 or 8");
     m->tz_p2g = tz_p2g;
     m->tz_g2p = tz_g2p;
+    m->tz_chosen = true;
     m->invalidate_plans();
     return EPIC_OK;
 }

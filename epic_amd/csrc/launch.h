@@ -19,6 +19,7 @@ constexpr int PER_BLOCK = 1024;
 // parcels in fewer rounds.  Push per step at 256, 512, 1024 threads, in us:
 // 36 work-groups (16^3) 270, 193, 158; 117 (24^3) 295, 214, 176; 272 (32^3)
 // 315, 231, 263; 612 (48x48x32) 386, 400, 437; 2112 (64^3) 1027, 1109, 1315.
+// (Chunks of 4 and 8 layers take 128 threads a layer at least.)
 inline int tile_threads(int64_t n) { return n <= 256 ? 1024 : n <= 512 ? 512 : 256; }
 
 // ---- cell sort (p2g.hip) ----
@@ -61,7 +62,15 @@ void launch_cell_order(int64_t nc, const int *cell_start, const int *perm_tmp, c
 // work-groups of 1024 parcels per CU.  Boxes of 7 planes for 4 layers stage
 // 30 % less than of 5 for 2 (par2grid per step: 5.46 -> 5.20 ms at 128^3, 0.94
 // -> 0.90 at 64^3); smaller grids need the work-groups (32^3: 0.42 -> 0.43).
-inline int p2g_default_tz(int ntx, int nty, int nz) { return (int64_t)ntx * nty * ((nz + 5) / 4) >= 1024 ? 4 : 2; }
+inline int64_t p2g_chunks4(const Grid &g) { return (int64_t)((g.nx + P2G_TX - 1) / P2G_TX) * ((g.ny + P2G_TY - 1) / P2G_TY) * ((g.nz + 5) / 4); }
+inline int p2g_default_tz(int64_t chunks4) { return chunks4 >= 1024 ? 4 : 2; }
+// and of the push, for all members of a launch together: a box of 7 planes for
+// 4 layers loads 30 % less than of 5 for 2, where work-groups of 512 parcels
+// still leave two per CU.  At 2 layers (256 threads, four work-groups a CU) and
+// at 4 (512, two), in us a launch: 34.0 and 34.8 at 32^3 (144 chunks of 4), 57.9
+// and 57.5 at 48x48x32 (324), 79.2 and 73.5 at 64x64x32 (576), 158.5 and 146.9
+// at 64^3, 1195 and 1150 at 128^3.
+inline int g2p_default_tz(int64_t chunks4) { return chunks4 >= 512 ? 4 : 2; }
 struct P2GLayout {
     int tz, ntx, nty, nchz;
     int64_t staging_elems;   // FP64 values

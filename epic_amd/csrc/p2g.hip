@@ -1145,7 +1145,7 @@ P2GLayout p2g_layout(const Grid &g)
     // multiple of 8: its cells beyond the grid hold no parcels
     L.ntx = (g.nx + P2G_TX - 1) / P2G_TX;
     L.nty = (g.ny + P2G_TY - 1) / P2G_TY;
-    L.tz = p2g_default_tz(L.ntx, L.nty, g.nz);
+    L.tz = p2g_default_tz(p2g_chunks4(g));
     L.nchz = (g.nz + 2 + L.tz - 1) / L.tz;
     L.staging_elems = (int64_t)L.ntx * L.nty * L.nchz * (L.tz + 3) * P2G_BOX * P2G_BOX * P2G_NF;
     return L;
