@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -38,6 +39,12 @@ constexpr int NSPEC = 15;
 }  // namespace
 
 struct epic_member {
+    static inline std::atomic<int> live{0};   // members of the process
+    epic_member() { ++live; }
+    ~epic_member() { --live; }
+    epic_member(const epic_member &) = delete;
+    epic_member &operator=(const epic_member &) = delete;
+
     Grid g{};
     int rk_order = 4;
     int64_t cap = 0, n = 0;
@@ -184,7 +191,7 @@ template <typename T> hipError_t dalloc(T **p, int64_t count, hipStream_t s)
 {
     *p = nullptr;
     if (count <= 0) count = 1;
-    hipError_t e = hipMalloc((void **)p, sizeof(T) * (size_t)count);
+    hipError_t e = device_malloc((void **)p, sizeof(T) * (size_t)count);
     if (e == hipSuccess) e = hipMemsetAsync(*p, 0, sizeof(T) * (size_t)count, s);
     return e;
 }
@@ -986,6 +993,7 @@ int epic_destroy(epic_handle m)
     if (m->n_h) (void)hipHostFree(m->n_h);
     if (m->s) (void)hipStreamDestroy(m->s);
     delete m;
+    if (epic_member::live == 0) release_staging();
     return EPIC_OK;
 }
 

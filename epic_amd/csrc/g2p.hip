@@ -135,12 +135,13 @@ __global__ __launch_bounds__(256) void k_grid2par(const G2PArgs *__restrict__ ta
 // parcel is loaded one round ahead, and parcel arrays are addressed as a
 // table pointer plus a 32-bit byte offset.
 //
-// What bounds it: HBM traffic (about 380 B a parcel at 4.8 TB/s, a large
-// copy's rate here) together with VALU issue; both only overlap as far as no
-// round waits for memory before its gather.  With the deltas taken into the
-// sums after the gather, constant LDS strides, offsets folded into the
-// accesses and the fields that a step does not change out of the maxima, no
-// register spills and a launch takes 1.20 ms at 128^3 (1.46 before).
+// What bounds it: HBM traffic (367 B a parcel at 4.9 TB/s, a large copy's rate
+// here, in a run that moves parcels by a cell in two steps), as long as no
+// round waits for memory before its gather: the deltas are taken into the sums
+// after the gather, LDS strides are constant, offsets are folded into the
+// accesses, the fields that a step does not change are out of the maxima, and
+// no register is spilled.  A launch at 128^3: 1.46 ms, 1.20 with these, 1.15
+// with chunks of four layers (g2p_default_tz).
 // ---------------------------------------------------------------------------
 size_t g2p_lds_bytes(int tz) { return (3 * sizeof(float4) + sizeof(float2)) * (tz + 3) * P2G_BOX * P2G_BOX; }
 

@@ -25,6 +25,11 @@ hipError_t download_parcels(int64_t n, const int *orig, int *inv, const std::vec
 hipError_t upload_parcels(int64_t n, const int *orig, int *inv, const std::vector<IoGroup> &groups, hipStream_t s);
 hipError_t launch_iota(int64_t n, int *p, hipStream_t s);
 
+// gives the idle staging buffers back
+void release_staging();
+// hipMalloc, tried again without them when memory is short
+hipError_t device_malloc(void **p, size_t bytes);
+
 // ncomp components of 32-bit words to out, (-1:nz+1, -1:ny+1, -1:nx+1[, ncomp])
 template <class In, class Out> hipError_t download_field(const Grid &g, const In *fld, int ncomp, Out *out, hipStream_t s);
 // the interior columns of in (its x and y halos are not read), planes -1..nz+1

@@ -26,8 +26,9 @@ namespace epic {
 namespace {
 
 // ---------------------------------------------------------------------------
-// staging buffers: a process-wide pool, at most POOL_KEEP idle ones kept; a
-// call owns the one it takes, so calls of several threads never share one
+// staging buffers: a process-wide pool, at most POOL_KEEP idle ones kept until
+// the last member goes or memory is short (release_staging); a call owns the
+// one it takes, so calls of several threads never share one
 // ---------------------------------------------------------------------------
 constexpr size_t STAGE_MIN = size_t(1) << 20, STAGE_MAX = size_t(32) << 20, POOL_KEEP = 4;
 
@@ -410,6 +411,25 @@ __global__ __launch_bounds__(256) void k_field_up(Grid g, const float *__restric
 }
 
 }  // namespace
+
+void release_staging()
+{
+    std::vector<Staging *> idle;
+    {
+        std::lock_guard<std::mutex> lk(stage_mu);
+        idle.swap(stage_pool);
+    }
+    for (Staging *b : idle) stage_free(b);
+}
+
+hipError_t device_malloc(void **p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess) return e;
+    (void)hipGetLastError();
+    release_staging();
+    return hipMalloc(p, bytes);
+}
 
 hipError_t download_parcels(int64_t n, const int *orig, int *inv, const std::vector<IoGroup> &groups, hipStream_t s)
 {

@@ -29,6 +29,7 @@
 // These kernels are launched directly (the merge is not part of the step).
 #include "common.h"
 #include "ellipsoid.h"
+#include "hostio.h"
 #include "launch.h"
 
 #include <algorithm>
@@ -638,7 +639,7 @@ int run_merge(const MergeCtx &c, int64_t *n_merge)
             sa.base = nullptr;
             sa.cap = 0;
             const size_t grow = need + need / 4;
-            if (hipMalloc((void **)&sa.base, grow) != hipSuccess) return -1;
+            if (device_malloc((void **)&sa.base, grow) != hipSuccess) return -1;
             sa.cap = grow;
         }
     }
@@ -652,7 +653,7 @@ int run_merge(const MergeCtx &c, int64_t *n_merge)
             return hipSuccess;
         }
         used += b;   // counted for the next call's arena
-        hipError_t e = hipMalloc(ptr, b);
+        hipError_t e = device_malloc(ptr, b);
         if (e == hipSuccess) owned.push_back(*ptr);
         return e;
     };
