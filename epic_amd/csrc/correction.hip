@@ -23,68 +23,134 @@ __device__ inline int64_t gtid() { return blockIdx.x * (int64_t)blockDim.x + thr
 inline unsigned nblk(int64_t n) { return (unsigned)std::max<int64_t>(1, (n + 255) / 256); }
 }  // namespace
 
-// one thread per (kx, ky) column; in: phi spectrum; fr, fi, et: FP64
-// scratch of (nz+1) ncol entries each, plane-major so that neighbouring
-// columns touch neighbouring words; out: the x, y, z gradient spectra
-__global__ void k_lapinv_columns(Grid g, const float2 *in, double *fr, double *fi, double *et, float2 *ox, float2 *oy,
-                                 float2 *oz)
+// the horizontal wavenumbers of column (kx, ky)
+struct LapColumn {
+    double ikx, iky, k2l2;
+    bool zero;
+};
+__device__ inline LapColumn lap_column(const Grid &g, int64_t col)
 {
-    const int64_t col = gtid();
-    const int ncol = g.ny * g.nxh;
-    if (col >= ncol) return;
     const int kx = (int)(col % g.nxh), ky = (int)(col / g.nxh);
-    const int nz = g.nz;
-    const int64_t base = col * (int64_t)g.nzp;
-    if (kx == 0 && ky == 0) {
-        for (int z = 0; z <= nz; ++z) ox[base + z] = oy[base + z] = oz[base + z] = float2{0.0f, 0.0f};
-        return;
-    }
     const int kys = (2 * ky <= g.ny) ? ky : ky - g.ny;
     const double rkx = 2.0 * 3.14159265358979323846 * kx / g.extent[0];
     const double rky = 2.0 * 3.14159265358979323846 * kys / g.extent[1];
-    const double ikx = (2 * kx == g.nx) ? 0.0 : rkx;     // diffx: zero at the x Nyquist
-    const double iky = (2 * ky == g.ny) ? 0.0 : rky;     // diffy: zero at the y Nyquist
-    const double k2l2 = rkx * rkx + rky * rky;
+    LapColumn c;
+    c.ikx = (2 * kx == g.nx) ? 0.0 : rkx;     // diffx: zero at the x Nyquist
+    c.iky = (2 * ky == g.ny) ? 0.0 : rky;     // diffy: zero at the y Nyquist
+    c.k2l2 = rkx * rkx + rky * rky;
+    c.zero = kx == 0 && ky == 0;
+    return c;
+}
+
+// the tridiagonal solve of one column with right side rhs(z), the solution in
+// fr, fi (S apart from plane to plane); et: scratch
+template <class Rhs>
+__device__ inline void lap_solve(const Grid &g, double k2l2, double *fr, double *fi, double *et, int64_t S, const Rhs &rhs)
+{
+    const int nz = g.nz;
     const double dzisq = g.dxi[2] * g.dxi[2], ap = dzisq;
     const double a0 = -2.0 * dzisq - k2l2;
-    fr += col;
-    fi += col;
-    et += col;
-    const int64_t S = ncol;   // plane stride of the scratch
     // forward elimination (htdv / etdv on the fly)
     double h = 1.0 / a0;
     double e = -2.0 * ap * h;
-    float2 r = in[base];
-    fr[0] = (double)r.x * h;
-    fi[0] = (double)r.y * h;
+    double2 r = rhs(0);
+    fr[0] = r.x * h;
+    fi[0] = r.y * h;
     et[0] = e;
     for (int z = 1; z <= nz - 1; ++z) {
         h = 1.0 / (a0 + ap * e);
-        r = in[base + z];
-        fr[z * S] = ((double)r.x - ap * fr[(z - 1) * S]) * h;
-        fi[z * S] = ((double)r.y - ap * fi[(z - 1) * S]) * h;
+        r = rhs(z);
+        fr[z * S] = (r.x - ap * fr[(z - 1) * S]) * h;
+        fi[z * S] = (r.y - ap * fi[(z - 1) * S]) * h;
         e = -ap * h;
         et[z * S] = e;
     }
     h = 1.0 / (a0 + 2.0 * ap * e);
-    r = in[base + nz];
-    fr[nz * S] = ((double)r.x - 2.0 * ap * fr[(nz - 1) * S]) * h;
-    fi[nz * S] = ((double)r.y - 2.0 * ap * fi[(nz - 1) * S]) * h;
+    r = rhs(nz);
+    fr[nz * S] = (r.x - 2.0 * ap * fr[(nz - 1) * S]) * h;
+    fi[nz * S] = (r.y - 2.0 * ap * fi[(nz - 1) * S]) * h;
     // back substitution
     for (int z = nz - 1; z >= 0; --z) {
         fr[z * S] = et[z * S] * fr[(z + 1) * S] + fr[z * S];
         fi[z * S] = et[z * S] * fi[(z + 1) * S] + fi[z * S];
     }
-    // gradient spectra: i kx f, i ky f, central z differences (0 at the walls)
+}
+
+// gradient spectra at plane z: i kx f, i ky f, central z differences (0 at the walls)
+__device__ inline void lap_gradient(const Grid &g, const LapColumn &c, const double *fr, const double *fi, int z, int64_t S,
+                                    float2 &x, float2 &y, float2 &d)
+{
     const double hdzi = 0.5 * g.dxi[2];
-    for (int z = 0; z <= nz; ++z) {
-        ox[base + z] = float2{(float)(-ikx * fi[z * S]), (float)(ikx * fr[z * S])};
-        oy[base + z] = float2{(float)(-iky * fi[z * S]), (float)(iky * fr[z * S])};
-        if (z == 0 || z == nz) oz[base + z] = float2{0.0f, 0.0f};
-        else
-            oz[base + z] = float2{(float)((fr[(z + 1) * S] - fr[(z - 1) * S]) * hdzi),
-                                  (float)((fi[(z + 1) * S] - fi[(z - 1) * S]) * hdzi)};
+    x = float2{(float)(-c.ikx * fi[z * S]), (float)(c.ikx * fr[z * S])};
+    y = float2{(float)(-c.iky * fi[z * S]), (float)(c.iky * fr[z * S])};
+    if (z == 0 || z == g.nz) d = float2{0.0f, 0.0f};
+    else
+        d = float2{(float)((fr[(z + 1) * S] - fr[(z - 1) * S]) * hdzi), (float)((fi[(z + 1) * S] - fi[(z - 1) * S]) * hdzi)};
+}
+
+// in: phi spectrum; out: the x, y, z gradient spectra.  A block takes LAP_COLS
+// (kx, ky) columns in LDS: all its threads load them and form the gradients in
+// whole lines, one thread per column runs the two recurrences, a chain of nz
+// divisions.  With a thread per column throughout and the recurrences in global
+// memory (the form below, kept for columns beyond LDS) it was bound by that
+// memory's latency on 5 work-groups: 63 us at 48x48x32, 11.5 here
+// (apply_laplace 239 -> 191 us, 460 -> 329 at 64^3).
+constexpr int LAP_COLS = 16, LAP_PITCH = LAP_COLS + 1;   // (a pitch of 17: no bank conflicts along z)
+static size_t lap_lds(const Grid &g) { return 3 * sizeof(double) * LAP_PITCH * (size_t)(g.nz + 1); }
+__global__ __launch_bounds__(256) void k_lapinv_columns(Grid g, const float2 *in, float2 *ox, float2 *oy, float2 *oz)
+{
+    extern __shared__ double lap[];
+    const int nz1 = g.nz + 1, total = LAP_COLS * nz1;
+    double *fr = lap, *fi = fr + LAP_PITCH * nz1, *et = fi + LAP_PITCH * nz1;
+    const int64_t col0 = blockIdx.x * (int64_t)LAP_COLS, ncol = (int64_t)g.ny * g.nxh;
+    for (int t = threadIdx.x; t < total; t += 256) {
+        const int c = t / nz1, z = t - c * nz1;
+        if (col0 + c >= ncol) break;
+        const float2 r = in[(col0 + c) * g.nzp + z];
+        fr[z * LAP_PITCH + c] = (double)r.x;
+        fi[z * LAP_PITCH + c] = (double)r.y;
     }
+    __syncthreads();
+    if (threadIdx.x < LAP_COLS && col0 + threadIdx.x < ncol) {
+        const LapColumn c = lap_column(g, col0 + threadIdx.x);
+        double *r = fr + threadIdx.x, *i = fi + threadIdx.x;
+        if (!c.zero) lap_solve(g, c.k2l2, r, i, et + threadIdx.x, LAP_PITCH, [&](int z) { return double2{r[z * LAP_PITCH], i[z * LAP_PITCH]}; });
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < total; t += 256) {
+        const int c = t / nz1, z = t - c * nz1;
+        if (col0 + c >= ncol) break;
+        const LapColumn k = lap_column(g, col0 + c);
+        float2 x = float2{0.0f, 0.0f}, y = x, d = x;
+        if (!k.zero) lap_gradient(g, k, fr + c, fi + c, z, LAP_PITCH, x, y, d);
+        const int64_t o = (col0 + c) * g.nzp + z;
+        ox[o] = x;
+        oy[o] = y;
+        oz[o] = d;
+    }
+}
+
+// one thread per column; fr, fi, et: FP64 scratch of (nz+1) ncol entries each,
+// plane-major so that neighbouring columns touch neighbouring words
+__global__ void k_lapinv_columns_long(Grid g, const float2 *in, double *fr, double *fi, double *et, float2 *ox, float2 *oy,
+                                      float2 *oz)
+{
+    const int64_t col = gtid(), ncol = (int64_t)g.ny * g.nxh;
+    if (col >= ncol) return;
+    const int64_t base = col * (int64_t)g.nzp;
+    const LapColumn c = lap_column(g, col);
+    if (c.zero) {
+        for (int z = 0; z <= g.nz; ++z) ox[base + z] = oy[base + z] = oz[base + z] = float2{0.0f, 0.0f};
+        return;
+    }
+    fr += col;
+    fi += col;
+    et += col;
+    lap_solve(g, c.k2l2, fr, fi, et, ncol, [&](int z) {
+        const float2 r = in[base + z];
+        return double2{(double)r.x, (double)r.y};
+    });
+    for (int z = 0; z <= g.nz; ++z) lap_gradient(g, c, fr, fi, z, ncol, ox[base + z], oy[base + z], oz[base + z]);
 }
 
 // z halo of the gradient fields: linear extrapolation
@@ -268,8 +334,12 @@ __global__ void k_vortcor(ParcelsDev p, double d0, double d1, double d2)
 void launch_lapinv_columns(const Grid &g, const float2 *in, double *fr, double *fi, double *et, float2 *ox, float2 *oy,
                            float2 *oz, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_lapinv_columns, dim3(nblk((int64_t)g.ny * g.nxh)), dim3(256), 0, s, g, in, fr, fi, et, ox, oy,
-                       oz);
+    const int64_t ncol = (int64_t)g.ny * g.nxh;
+    if (lap_lds(g) <= (160 << 10))
+        hipLaunchKernelGGL(k_lapinv_columns, dim3((unsigned)((ncol + LAP_COLS - 1) / LAP_COLS)), dim3(256), lap_lds(g), s, g, in, ox,
+                           oy, oz);
+    else
+        hipLaunchKernelGGL(k_lapinv_columns_long, dim3(nblk(ncol)), dim3(256), 0, s, g, in, fr, fi, et, ox, oy, oz);
 }
 void launch_grad_halo(const Grid &g, float *fld, hipStream_t s)
 {

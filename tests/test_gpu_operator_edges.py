@@ -80,3 +80,22 @@ def test_stage_operators(grid):
     assert np.abs(p["position"] - st.position).max() <= TOL * max(mem.dx)
     for k in ("vorticity", "B"):
         assert maxrel(p[k], getattr(st, k)) <= TOL, k
+
+
+# the longest columns that the vertical solve of the Laplace correction keeps in
+# LDS, the next length, and a last block of columns that is not full
+@pytest.mark.parametrize("grid", [(8, 8, 400), (8, 8, 405), (20, 18, 10)], ids=lambda g: "x".join(map(str, g)))
+def test_laplace_columns(grid):
+    nx, ny, nz = grid
+    print(f"laplace columns: {grid}", flush=True)
+    mem = W.rising_thermal(nx, seed=5 + nz, ny=ny, nz=nz)
+    s = (1.0 + 0.3 * np.random.default_rng(nz).uniform(-1.0, 1.0, mem.n)).astype(np.float32).astype(np.float64)
+    mem.volume = (mem.volume * s).astype(np.float32).astype(np.float64)
+    mem.B = (mem.B * s[:, None] ** (2.0 / 3.0)).astype(np.float32).astype(np.float64)
+    st, gm = oracle_state(mem), Member.from_workload(mem)
+    st.apply_laplace()
+    gm.apply_laplace()
+    d = [p - mem.position for p in (st.position, gm.get_parcels()["position"])]
+    for v in d:
+        v[:, :2] -= np.asarray(mem.extent)[:2] * np.round(v[:, :2] / np.asarray(mem.extent)[:2])
+    assert np.abs(d[1] - d[0]).max() <= TOL * np.abs(d[0]).max()
