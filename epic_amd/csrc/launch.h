@@ -65,12 +65,13 @@ void launch_cell_order(int64_t nc, const int *cell_start, const int *perm_tmp, c
 inline int64_t p2g_chunks4(const Grid &g) { return (int64_t)((g.nx + P2G_TX - 1) / P2G_TX) * ((g.ny + P2G_TY - 1) / P2G_TY) * ((g.nz + 5) / 4); }
 inline int p2g_default_tz(int64_t chunks4) { return chunks4 >= 1024 ? 4 : 2; }
 // and of the push, for all members of a launch together: a box of 7 planes for
-// 4 layers loads 30 % less than of 5 for 2, where work-groups of 512 parcels
-// still leave two per CU.  At 2 layers (256 threads, four work-groups a CU) and
-// at 4 (512, two), in us a launch: 34.0 and 34.8 at 32^3 (144 chunks of 4), 57.9
-// and 57.5 at 48x48x32 (324), 79.2 and 73.5 at 64x64x32 (576), 158.5 and 146.9
-// at 64^3, 1195 and 1150 at 128^3.
-inline int g2p_default_tz(int64_t chunks4) { return chunks4 >= 512 ? 4 : 2; }
+// 4 layers loads 30 % less than of 5 for 2, unless that leaves CUs without a
+// work-group.  At 2 layers and at 4 (512 threads, 1024 up to 256 work-groups),
+// in us a launch: 34.0 and 34.8 at 32^3 (144 chunks of 4), 32.8 and 34.3 at
+// 40x36x20 (150), 40.1 and 36.8 at 40x40x24 (175), 42.5 and 39.5 at 48x48x24
+// (252), 55.2 and 50.8 at 32x64x32 (288), 65.7 and 65.8 at 64x48x32 (432), 79.2
+// and 73.5 at 64x64x32 (576), 158.5 and 146.9 at 64^3, 1195 and 1150 at 128^3.
+inline int g2p_default_tz(int64_t chunks4) { return chunks4 >= 160 ? 4 : 2; }
 struct P2GLayout {
     int tz, ntx, nty, nchz;
     int64_t staging_elems;   // FP64 values

@@ -34,7 +34,9 @@ GRIDS = [
     (64, 64, 16),     # 576 work-groups: 256 threads; 2^16 nodes
     (72, 64, 6),      # about the largest planes of the one-launch transforms
     (80, 72, 5),      # and beyond them
-    (64, 64, 27),     # 512 chunks of four layers: the push takes those
+    (40, 40, 18),     # 125 chunks of four layers: the push takes two, of 1024 threads
+    (64, 40, 12),     # 160: it takes four
+    (64, 64, 27),     # 512, of 512 threads
     (64, 40, 15),     # 360 work-groups: 512 threads
 ]
 
