@@ -460,6 +460,7 @@ struct P2GSel {
     bool max_from_push = false;   // the previous push and stages left the fixed-point maxima: no k_p2g_max
     bool max_done = false;        // k_axes_max has taken them
     bool push_next = false;       // a push that fills the vorticity's maxima follows: the others stay
+    int tz = 0;                   // the tile scatter's z chunk (0: the member's own)
 };
 
 void build_p2g(Plan &P, const Members &ms, const std::vector<P2GSel> &sel)
@@ -475,7 +476,7 @@ void build_p2g(Plan &P, const Members &ms, const std::vector<P2GSel> &sel)
         sc.push_back(ScanArgs{m->cnt[q.rd], nc, m->cell_start, m->bsum, m->cursor, m->far_flag, m->far_acc,
                               (int64_t)P2G_NF * field_stride(m->g)});
         pl.push_back(PlaceArgs{m->n, m->keys, m->cell_start, m->cursor, m->perm, m->cap, m->n_dev, m->far_flag});
-        const P2GLayout L = layout_tz(m->g, m->tz_p2g);
+        const P2GLayout L = layout_tz(m->g, q.tz ? q.tz : m->tz_p2g);
         P2GArgs a{};
         a.g = m->g;
         a.p = m->pd;
@@ -637,8 +638,14 @@ struct StepItem {
 void build_step(Plan &P, const std::vector<StepItem> &items)
 {
     int maxns = 0;
+    // members whose tiling nobody chose share one launch of each tile kernel: of
+    // the scatter with the smallest one's chunk (an ensemble of eight, one of
+    // which takes 4 layers alone: 4.89 ms a step with 2 for all, 4.96 in two
+    // launches), of the push with the chunk of all of them together
     int64_t chunks = 0;
+    int tz_p2g = 8;
     for (const StepItem &it : items) {
+        if (!it.m->tz_chosen) tz_p2g = std::min(tz_p2g, it.m->tz_p2g);
         maxns = std::max(maxns, it.m->rk_order == 4 ? 5 : 3);
         chunks += p2g_chunks4(it.m->g);
     }
@@ -660,7 +667,8 @@ void build_step(Plan &P, const std::vector<StepItem> &items)
             float *const *a = last ? m->ax_stale : m->ax_cur;
             ax.push_back(a);
             const int rd = (s - 1) % 3, wr = last ? 0 : (s % 3);
-            sel.push_back(P2GSel{a, m->ax_stale, s == 1 ? &it->tm->reuse : nullptr, rd, wr, s > 1, s == 1, !last});
+            sel.push_back(P2GSel{a, m->ax_stale, s == 1 ? &it->tm->reuse : nullptr, rd, wr, s > 1, s == 1, !last,
+                                 m->tz_chosen ? 0 : tz_p2g});
         }
         if (s == 1) build_axes(P, ms, ax, true);   // later stages: stored by the previous push
         build_p2g(P, ms, sel);

@@ -16,11 +16,13 @@ constexpr int PER_BLOCK = 1024;
 // Threads of a tile kernel's work-group (about 1024 parcels at tz = 2) in a
 // launch of n of them.  Four 256-thread work-groups fill a CU and overlap
 // their phases; while there are fewer than that, larger ones take a tile's
-// parcels in fewer rounds.  Push per step at 256, 512, 1024 threads, in us:
-// 36 work-groups (16^3) 270, 193, 158; 117 (24^3) 295, 214, 176; 272 (32^3)
-// 315, 231, 263; 612 (48x48x32) 386, 400, 437; 2112 (64^3) 1027, 1109, 1315.
-// (Chunks of 4 and 8 layers take 128 threads a layer at least.)
-inline int tile_threads(int64_t n) { return n <= 256 ? 1024 : n <= 512 ? 512 : 256; }
+// parcels in fewer rounds.  Tile scatter at 256, 512, 1024 threads, in us a
+// launch: 36 work-groups (16^3) 22.6, 16.6, 15.4; 272 (32^3) 27.8, 20.1, 24.2;
+// 612 (48x48x32) 41.9, 39.6, 47.2; 1088 (64x64x32) 54.2, 53.5, 71.2; 16640
+// (128^3) 697, 731, 1079.  Push per step at 36: 270, 193, 158; 117 (24^3) 295,
+// 214, 176; 272: 315, 231, 263.  (Chunks of 4 and 8 layers take 128 threads a
+// layer at least.)
+inline int tile_threads(int64_t n) { return n <= 256 ? 1024 : n <= 1024 ? 512 : 256; }
 
 // ---- cell sort (p2g.hip) ----
 struct KeysArgs {
@@ -58,12 +60,13 @@ void launch_cell_order(int64_t nc, const int *cell_start, const int *perm_tmp, c
                        hipStream_t s);
 
 // ---- support-point half axes + par2grid (p2g.hip) ----
-// default z chunk of the tile scatter: 4 layers where that still leaves four
-// work-groups of 1024 parcels per CU.  Boxes of 7 planes for 4 layers stage
-// 30 % less than of 5 for 2 (par2grid per step: 5.46 -> 5.20 ms at 128^3, 0.94
-// -> 0.90 at 64^3); smaller grids need the work-groups (32^3: 0.42 -> 0.43).
+// default z chunk of the tile scatter: 4 layers where that still leaves two
+// work-groups of 512 threads per CU.  Boxes of 7 planes for 4 layers stage 30 %
+// less than of 5 for 2.  Tiles + finalize at 2 and 4 layers, in us a launch: 52.9
+// and 57.1 at 48x48x32 (324 chunks of 4), 67.9 and 64.7 at 64x64x32 (576), 118 and
+// 113 at 64^3, 830 and 787 at 128^3.
 inline int64_t p2g_chunks4(const Grid &g) { return (int64_t)((g.nx + P2G_TX - 1) / P2G_TX) * ((g.ny + P2G_TY - 1) / P2G_TY) * ((g.nz + 5) / 4); }
-inline int p2g_default_tz(int64_t chunks4) { return chunks4 >= 1024 ? 4 : 2; }
+inline int p2g_default_tz(int64_t chunks4) { return chunks4 >= 512 ? 4 : 2; }
 // and of the push, for all members of a launch together: a box of 7 planes for
 // 4 layers loads 30 % less than of 5 for 2, unless that leaves CUs without a
 // work-group.  At 2 layers and at 4 (512 threads, 1024 up to 256 work-groups),

@@ -31,12 +31,12 @@ GRIDS = [
     (8, 128, 6),
     (16, 32, 30),     # 8 x 2048 cells: the one-launch scan, and one block more
     (16, 32, 32),
-    (64, 64, 16),     # 576 work-groups: 256 threads; 2^16 nodes
+    (64, 64, 16),     # 576 work-groups: 512 threads; 2^16 nodes
     (72, 64, 6),      # about the largest planes of the one-launch transforms
     (80, 72, 5),      # and beyond them
     (40, 40, 18),     # 125 chunks of four layers: the push takes two, of 1024 threads
     (64, 40, 12),     # 160: it takes four
-    (64, 64, 27),     # 512, of 512 threads
+    (64, 64, 27),     # 512, and the tile scatter takes four too
     (64, 40, 15),     # 360 work-groups: 512 threads
 ]
 
