@@ -460,7 +460,7 @@ def main():
                                "replayed step graph on the member's stream" +
                                (" (eager launches between HIP events)" if args.eager else "") +
                                "; traffic from rocprofv3 counters (" + os.path.relpath(TRAFFIC_SUMMARY, ROOT) + ")")
-        roof["limiter"] = "memory latency and VALU issue (per-kernel counters in the profiles), below the HBM bound"
+        roof["limiter"] = "HBM traffic at a large copy's rate, more bytes than the algorithmic ones (per-kernel counters in the profiles)"
     if args.copy_calibration:
         device_copy_calibration()
     line = {
