@@ -803,9 +803,10 @@ __global__ __launch_bounds__(1024, 4) void k_p2g_tiles(const P2GArgs *__restrict
 // ---------------------------------------------------------------------------
 // tile d = -1, 0, 1 beside the one of node i (of n >= P2G_BOX nodes in nt >= 2
 // tiles of 8, the last one shorter when n is not a multiple of 8): its number t
-// and the node's place l in its box; false when the box does not hold the node.
+// and the node's place l in its box; false when it holds nothing for the node.
 // No box of such a row meets itself, and of two tiles one is beside the other
-// once.
+// once.  Beyond a last tile of one node, node 0 is also the last place of the
+// box of the tile before it (d = 1, where node 0 has no other).
 __device__ inline bool box_place(int d, int i, int n, int nt, int &t, int &l)
 {
     const int own = i >> 3, r = i & 7;
@@ -829,7 +830,10 @@ __device__ inline bool box_place(int d, int i, int n, int nt, int &t, int &l)
         }
     } else if (d > 0) {
         l = 0;
-        if (i == n - 1) t = 0;
+        if (i == 0 && n == 8 * (nt - 1) + 1) {
+            t = nt - 2;
+            l = P2G_BOX - 1;
+        } else if (i == n - 1) t = 0;
         else if (r != 7) return false;
     }
     return true;
@@ -907,15 +911,18 @@ __device__ inline void stage_add(const FinalizeArgs &a, int i, int j, int k, dou
         return;
     }
     const int txa = i / P2G_TX, tya = j / P2G_TY;
+    // (nx is even: only along y can a last tile have one node, and the box of
+    // the tile before it reach node 0)
+    const bool beyond = a.nty > 3 && j == 0 && g.ny == P2G_TY * (a.nty - 1) + 1;
     for (int dcz = -1; dcz <= 1; ++dcz) {
         const int cz = cza + dcz;
         if (cz < 0 || cz >= a.nchz) continue;
         const int lp = k - (cz * a.tz - 2);   // box plane index
         if (lp < 0 || lp >= nbox) continue;
-            for (int dty = -1; dty <= 1; ++dty) {
+        for (int dty = -1; dty <= (beyond ? 2 : 1); ++dty) {
             // distinct candidate tiles only (grids of one or two tiles wrap)
             if ((a.nty == 1 && dty != 0) || (a.nty == 2 && dty == 1)) continue;
-            const int ty = wrap(tya + dty, a.nty);
+            const int ty = dty == 2 ? a.nty - 2 : wrap(tya + dty, a.nty);
             for (int ly = wrap(j - (ty * P2G_TY - 1), g.ny); ly < P2G_BOX; ly += g.ny) {
                 for (int dtx = -1; dtx <= 1; ++dtx) {
                     if ((a.ntx == 1 && dtx != 0) || (a.ntx == 2 && dtx == 1)) continue;
