@@ -635,6 +635,10 @@ struct StepItem {
     bool adaptive;
 };
 
+// the humidity bounds the condensate: the later stages of a step need no pass
+// over the parcels for par2grid's scales
+bool p2g_bounded(const epic_member *m) { return m->g.q0 >= 0.0; }
+
 void build_step(Plan &P, const std::vector<StepItem> &items)
 {
     int maxns = 0;
@@ -667,8 +671,9 @@ void build_step(Plan &P, const std::vector<StepItem> &items)
             float *const *a = last ? m->ax_stale : m->ax_cur;
             ax.push_back(a);
             const int rd = (s - 1) % 3, wr = last ? 0 : (s % 3);
-            sel.push_back(P2GSel{a, m->ax_stale, s == 1 ? &it->tm->reuse : nullptr, rd, wr, s > 1, s == 1, !last,
-                                 m->tz_chosen ? 0 : tz_p2g});
+            const bool bounded = p2g_bounded(m);
+            sel.push_back(P2GSel{a, m->ax_stale, s == 1 ? &it->tm->reuse : nullptr, rd, wr, s > 1 && bounded, s == 1,
+                                 !last && bounded, m->tz_chosen ? 0 : tz_p2g});
         }
         if (s == 1) build_axes(P, ms, ax, true);   // later stages: stored by the previous push
         build_p2g(P, ms, sel);
@@ -695,7 +700,8 @@ void build_step(Plan &P, const std::vector<StepItem> &items)
             for (int c = 0; c < 6; ++c) a.axes[c] = ax[i][c];
             if (!last) {
                 for (int c = 0; c < 6; ++c) a.axes_next[c] = (s + 1 == ns) ? m->ax_stale[c] : m->ax_cur[c];
-                a.tmax_next = m->pmax_out;   // its vorticity entries cleared by this stage's finalize
+                // its vorticity entries cleared by this stage's finalize
+                a.tmax_next = p2g_bounded(m) ? m->pmax_out : nullptr;
             }
             a.perm = m->perm;
             a.cell_start = m->cell_start;

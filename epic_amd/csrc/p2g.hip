@@ -404,11 +404,13 @@ __device__ inline void p2g_values(const Grid &g, const ParcelsDev &p, unsigned o
 // runs this pass: volume, buoyancy and humidity do not change in a step, so
 // their maxima stay for the later stages, the vorticity maxima come from the
 // previous push, and the moist contributions, which follow the height, are
-// bounded by the humidity: the condensate is at most the humidity, so |tbuoy|
-// <= |buoy| + glat hum and |tbuoy - buoy| <= glat hum (exact when there is no
-// humidity; P2G_MAX_BOUND onwards).  A scale from a bound is at most one power
-// of two coarser, and the fixed-point sums keep a factor 2 of headroom for
-// rounding.
+// bounded by the humidity: the condensate is at most the humidity (q0 >= 0;
+// otherwise every stage runs this pass), so |tbuoy| <= |buoy| + glat hum and
+// |tbuoy - buoy| <= glat hum (P2G_MAX_BOUND onwards; exact where there is no
+// humidity).  A contribution at its maximum fills the 32 bits of a quad's sum,
+// so the first bound is raised by 2^-20: its roundings and those of the
+// contribution are at most seven, of 2^-24 each.  A scale from a bound is at
+// most one power of two coarser.
 __device__ inline void take_maxima(const Grid &g, const ParcelsDev &p, int64_t q, float mx[P2G_MAXIMA])
 {
     float v[P2G_NF];
@@ -416,8 +418,8 @@ __device__ inline void take_maxima(const Grid &g, const ParcelsDev &p, int64_t q
 #pragma unroll
     for (int f = 0; f < P2G_NF; ++f) mx[f] = fmaxf(mx[f], fabsf(v[f]));
     mx[P2G_NF] = fmaxf(mx[P2G_NF], fabsf(v[4] - v[5]));
-    const float hb = fabsf(v[0] * (float)g.glat * at(p.hum, (unsigned)q * 4u));
-    mx[P2G_MAX_BOUND] = fmaxf(mx[P2G_MAX_BOUND], fabsf(v[5]) + hb);
+    const float hum = at(p.hum, (unsigned)q * 4u), hb = fabsf(v[0] * (float)g.glat * hum), b = fabsf(v[5]) + hb;
+    mx[P2G_MAX_BOUND] = fmaxf(mx[P2G_MAX_BOUND], hum != 0.0f ? b * (1.0f + 0x1p-20f) : b);
     mx[P2G_MAX_BOUND + 1] = fmaxf(mx[P2G_MAX_BOUND + 1], hb);
 }
 // the block's maxima to out[] (256 threads).  A block whose maximum is not
