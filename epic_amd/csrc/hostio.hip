@@ -20,6 +20,7 @@
 #include <mutex>
 #include <system_error>
 #include <thread>
+#include <tuple>
 
 namespace epic {
 
@@ -284,7 +285,20 @@ __global__ __launch_bounds__(256) void k_parcel_io(IoArrays a, const int *__rest
     }
 }
 
-int blocks_of(int64_t n) { return (int)((n + 255) / 256); }
+int64_t blocks_of(int64_t n) { return (n + 255) / 256; }
+
+// a launch with its own status: the thread's last-error slot, which may hold an
+// earlier call's error, is neither read nor cleared
+template <class... P, class... A> hipError_t launch(void (*kernel)(P...), int64_t blocks, hipStream_t s, A... a)
+{
+    std::tuple<P...> v{a...};
+    return std::apply(
+        [&](P &...p) {
+            void *args[] = {(void *)&p...};
+            return hipLaunchKernel((const void *)kernel, dim3((unsigned)blocks), dim3(256), args, 0, s);
+        },
+        v);
+}
 
 hipError_t parcel_io(bool up, int64_t n, const int *orig, int *inv, std::vector<IoGroup> groups, hipStream_t s)
 {
@@ -308,10 +322,7 @@ hipError_t parcel_io(bool up, int64_t n, const int *orig, int *inv, std::vector<
     if (e != hipSuccess) return e;
     const int64_t ch = std::min<int64_t>(n, (int64_t)b->size / per & ~int64_t(1));   // even: FP64 groups stay aligned
     const int64_t nch = (n + ch - 1) / ch;
-    if (orig) {
-        hipLaunchKernelGGL(k_inverse, dim3(blocks_of(n)), dim3(256), 0, s, n, orig, inv);
-        e = hipGetLastError();
-    }
+    if (orig) e = launch(k_inverse, blocks_of(n), s, n, orig, inv);
     {
         Team team(std::min(n, ch) * values);
         auto part = [&](int64_t m, int t, int nt, int64_t &lo, int64_t &hi) {
@@ -350,8 +361,7 @@ hipError_t parcel_io(bool up, int64_t n, const int *orig, int *inv, std::vector<
                 b, nch, s,
                 [&](int64_t c, char *dev, char *pin) {
                     const int64_t m = chunk(c);
-                    hipLaunchKernelGGL(k_parcel_io<false>, dim3(blocks_of(m)), dim3(256), 0, s, a, map, c * ch, m, dev);
-                    const hipError_t le = hipGetLastError();
+                    const hipError_t le = launch(k_parcel_io<false>, blocks_of(m), s, a, map, c * ch, m, dev);
                     return le != hipSuccess ? le : hipMemcpyAsync(pin, dev, (size_t)(m * per), hipMemcpyDeviceToHost, s);
                 },
                 convert);
@@ -360,8 +370,7 @@ hipError_t parcel_io(bool up, int64_t n, const int *orig, int *inv, std::vector<
                 const int64_t m = chunk(c);
                 const hipError_t le = hipMemcpyAsync(dev, pin, (size_t)(m * per), hipMemcpyHostToDevice, s);
                 if (le != hipSuccess) return le;
-                hipLaunchKernelGGL(k_parcel_io<true>, dim3(blocks_of(m)), dim3(256), 0, s, a, map, c * ch, m, dev);
-                return hipGetLastError();
+                return launch(k_parcel_io<true>, blocks_of(m), s, a, map, c * ch, m, dev);
             });
     }
     stage_put(b);
@@ -443,8 +452,7 @@ hipError_t upload_parcels(int64_t n, const int *orig, int *inv, const std::vecto
 
 hipError_t launch_iota(int64_t n, int *p, hipStream_t s)
 {
-    if (n > 0) hipLaunchKernelGGL(k_iota, dim3(blocks_of(n)), dim3(256), 0, s, n, p);
-    return hipGetLastError();
+    return n > 0 ? launch(k_iota, blocks_of(n), s, n, p) : hipSuccess;
 }
 
 template <class In, class Out>
@@ -466,9 +474,7 @@ hipError_t download_field(const Grid &g, const In *fld, int ncomp, Out *out, hip
             b, nch, s,
             [&](int64_t c, char *dev, char *pin) {
                 const int u0 = (int)c * uch, u1 = std::min(nu, u0 + uch);
-                hipLaunchKernelGGL(k_field_down, dim3((unsigned)((int64_t)(u1 - u0) * hy * nzb)), dim3(256), 0, s, g,
-                                   (const int *)fld, u0, nzb, (int *)dev);
-                const hipError_t le = hipGetLastError();
+                const hipError_t le = launch(k_field_down, (int64_t)(u1 - u0) * hy * nzb, s, g, (const int *)fld, u0, nzb, (int *)dev);
                 return le != hipSuccess ? le : hipMemcpyAsync(pin, dev, (size_t)(4 * (col(u1) - col(u0)) * line), hipMemcpyDeviceToHost, s);
             },
             [&](int64_t c, char *pin) {
@@ -517,9 +523,7 @@ hipError_t upload_field(const Grid &g, float *fld, int ncomp, const double *in, 
                 const int x0 = (int)(c % per) * xch, nxs = std::min(xch, g.nx - x0);
                 const hipError_t le = hipMemcpyAsync(dev, pin, (size_t)(4 * nxs * line), hipMemcpyHostToDevice, s);
                 if (le != hipSuccess) return le;
-                hipLaunchKernelGGL(k_field_up, dim3(blocks_of((int64_t)nxs * line)), dim3(256), 0, s, g, (const float *)dev, x0,
-                                   nxs, fld + (c / per) * FS);
-                return hipGetLastError();
+                return launch(k_field_up, blocks_of((int64_t)nxs * line), s, g, (const float *)dev, x0, nxs, fld + (c / per) * FS);
             });
     }
     stage_put(b);
