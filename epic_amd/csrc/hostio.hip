@@ -36,7 +36,7 @@ constexpr size_t STAGE_MIN = size_t(1) << 20, STAGE_MAX = size_t(32) << 20, POOL
 struct Staging {
     size_t size = 0;   // bytes of each of the two buffers
     int device = 0;
-    char *pin[2] = {}, *dev[2] = {};
+    char *pin[2] = {}, *map[2] = {}, *dev[2] = {};   // pinned, its address on the device, device memory
     hipEvent_t ev[2] = {};
 };
 
@@ -61,6 +61,7 @@ hipError_t stage_new(size_t size, int device, Staging **out)
     hipError_t e = hipSuccess;
     for (int i = 0; i < 2 && e == hipSuccess; ++i) {
         e = hipHostMalloc((void **)&b->pin[i], size, hipHostMallocDefault);
+        if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&b->map[i], b->pin[i], 0);
         if (e == hipSuccess) e = hipMalloc((void **)&b->dev[i], size);
         if (e == hipSuccess) e = hipEventCreateWithFlags(&b->ev[i], hipEventDisableTiming);
     }
@@ -110,6 +111,11 @@ void stage_put(Staging *b)
     }
     stage_free(b);
 }
+
+// up to so many bytes a field's launch works on the pinned memory itself, with no
+// copy behind it (one component of 32x32x16: 33 us down, 25 so; 8 components of
+// 32x32x16, 0.7 MB, up: 69 and 81)
+constexpr int64_t DIRECT_MAX = 256 << 10;
 
 // ---------------------------------------------------------------------------
 // host threads of one call: run(job) calls job(t, nt) on the caller's thread
@@ -407,16 +413,21 @@ __global__ __launch_bounds__(256) void k_field_down(Grid g, const int *__restric
         if (x0 + r < hx && z0 + lx < hz) buf[((me + r) * hy + iy) * hz + z0 + lx] = t[lx][r];
 }
 
-// one component's interior columns [x0, x0 + nxs) from the staging buffer
-__global__ __launch_bounds__(256) void k_field_up(Grid g, const float *__restrict__ buf, int x0, int nxs, float *__restrict__ fld)
+// interior columns [q0, q0 + nq) of component after component from the staging
+// buffer: block = (32 columns, y, 32 z), transposed the same way
+__global__ __launch_bounds__(256) void k_field_up(Grid g, const float *__restrict__ buf, int q0, int nq, int nzb, float *__restrict__ fld)
 {
-    const int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;   // (k, j, i), i fastest
+    __shared__ float t[32][33];
     const int hz = g.nz + 3;
-    if (q >= (int64_t)nxs * g.ny * hz) return;
-    const int i = (int)(q % nxs);
-    const int64_t r = q / nxs;
-    const int j = (int)(r % g.ny), k = (int)(r / g.ny);
-    fld[(int64_t)k * plane_stride(g) + (int64_t)j * g.nx + x0 + i] = buf[((int64_t)i * g.ny + j) * hz + k];
+    const int zb = blockIdx.x % nzb, iy = (blockIdx.x / nzb) % g.ny, c0 = blockIdx.x / (nzb * g.ny) * XB, z0 = zb * 32;
+    const int lx = threadIdx.x & 31, l8 = threadIdx.x >> 5;
+    for (int r = l8; r < XB; r += 8)
+        if (c0 + r < nq && z0 + lx < hz) t[lx][r] = buf[((int64_t)(c0 + r) * g.ny + iy) * hz + z0 + lx];
+    __syncthreads();
+    const int q = q0 + c0 + lx, c = q / g.nx, x = q - c * g.nx;
+    float *out = fld + c * field_stride(g) + (int64_t)iy * g.nx + x;
+    for (int r = l8; r < 32; r += 8)
+        if (c0 + lx < nq && z0 + r < hz) out[(int64_t)(z0 + r) * plane_stride(g)] = t[r][lx];
 }
 
 }  // namespace
@@ -455,16 +466,58 @@ hipError_t launch_iota(int64_t n, int *p, hipStream_t s)
     return n > 0 ? launch(k_iota, blocks_of(n), s, n, p) : hipSuccess;
 }
 
+// Small fields.  A launch and a copy behind it cost more than the transposition
+// of a few thousand values here, so small ones are copied as they lie on the
+// device; not where their planes are whole pages apart, whose lines then share
+// a few sets of the host's cache (32x32x16, one component: 29 us down and 50 up
+// this way, 25 and 25 the other).  Pageable copies down of at most 16 KB take
+// longer than larger ones (23 us and 13).  16^3, one component: 13 us down and
+// 12 up; with a launch and a copy 28 and 25, with a launch that works on the
+// pinned memory itself (DIRECT_MAX) 19 and 19.
+constexpr size_t PAGEABLE_MIN = 16 << 10, SMALL_DOWN = 160 << 10, SMALL_UP = 320 << 10;
+// bytes on the device, 0 where the planes are whole pages apart
+static size_t small_field(const Grid &g, int ncomp)
+{
+    return plane_stride(g) % 1024 == 0 ? 0 : sizeof(float) * (size_t)ncomp * (size_t)field_stride(g);
+}
+// f(word on the device, value in the caller's array) of the plane -1 of every
+// column, the halo columns too when x0 is -1
+template <class F> static void small_columns(const Grid &g, int ncomp, int x0, F f)
+{
+    const int hx = g.nx + 3, hy = g.ny + 3, hz = g.nz + 3, halo = x0 < 0 ? 1 : -1;
+    for (int c = 0; c < ncomp; ++c)
+        for (int x = x0; x <= g.nx + halo; ++x)
+            for (int y = x0; y <= g.ny + halo; ++y) {
+                const int wx = (x + g.nx) % g.nx, wy = (y + g.ny) % g.ny;
+                f(c * field_stride(g) + (int64_t)wy * g.nx + wx, (((int64_t)c * hx + x + 1) * hy + y + 1) * hz);
+            }
+}
+
 template <class In, class Out>
 hipError_t download_field(const Grid &g, const In *fld, int ncomp, Out *out, hipStream_t s)
 {
     static_assert(sizeof(In) == 4, "32-bit words");
+    if (const size_t bytes = small_field(g, ncomp); bytes > PAGEABLE_MIN && bytes <= SMALL_DOWN) {
+        std::vector<In> h(bytes / 4);
+        hipError_t e = hipMemcpyAsync(h.data(), fld, bytes, hipMemcpyDeviceToHost, s);
+        const hipError_t e1 = hipStreamSynchronize(s);
+        if (e == hipSuccess) e = e1;
+        if (e != hipSuccess) return e;
+        const In *const raw = h.data();
+        small_columns(g, ncomp, -1, [=](int64_t dev, int64_t host) {
+            const In *__restrict__ v = raw + dev;
+            Out *__restrict__ o = out + host;
+            for (int z = 0; z < g.nz + 3; ++z) o[z] = (Out)v[z * plane_stride(g)];
+        });
+        return hipSuccess;
+    }
     const int hx = g.nx + 3, hy = g.ny + 3, hz = g.nz + 3, nxb = (hx + XB - 1) / XB, nzb = (hz + 31) / 32;
     const int64_t line = (int64_t)hy * hz;   // words of one x column
     const int nu = ncomp * nxb;
     Staging *b = nullptr;
     hipError_t e = stage_get((size_t)(4 * ncomp * hx * line), (size_t)(4 * XB * line), &b);
     if (e != hipSuccess) return e;
+    const bool direct = 4 * ncomp * hx * line <= DIRECT_MAX;
     const int uch = (int)std::min<int64_t>(nu, (int64_t)b->size / (4 * XB * line));
     const int nch = (nu + uch - 1) / uch;
     auto col = [&](int u) { return (int64_t)(u / nxb) * hx + std::min((u % nxb) * XB, hx); };   // columns before unit u
@@ -474,8 +527,9 @@ hipError_t download_field(const Grid &g, const In *fld, int ncomp, Out *out, hip
             b, nch, s,
             [&](int64_t c, char *dev, char *pin) {
                 const int u0 = (int)c * uch, u1 = std::min(nu, u0 + uch);
+                if (direct) dev = b->map[c & 1];
                 const hipError_t le = launch(k_field_down, (int64_t)(u1 - u0) * hy * nzb, s, g, (const int *)fld, u0, nzb, (int *)dev);
-                return le != hipSuccess ? le : hipMemcpyAsync(pin, dev, (size_t)(4 * (col(u1) - col(u0)) * line), hipMemcpyDeviceToHost, s);
+                return le != hipSuccess || direct ? le : hipMemcpyAsync(pin, dev, (size_t)(4 * (col(u1) - col(u0)) * line), hipMemcpyDeviceToHost, s);
             },
             [&](int64_t c, char *pin) {
                 const int u0 = (int)c * uch, u1 = std::min(nu, u0 + uch);
@@ -496,34 +550,50 @@ template hipError_t download_field(const Grid &, const int *, int, int *, hipStr
 
 hipError_t upload_field(const Grid &g, float *fld, int ncomp, const double *in, hipStream_t s)
 {
-    const int hy = g.ny + 3, hz = g.nz + 3;
-    const int64_t line = (int64_t)g.ny * hz, H = (int64_t)(g.nx + 3) * hy * hz, FS = field_stride(g);
+    if (const size_t bytes = small_field(g, ncomp); bytes > 0 && bytes <= SMALL_UP) {
+        Staging *b = nullptr;
+        hipError_t e = stage_get(bytes, 0, &b);
+        if (e != hipSuccess) return e;
+        float *h = (float *)b->pin[0];
+        small_columns(g, ncomp, 0, [=](int64_t dev, int64_t host) {
+            const double *__restrict__ v = in + host;
+            float *__restrict__ o = h + dev;
+            for (int z = 0; z < g.nz + 3; ++z) o[z * plane_stride(g)] = (float)v[z];
+        });
+        e = hipMemcpyAsync(fld, h, bytes, hipMemcpyHostToDevice, s);
+        const hipError_t e1 = hipStreamSynchronize(s);
+        stage_put(b);
+        return e != hipSuccess ? e : e1;
+    }
+    const int hy = g.ny + 3, hz = g.nz + 3, nzb = (hz + 31) / 32, nq = ncomp * g.nx;
+    const int64_t line = (int64_t)g.ny * hz, H = (int64_t)(g.nx + 3) * hy * hz;
     Staging *b = nullptr;
-    hipError_t e = stage_get((size_t)(4 * g.nx * line), (size_t)(4 * line), &b);
+    hipError_t e = stage_get((size_t)(4 * nq * line), (size_t)(4 * line), &b);
     if (e != hipSuccess) return e;
-    const int xch = (int)std::min<int64_t>(g.nx, (int64_t)b->size / (4 * line));
-    const int per = (g.nx + xch - 1) / xch;
+    const bool direct = 4 * nq * line <= DIRECT_MAX;
+    const int qch = (int)std::min<int64_t>(nq, (int64_t)b->size / (4 * line));
+    auto columns = [&](int64_t c) { return std::min(qch, nq - (int)c * qch); };
     {
-        Team team((int64_t)xch * line);
+        Team team((int64_t)qch * line);
         e = pipeline_up(
-            b, (int64_t)ncomp * per, s,
+            b, (nq + qch - 1) / qch, s,
             [&](int64_t c, char *pin) {
-                const int x0 = (int)(c % per) * xch, nxs = std::min(xch, g.nx - x0);
-                const double *src = in + (c / per) * H;
+                const int64_t rows = (int64_t)columns(c) * g.ny, first = c * qch * g.ny;   // (component, x, y)
                 float *p = (float *)pin;
                 team.run([&](int t, int nt) {
-                    const int64_t rows = (int64_t)nxs * g.ny;
                     for (int64_t r = rows * t / nt; r < rows * (t + 1) / nt; ++r) {
-                        const double *q = src + ((x0 + r / g.ny + 1) * hy + (r % g.ny + 1)) * hz;
-                        for (int k = 0; k < hz; ++k) p[r * hz + k] = (float)q[k];
+                        const int64_t q = (first + r) / g.ny, y = (first + r) % g.ny, x = q % g.nx;
+                        const double *src = in + q / g.nx * H + ((x + 1) * hy + (y + 1)) * hz;
+                        for (int k = 0; k < hz; ++k) p[r * hz + k] = (float)src[k];
                     }
                 });
             },
             [&](int64_t c, char *pin, char *dev) {
-                const int x0 = (int)(c % per) * xch, nxs = std::min(xch, g.nx - x0);
-                const hipError_t le = hipMemcpyAsync(dev, pin, (size_t)(4 * nxs * line), hipMemcpyHostToDevice, s);
+                const int n = columns(c);
+                if (direct) dev = b->map[c & 1];
+                const hipError_t le = direct ? hipSuccess : hipMemcpyAsync(dev, pin, (size_t)(4 * n * line), hipMemcpyHostToDevice, s);
                 if (le != hipSuccess) return le;
-                return launch(k_field_up, blocks_of((int64_t)nxs * line), s, g, (const float *)dev, x0, nxs, fld + (c / per) * FS);
+                return launch(k_field_up, (int64_t)((n + XB - 1) / XB) * g.ny * nzb, s, g, (const float *)dev, (int)c * qch, n, nzb, fld);
             });
     }
     stage_put(b);
