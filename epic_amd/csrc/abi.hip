@@ -1007,7 +1007,7 @@ int epic_destroy(epic_handle m)
     if (m->n_h) (void)hipHostFree(m->n_h);
     if (m->s) (void)hipStreamDestroy(m->s);
     delete m;
-    if (epic_member::live == 0) release_staging();
+    if (epic_member::live == 0) release_staging(false);
     return EPIC_OK;
 }
 

@@ -25,8 +25,8 @@ hipError_t download_parcels(int64_t n, const int *orig, int *inv, const std::vec
 hipError_t upload_parcels(int64_t n, const int *orig, int *inv, const std::vector<IoGroup> &groups, hipStream_t s);
 hipError_t launch_iota(int64_t n, int *p, hipStream_t s);
 
-// gives the idle staging buffers back
-void release_staging();
+// gives the idle staging buffers back, all of them or all but one set
+void release_staging(bool all);
 // hipMalloc, tried again without them when memory is short
 hipError_t device_malloc(void **p, size_t bytes);
 

@@ -27,9 +27,12 @@ namespace epic {
 namespace {
 
 // ---------------------------------------------------------------------------
-// staging buffers: a process-wide pool, at most POOL_KEEP idle ones kept until
-// the last member goes or memory is short (release_staging); a call owns the
-// one it takes, so calls of several threads never share one
+// staging buffers: a process-wide pool of at most POOL_KEEP idle sets.  When the
+// last member goes the largest stays (up to STAGE_MAX a buffer: a program that
+// makes one member at a time would allocate it again in each, at 64x64x32 5 ms
+// of the 21 from create to destroy); when device memory is short all are given
+// back (device_malloc).  A call owns the set it takes, so calls of several
+// threads never share one.
 // ---------------------------------------------------------------------------
 constexpr size_t STAGE_MIN = size_t(1) << 20, STAGE_MAX = size_t(32) << 20, POOL_KEEP = 4;
 
@@ -432,12 +435,21 @@ __global__ __launch_bounds__(256) void k_field_up(Grid g, const float *__restric
 
 }  // namespace
 
-void release_staging()
+void release_staging(bool all)
 {
     std::vector<Staging *> idle;
     {
         std::lock_guard<std::mutex> lk(stage_mu);
         idle.swap(stage_pool);
+        if (!all) {
+            auto keep = idle.end();
+            for (auto it = idle.begin(); it != idle.end(); ++it)
+                if ((*it)->size <= STAGE_MAX && (keep == idle.end() || (*it)->size > (*keep)->size)) keep = it;
+            if (keep != idle.end()) {
+                stage_pool.push_back(*keep);
+                idle.erase(keep);
+            }
+        }
     }
     for (Staging *b : idle) stage_free(b);
 }
@@ -447,7 +459,7 @@ hipError_t device_malloc(void **p, size_t bytes)
     hipError_t e = hipMalloc(p, bytes);
     if (e == hipSuccess) return e;
     (void)hipGetLastError();
-    release_staging();
+    release_staging(true);
     return hipMalloc(p, bytes);
 }
 

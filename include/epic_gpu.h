@@ -95,7 +95,12 @@ enum {
 #define EPIC_MAX_PARCELS ((int64_t)0x3fffffff)
 int epic_create(const epic_grid_t *grid, const epic_phys_t *phys, const epic_flags_t *flags,
                 int64_t max_parcels, epic_handle *out);
-/* finalise_inversion + field_dealloc + parcels%deallocate */
+/* finalise_inversion + field_dealloc + parcels%deallocate.  The set/get calls
+ * stage their copies in buffers that outlive the call and the member: at most
+ * four idle sets of 2 x 32 MB of device and as much pinned host memory in the
+ * process (a set is larger where 32 x columns of a field exceed 32 MB), one of
+ * them after the last member has gone.  All are given back when an allocation
+ * of this library finds device memory short. */
 int epic_destroy(epic_handle h);
 const char *epic_last_error(epic_handle h);
 

@@ -1,0 +1,48 @@
+"""Staging buffers of the host copies, seen from the allocator (a child process
+whose large allocations pass through alloc_watch.cpp)."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+PRELUDE = """
+import ctypes as C, sys
+sys.path.insert(0, {root!r})
+watch = C.CDLL({lib!r}, mode=C.RTLD_GLOBAL)
+import numpy as np
+from epic_amd import workloads as W
+from epic_amd.core import Member
+refuse = C.c_int.in_dll(watch, "watch_refuse_device")
+device, pinned = (C.c_long.in_dll(watch, n) for n in ("watch_device", "watch_pinned"))
+"""
+
+
+def _run(tmp_path, body):
+    lib = str(tmp_path / "alloc_watch.so")
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", "-o", lib, os.path.join(HERE, "alloc_watch.cpp"), "-ldl"], check=True)
+    code = PRELUDE.format(root=os.path.dirname(HERE), lib=lib) + body
+    print("staging: child process", flush=True)
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
+    return r.stdout
+
+
+def test_one_set_stays_when_the_last_member_goes(tmp_path):
+    _run(tmp_path, """
+def cycle():
+    mem = W.rising_thermal(32, seed=3)
+    gm = Member.from_workload(mem)
+    gm.par2grid()
+    gm.get_field("velgradg"), gm.get_tendencies(), gm.get_parcels()
+    gm.close()
+    return pinned.value
+
+first = cycle()
+assert first > 0, "the allocator is not watched"
+assert cycle() == first, "pinned buffers allocated again for the next member"
+""")
