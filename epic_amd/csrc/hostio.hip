@@ -39,7 +39,9 @@ constexpr size_t STAGE_MIN = size_t(1) << 20, STAGE_MAX = size_t(32) << 20, POOL
 struct Staging {
     size_t size = 0;   // bytes of each of the two buffers
     int device = 0;
-    char *pin[2] = {}, *map[2] = {}, *dev[2] = {};   // pinned, its address on the device, device memory
+    // pinned, its address on the device, device memory (null in a set made while
+    // there was none: launches then work on the pinned memory)
+    char *pin[2] = {}, *map[2] = {}, *dev[2] = {};
     hipEvent_t ev[2] = {};
 };
 
@@ -56,7 +58,7 @@ void stage_free(Staging *b)
     delete b;
 }
 
-hipError_t stage_new(size_t size, int device, Staging **out)
+hipError_t stage_new(size_t size, int device, bool on_device, Staging **out)
 {
     Staging *b = new Staging();
     b->size = size;
@@ -65,7 +67,7 @@ hipError_t stage_new(size_t size, int device, Staging **out)
     for (int i = 0; i < 2 && e == hipSuccess; ++i) {
         e = hipHostMalloc((void **)&b->pin[i], size, hipHostMallocDefault);
         if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&b->map[i], b->pin[i], 0);
-        if (e == hipSuccess) e = hipMalloc((void **)&b->dev[i], size);
+        if (e == hipSuccess && on_device) e = device_malloc((void **)&b->dev[i], size);
         if (e == hipSuccess) e = hipEventCreateWithFlags(&b->ev[i], hipEventDisableTiming);
     }
     if (e != hipSuccess) {
@@ -78,7 +80,8 @@ hipError_t stage_new(size_t size, int device, Staging **out)
 }
 
 // buffers of at least need bytes, capped at STAGE_MAX (the caller chunks), or
-// smaller ones when memory is short; never less than least bytes
+// smaller ones when memory is short; never less than least bytes.  A copy does
+// not fail for want of device memory: without any it takes pinned buffers alone
 hipError_t stage_get(size_t need, size_t least, Staging **out)
 {
     int device = 0;
@@ -95,15 +98,16 @@ hipError_t stage_get(size_t need, size_t least, Staging **out)
                 return hipSuccess;
             }
     }
-    for (; size >= std::max(least, STAGE_MIN); size /= 2)
-        if ((e = stage_new(size, device, out)) == hipSuccess) return hipSuccess;
+    for (const bool on_device : {true, false})
+        for (size_t n = size; n >= std::max(least, STAGE_MIN); n /= 2)
+            if ((e = stage_new(n, device, on_device, out)) == hipSuccess) return hipSuccess;
     return e;
 }
 
 // back to the pool, which keeps the largest
 void stage_put(Staging *b)
 {
-    {
+    if (b->dev[1]) {
         std::lock_guard<std::mutex> lk(stage_mu);
         stage_pool.push_back(b);
         if (stage_pool.size() <= POOL_KEEP) return;
@@ -370,16 +374,16 @@ hipError_t parcel_io(bool up, int64_t n, const int *orig, int *inv, std::vector<
                 b, nch, s,
                 [&](int64_t c, char *dev, char *pin) {
                     const int64_t m = chunk(c);
-                    const hipError_t le = launch(k_parcel_io<false>, blocks_of(m), s, a, map, c * ch, m, dev);
-                    return le != hipSuccess ? le : hipMemcpyAsync(pin, dev, (size_t)(m * per), hipMemcpyDeviceToHost, s);
+                    const hipError_t le = launch(k_parcel_io<false>, blocks_of(m), s, a, map, c * ch, m, dev ? dev : b->map[c & 1]);
+                    return le != hipSuccess || !dev ? le : hipMemcpyAsync(pin, dev, (size_t)(m * per), hipMemcpyDeviceToHost, s);
                 },
                 convert);
         else if (e == hipSuccess)
             e = pipeline_up(b, nch, s, convert, [&](int64_t c, char *pin, char *dev) {
                 const int64_t m = chunk(c);
-                const hipError_t le = hipMemcpyAsync(dev, pin, (size_t)(m * per), hipMemcpyHostToDevice, s);
+                const hipError_t le = dev ? hipMemcpyAsync(dev, pin, (size_t)(m * per), hipMemcpyHostToDevice, s) : hipSuccess;
                 if (le != hipSuccess) return le;
-                return launch(k_parcel_io<true>, blocks_of(m), s, a, map, c * ch, m, dev);
+                return launch(k_parcel_io<true>, blocks_of(m), s, a, map, c * ch, m, dev ? dev : b->map[c & 1]);
             });
     }
     stage_put(b);
@@ -529,7 +533,7 @@ hipError_t download_field(const Grid &g, const In *fld, int ncomp, Out *out, hip
     Staging *b = nullptr;
     hipError_t e = stage_get((size_t)(4 * ncomp * hx * line), (size_t)(4 * XB * line), &b);
     if (e != hipSuccess) return e;
-    const bool direct = 4 * ncomp * hx * line <= DIRECT_MAX;
+    const bool direct = !b->dev[0] || 4 * ncomp * hx * line <= DIRECT_MAX;
     const int uch = (int)std::min<int64_t>(nu, (int64_t)b->size / (4 * XB * line));
     const int nch = (nu + uch - 1) / uch;
     auto col = [&](int u) { return (int64_t)(u / nxb) * hx + std::min((u % nxb) * XB, hx); };   // columns before unit u
@@ -582,7 +586,7 @@ hipError_t upload_field(const Grid &g, float *fld, int ncomp, const double *in, 
     Staging *b = nullptr;
     hipError_t e = stage_get((size_t)(4 * nq * line), (size_t)(4 * line), &b);
     if (e != hipSuccess) return e;
-    const bool direct = 4 * nq * line <= DIRECT_MAX;
+    const bool direct = !b->dev[0] || 4 * nq * line <= DIRECT_MAX;
     const int qch = (int)std::min<int64_t>(nq, (int64_t)b->size / (4 * line));
     auto columns = [&](int64_t c) { return std::min(qch, nq - (int)c * qch); };
     {

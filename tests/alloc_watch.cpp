@@ -1,5 +1,5 @@
-// Device and pinned allocations of at least 1 MB, counted and refused on demand:
-// loaded with RTLD_GLOBAL before libepic_gpu.so, whose calls then come here.
+// Device and pinned allocations of at least 1 MB, counted; device memory refused
+// on demand (1: those, -1: the next of any size).  Loaded with RTLD_GLOBAL before libepic_gpu.so, whose calls then come here.
 #include <dlfcn.h>
 
 #include <cstddef>
@@ -19,13 +19,12 @@ constexpr size_t LARGE = size_t(1) << 20;
 
 extern "C" int hipMalloc(void **p, size_t n)
 {
-    if (n >= LARGE) {
-        if (watch_refuse_device) {
-            *p = nullptr;
-            return 2;   // hipErrorOutOfMemory
-        }
-        ++watch_device;
+    if (watch_refuse_device < 0 || (watch_refuse_device > 0 && n >= LARGE)) {
+        if (watch_refuse_device < 0) watch_refuse_device = 0;
+        *p = nullptr;
+        return 2;   // hipErrorOutOfMemory
     }
+    if (n >= LARGE) ++watch_device;
     return real<int (*)(void **, size_t)>("hipMalloc")(p, n);
 }
 

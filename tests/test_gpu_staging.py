@@ -46,3 +46,27 @@ first = cycle()
 assert first > 0, "the allocator is not watched"
 assert cycle() == first, "pinned buffers allocated again for the next member"
 """)
+
+
+def test_copies_need_no_device_memory(tmp_path):
+    _run(tmp_path, """
+rng = np.random.default_rng(1)
+f32 = lambda *s: rng.standard_normal(s).astype(np.float32).astype(np.float64)
+grid, n = (96, 128, 80), 600001   # several chunks each
+gm = Member(*grid, (0.0, 0.0, 0.0), (1.0, 1.0, 1.0), max_parcels=n)
+small = Member(16, 16, 16, (0.0, 0.0, 0.0), (1.0, 1.0, 1.0))
+refuse.value = 1
+want = [rng.uniform(0.0, 1.0, (n, 3)), f32(n, 3), f32(n, 5), f32(n), f32(n), f32(n)]
+gm.set_parcels(*want)
+assert all(np.array_equal(a, b) for a, b in zip(gm.get_parcels().values(), want))
+dp, dv = f32(n, 3), f32(n, 3)
+gm.set_tendencies(dp, dv)
+got = gm.get_tendencies()
+assert np.array_equal(got[0], dp) and np.array_equal(got[1], dv)
+for m, g in ((gm, grid), (small, (16, 16, 16))):
+    f = f32(8, *(k + 3 for k in g))
+    m.set_field("velgradg", f)
+    got = m.get_field("velgradg")
+    assert np.array_equal(got[:, 1:-2, 1:-2], f[:, 1:-2, 1:-2])
+assert device.value > 0, "the allocator is not watched"
+""")
