@@ -8,6 +8,7 @@
 
 #include "epic_gpu.h"
 #include "ellipsoid.h"
+#include "hostio.h"
 
 using namespace epic;
 
@@ -62,8 +63,8 @@ extern "C" int epic_diagonalise(int64_t n, const double *A, double *D, double *V
         return true;
     };
     const size_t b9 = sizeof(double) * 9 * (size_t)n, b3 = sizeof(double) * 3 * (size_t)n;
-    if (hip(hipMalloc((void **)&dA, b9), "hipMalloc") || hip(hipMalloc((void **)&dD, b3), "hipMalloc") ||
-        hip(hipMalloc((void **)&dV, b9), "hipMalloc")) {
+    if (hip(device_malloc((void **)&dA, b9), "hipMalloc") || hip(device_malloc((void **)&dD, b3), "hipMalloc") ||
+        hip(device_malloc((void **)&dV, b9), "hipMalloc")) {
         cleanup();
         return EPIC_E_NOMEM;
     }

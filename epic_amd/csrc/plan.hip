@@ -2,6 +2,8 @@
 // (optionally with the phase timers captured as event-record nodes).
 #include "plan.h"
 
+#include "hostio.h"
+
 #include <mutex>
 #include <utility>
 
@@ -64,7 +66,7 @@ hipError_t pool_get(size_t bytes, hipStream_t s, char **out, size_t *got)
             return hipSuccess;
         }
     }
-    e = hipMalloc((void **)out, want);
+    e = device_malloc((void **)out, want);
     if (e != hipSuccess) return e;
     *got = want;
     return hipSuccess;
@@ -228,7 +230,7 @@ hipError_t Plan::prepare_graph(hipStream_t s, bool timed)
                     stamp_phase_.push_back(r.phase);
                     cur = r.phase;
                 }
-            e = hipMalloc((void **)&stamps_, sizeof(unsigned long long) * 2 * std::max<size_t>(1, stamp_phase_.size()));
+            e = device_malloc((void **)&stamps_, sizeof(unsigned long long) * 2 * std::max<size_t>(1, stamp_phase_.size()));
             if (e != hipSuccess) return e;
             int dev = 0, khz = 0;
             e = hipGetDevice(&dev);

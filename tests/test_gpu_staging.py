@@ -70,3 +70,18 @@ for m, g in ((gm, grid), (small, (16, 16, 16))):
     assert np.array_equal(got[:, 1:-2, 1:-2], f[:, 1:-2, 1:-2])
 assert device.value > 0, "the allocator is not watched"
 """)
+
+
+def test_idle_buffers_give_way(tmp_path):
+    """An allocation that finds device memory short gets it once the idle
+    staging buffers are back."""
+    _run(tmp_path, """
+mem = W.rising_thermal(32, seed=3)
+gm = Member.from_workload(mem)
+gm.get_parcels()
+held = device.value
+refuse.value = -1   # the launch tables of the next call
+gm.par2grid()
+gm.get_parcels()
+assert device.value > held, "no staging buffers were given back"
+""")
