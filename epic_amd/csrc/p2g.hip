@@ -807,8 +807,8 @@ __global__ __launch_bounds__(1024, 4) void k_p2g_tiles(const P2GArgs *__restrict
 // tiles of 8, the last one shorter when n is not a multiple of 8): its number t
 // and the node's place l in its box; false when it holds nothing for the node.
 // No box of such a row meets itself, and of two tiles one is beside the other
-// once.  Beyond a last tile of one node, node 0 is also the last place of the
-// box of the tile before it (d = 1, where node 0 has no other).
+// once.  (Not here: beyond a last tile of one node, node 0 is also the last
+// place of the box of the tile before it.)
 __device__ inline bool box_place(int d, int i, int n, int nt, int &t, int &l)
 {
     const int own = i >> 3, r = i & 7;
@@ -832,10 +832,7 @@ __device__ inline bool box_place(int d, int i, int n, int nt, int &t, int &l)
         }
     } else if (d > 0) {
         l = 0;
-        if (i == 0 && n == 8 * (nt - 1) + 1) {
-            t = nt - 2;
-            l = P2G_BOX - 1;
-        } else if (i == n - 1) t = 0;
+        if (i == n - 1) t = 0;
         else if (r != 7) return false;
     }
     return true;
@@ -843,8 +840,8 @@ __device__ inline bool box_place(int d, int i, int n, int nt, int &t, int &l)
 
 // adds the staged sums of node (i, j, k) to out[], and its far-point sums
 // when there are any (far).  NS fields are staged; of P2G_DRY, field 5 is
-// field 4 and field 6 zero.  A node lies in one box, or in two (three where
-// the last tile has a single node) along each direction.  The kernel was bound
+// field 4 and field 6 zero.  A node lies in one box, or in two along each
+// direction (three beside a last tile of a single node).  The kernel was bound
 // by its waits, one per box; the up to four boxes of a z chunk are loaded
 // together instead: 19.3 -> 11.6 us at 16^3, 24.9 -> 20.9 at 64^3, 143 -> 103 at
 // 128^3 (290 MB of dry staging).  All nine combinations at once take 184
@@ -866,9 +863,13 @@ __device__ inline void stage_add(const FinalizeArgs &a, int i, int j, int k, dou
     };
     const int nbox = a.tz + 3;
     const int cza = (k + 1) / a.tz;
+    // node row 0 in the box of the tile before a last one of one row, which does
+    // not lie beside its own (only along y, as nx is even, and from 25 rows on:
+    // the transforms do not take 17)
+    const bool beyond = a.nty > 3 && g.ny == P2G_TY * (a.nty - 1) + 1 && j == 0;
     if (a.ntx >= 2 && a.nty >= 2 && g.nx >= P2G_BOX && g.ny >= P2G_BOX) {
         // offsets of the boxes' tiles and places along x and y, -1 for none:
-        // its own tile's, a neighbour's, and (a last tile of one node only)
+        // its own tile's, a neighbour's, and (a last tile of one row only)
         // the other neighbour's
         int64_t ox[3], oy[3];
         auto places = [&](int64_t o[3], int p, int n, int nt, int64_t tile, int node) {
@@ -910,12 +911,19 @@ __device__ inline void stage_add(const FinalizeArgs &a, int i, int j, int k, dou
                 }
             }
         }
+        if (beyond) {   // (apart, so that other rows' loads wait for nothing: 281 -> 277 us of par2grid a step at 32^3)
+            const int64_t y = (int64_t)(a.nty - 2) * a.ntx * nbox * PLANE + (P2G_BOX - 1) * P2G_BOX * NS;
+#pragma unroll 1
+            for (int q = 0; q < 9; ++q) {   // (z chunk, box along x)
+                const int cz = cza + q / 3 - 1, lp = k - (cz * a.tz - 2), c = q % 3;
+                const int64_t x = c == 0 ? ox[0] : c == 1 ? ox[1] : ox[2];
+                if (x >= 0 && cz >= 0 && cz < a.nchz && lp >= 0 && lp < nbox)
+                    add(gl(a.staging) + (int64_t)cz * a.nty * a.ntx * nbox * PLANE + lp * PLANE + y + x);
+            }
+        }
         return;
     }
     const int txa = i / P2G_TX, tya = j / P2G_TY;
-    // (nx is even: only along y can a last tile have one node, and the box of
-    // the tile before it reach node 0)
-    const bool beyond = a.nty > 3 && j == 0 && g.ny == P2G_TY * (a.nty - 1) + 1;
     for (int dcz = -1; dcz <= 1; ++dcz) {
         const int cz = cza + dcz;
         if (cz < 0 || cz >= a.nchz) continue;
