@@ -1475,7 +1475,7 @@ int64_t epic_member_bytes(const epic_grid_t *grid, int64_t max_parcels)
     b += 4 * (6 * nc + (nc + 1) + nc);                                        // histograms, cell_start, cursor
     b += 4 * scan_scratch_ints(std::max<int64_t>(std::max<int64_t>(nc, c), (int64_t)(g.nx + 3) * (g.ny + 3) * (g.nz + 2)));
     b += 4 * ((int64_t)F_COUNT * FS + 2 * FS) + 8 * staging_elems_max(g);   // fields, counts, staging
-    b += 8 * (int64_t)P2G_NF * FS + 8 + 8 * P2G_NF;                          // far-point sums
+    b += 8 * (int64_t)P2G_NF * FS + 12 + 8 * P2G_NF;                         // far-point sums
     b += 20 * c + 4096;                                                       // merge scratch (its first phase)
     b += (int64_t)NSPEC * 8 * spec_size(g);                                  // spectra
     return b;

@@ -477,9 +477,14 @@ __global__ __launch_bounds__(NT, 4) void k_g2p_tiles(const G2PTileArgs *__restri
     if (e) atomicOr(a.err, e);
 }
 
+// (128 threads a layer at least: add_rk_stage_tiles)
 template <int TZ> static const void *tiles_kernel(int nt)
 {
-    return nt == 1024 ? (const void *)k_g2p_tiles<1024, TZ> : nt == 512 ? (const void *)k_g2p_tiles<512, TZ> : (const void *)k_g2p_tiles<256, TZ>;
+    if constexpr (TZ <= 2)
+        if (nt == 256) return (const void *)k_g2p_tiles<256, TZ>;
+    if constexpr (TZ <= 4)
+        if (nt == 512) return (const void *)k_g2p_tiles<512, TZ>;
+    return (const void *)k_g2p_tiles<1024, TZ>;
 }
 
 void add_rk_stage_tiles(Plan &P, int phase, const std::vector<G2PTileArgs> &all)

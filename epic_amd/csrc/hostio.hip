@@ -133,7 +133,8 @@ public:
     explicit Team(int64_t elements)
     {
         const unsigned hw = std::thread::hardware_concurrency();
-        // (starting a helper takes as long as half a million conversions)
+        // one thread per 2^20 elements, which one converts in 0.2 ms; to start
+        // and join a helper takes 18 us, 15 of them 190
         const int nt = (int)std::min<int64_t>(std::min<unsigned>(hw ? hw : 1, 16u), elements / (1 << 20) + 1);
         try {
             for (int t = 1; t < nt; ++t) th_.emplace_back([this, t]() { work(t); });

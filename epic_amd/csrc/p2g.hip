@@ -242,8 +242,9 @@ int64_t scan_scratch_ints(int64_t n) { return (n + SCAN_BLOCK - 1) / SCAN_BLOCK 
 // ---------------------------------------------------------------------------
 // 3./4. placement and per-cell ordering
 // ---------------------------------------------------------------------------
-// Runs of equal keys in consecutive lanes (the parcels are nearly in cell
-// order) take one ticket per run.
+// Lanes of a wave that hold the same key in a row (the parcels are nearly in cell
+// order) share one atomicAdd on the key's cursor; a lane's ticket is the cursor's
+// old value and its rank in the run.
 __global__ __launch_bounds__(256) void k_place(const PlaceArgs *__restrict__ tab, const int2 *__restrict__ bmap)
 {
     const ItemBlock ib = item_block(bmap);
@@ -263,7 +264,7 @@ __global__ __launch_bounds__(256) void k_place(const PlaceArgs *__restrict__ tab
 #pragma unroll
     for (int r = 0; r < NR; ++r) start[r] = (key[r] >= 0) ? gl(a.cell_start)[key[r]] : 0;
 #pragma unroll
-    for (int r = 0; r < NR; ++r) {   // wave_run_ticket, its atomic left in flight
+    for (int r = 0; r < NR; ++r) {   // the atomics are left in flight
         const int prev = __shfl_up(key[r], 1, 64);
         const bool head = (lane == 0) || (prev != key[r]);
         const unsigned long long heads = __ballot(head);
@@ -550,7 +551,11 @@ __global__ __launch_bounds__(1024, 4) void k_p2g_tiles(const P2GArgs *__restrict
             for (int d = 0; d < 3; ++d) cc[d] = (int)floor((pos[d] - g.lower[d]) * g.dxi[d]);
             int cx = wrap(cc[0], g.nx) - i0, cy = wrap(cc[1], g.ny) - j0, lz = cc[2] - k0;
             if ((unsigned)cx >= (unsigned)P2G_TX || (unsigned)cy >= (unsigned)P2G_TY || (unsigned)lz >= (unsigned)tz) {
-                err |= ERR_CELL_MISMATCH;   // not in the cell it was sorted into: left out
+                // not in the cell it was sorted into: left out.  In lane 1 or 2 of a
+                // quad it also puts its share of the others' sums at the wrong node:
+                // no sum of the call counts once this is reported (a wave that took
+                // such quads apart ran 0.7 % longer)
+                err |= ERR_CELL_MISMATCH;
                 have = false;
                 cx = cy = lz = 0;
             }

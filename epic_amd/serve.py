@@ -9,7 +9,8 @@ step of every cohort without waiting (``Batch.launch``), so cohorts run
 concurrently on the GPU, and while they run the server
 
 * admits waiting requests in arrival order while the HBM budget
-  (``core.member_bytes`` of every resident member) and the slot limit allow:
+  (``core.member_bytes`` of every resident member; the library's staging
+  buffers are outside it and give way to members) and the slot limit allow:
   it allocates the member, uploads its parcels on the member's own stream
   and captures the new cohort's step graph, all overlapping the tick (a
   retired member's memory counts against the budget until it is released);
