@@ -56,3 +56,19 @@ def test_node_sums(grid):
     assert np.abs(p["position"] - st.position).max() <= TOL * max(mem.dx)
     for k in ("vorticity", "B"):
         assert maxrel(p[k], getattr(st, k)) <= TOL, k
+
+
+@pytest.mark.parametrize("tz", [2, 8])   # 256 and 1024 threads; 512 by default
+def test_humid_tilings_give_the_same_bits(tz):
+    print(f"par2grid edges: humid, chunks of {tz} layers", flush=True)
+    mem = W.rising_thermal(64, seed=21, ny=72, nz=27, humidity_plume=True, n_blobs=4)
+    a, b = Member.from_workload(mem), Member.from_workload(mem)
+    b.set_tiling(tz, tz)
+    for gm in (a, b):
+        gm.ls_rk_step(0.0, 0.001)
+        gm.par2grid()
+    for f in ("volg", "vortg", "tbuoyg", "dbuoyg", "humg", "nparg"):
+        assert np.array_equal(a.get_field(f), b.get_field(f)), f
+    p, q = a.get_parcels(), b.get_parcels()
+    for k in p:
+        assert np.array_equal(p[k], q[k]), k
